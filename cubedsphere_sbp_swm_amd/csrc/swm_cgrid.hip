@@ -532,23 +532,10 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
     if (t < 2 * CD_NQ + 2) part[(long long)tile_ * 10 + t] = sh[0][t];
 }
 
-// one thread over the block partials: {mass, KE_u, KE_v, PE, hmin, hmax}
-__global__ void __launch_bounds__(64) k_cdiag_final(const double *__restrict__ part, long long nblocks,
-                                                    double *__restrict__ out) {
-    if (threadIdx.x != 0) return;
-    double s[CD_NQ] = {0.0, 0.0, 0.0, 0.0}, cc[CD_NQ] = {0.0, 0.0, 0.0, 0.0};
-    double hmin = 1e300, hmax = -1e300;
-    for (long long b = 0; b < nblocks; ++b) {
-        for (int q = 0; q < CD_NQ; ++q) {
-            cd_add(s[q], cc[q], part[b * 10 + 2 * q]);
-            cc[q] += part[b * 10 + 2 * q + 1];
-        }
-        hmin = fmin(hmin, part[b * 10 + 2 * CD_NQ]);
-        hmax = fmax(hmax, part[b * 10 + 2 * CD_NQ + 1]);
-    }
-    for (int q = 0; q < CD_NQ; ++q) out[q] = s[q] + cc[q];
-    out[CD_NQ] = hmin;
-    out[CD_NQ + 1] = hmax;
+// the block partials summed by one block: {mass, KE_u, KE_v, PE, hmin, hmax}
+__global__ void __launch_bounds__(swm::FINAL_THREADS) k_cdiag_final(const double *__restrict__ part, long long nblocks,
+                                                                    double *__restrict__ out) {
+    swm::sum_partials<CD_NQ, 10>(part, nblocks, out);
 }
 
 #undef C_POINT
@@ -1041,7 +1028,7 @@ extern "C" int swm_c_diagnostics(swm_cctx *c, const void *state, double out[7]) 
     hipLaunchKernelGGL(swmc::k_cdiag_partial, grd, blk, 0, c->stream, g, (const double *)state, c->qw,
                        c->qw + (c->N + 2), c->dpart);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(swmc::k_cdiag_final, dim3(1), dim3(64), 0, c->stream, c->dpart, c->dblocks, res);
+    hipLaunchKernelGGL(swmc::k_cdiag_final, dim3(1), dim3(swm::FINAL_THREADS), 0, c->stream, c->dpart, c->dblocks, res);
     HIP_TRY(hipGetLastError());
     double r[6];
     HIP_TRY(hipMemcpyAsync(r, res, sizeof(r), hipMemcpyDeviceToHost, c->stream));
