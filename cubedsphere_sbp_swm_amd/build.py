@@ -21,7 +21,8 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", f"--offload-arch={ARCH}",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-result", "-Wno-unused-function"]
-HIP_SOURCES = ["swm_capi.hip", "stage_o21.hip"] + [f"{k}_o{o}{s}.hip" for o in (42, 43, 63)
+HIP_SOURCES = ["swm_capi.hip", "swm_adjoint.hip", "swm_hordiff.hip", "swm_ecs.hip", "swm_cgrid.hip", "swm_cgrid_ecs.hip",
+               "stage_o21.hip"] + [f"{k}_o{o}{s}.hip" for o in (42, 43, 63)
                                                 for k, s in (("stage", ""), ("stage", "_f32"), ("ens", ""))]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unused-function"]
 FC = shutil.which("amdflang") or "/opt/rocm/bin/amdflang"

@@ -1,5 +1,5 @@
 // Hand-written adjoint of the Ah-grid SWM right-hand side and of the RK4 step, FP64, SBP
-// families 42 / 43 / 63 (included into swm_capi.hip).
+// families 42 / 43 / 63.
 //
 // Forward map at a state y = (h, u, v) (operator_swm_mod.f90:61-113):
 //   ut, vt = Qi (u, v);  K = (u ut + v vt)/2 + g h (+ g hs)
@@ -28,6 +28,11 @@
 // Step states come from checkpoints every C steps: the reverse sweep recomputes one segment
 // of C steps from its checkpoint with the forward stage kernels, which also store each
 // step's stage inputs y1..y3 and the synced vorticity of y0..y3 for the adjoint kernels.
+
+#include <algorithm>
+#include <utility>
+
+#include "swm_ctx.h"
 
 namespace swm {
 
@@ -166,13 +171,6 @@ __global__ void adj_pre_edge(AdjGeo g, const double *__restrict__ y, const doubl
         W[2 * g.fs + o] = -mu / g.hxs;
         W[3 * g.fs + o] = -mv / g.hxs;
     }
-}
-
-__device__ __forceinline__ int edge_slot(int n, int i, int j) {
-    if (j == 0) return i;
-    if (j == n - 1) return n + i;
-    if (i == 0) return 2 * n + j - 1;
-    return 3 * n + j - 3;
 }
 
 struct AdjArgs {
@@ -431,7 +429,7 @@ __global__ void __launch_bounds__(TX * TY) adj_tile(AdjGeo g, AdjArgs A, AdjEll 
 
 // ------------------------------------------------------------------------------------------------
 // Host side
-namespace {
+namespace swm_host {
 
 struct AdjWork {
     int es = 0, ns = 0;
@@ -452,6 +450,10 @@ void free_adj_work(AdjWork *w) {
         if (p) (void)hipFree(p);
     delete w;
 }
+
+}  // namespace swm_host
+
+namespace {
 
 // CSR of the scalar sync and of the TRANSPOSED covariant vector sync
 int build_csr(int N, int vector, bool transpose, int nrows, std::vector<int> &ptr, std::vector<int> &col,

@@ -1,5 +1,4 @@
-// ECS halos on the C grid and the operators built on them (included into swm_capi.hip after
-// swm_cgrid.hip and swm_ecs.hip).
+// ECS halos on the C grid and the operators built on them.
 //
 // Vector halo: get_halo_vector of ecs_halo_vec_c_t ("ecs_C_vec", contravariant components) and
 // ecs_halo_vec_c_cov_t ("ecs_C_vec_covariant"), equiang_cs/ecs_halo_vec_c_mod.f90:76-595 with the
@@ -16,6 +15,12 @@
 // ECS_O halo on the C grid's o points (for gradient_c2_ecs, grad_c2_ecs_mod.f90:33-51, and
 // massflux_c_up4, massflux_Cgrid_mod.f90:87-104): the same procedure as swm_ecs_halo_o
 // (swm::ecs_o_fill), reading the exchanged cells from the gathered strips.
+
+#include <algorithm>
+#include <cmath>
+
+#include "ecs_o_kernel.h"
+#include "swm_cctx.h"
 
 namespace swmc {
 

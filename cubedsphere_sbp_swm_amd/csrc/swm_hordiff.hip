@@ -1,5 +1,5 @@
 // Hyperdiffusion of the Ah state with the narrow-stencil SBP Laplacians sbp21, sbp42 and sbp63,
-// FP64 (included into swm_capi.hip).  sbp21 (three-point rows, laplace_Ah_sbp21_narrow_mod.f90)
+// FP64.  sbp21 (three-point rows, laplace_Ah_sbp21_narrow_mod.f90)
 // runs as one point per thread (hd_lap21); the table-driven sbp42 / sbp63 on LDS tiles.
 //
 // Laplacian, laplace_Ah_sbp42_narrow_t%calc_laplace (differential_operators/horizontal/
@@ -22,6 +22,8 @@
 // h and the three Cartesian velocity components share every launch.  Panel-edge results are
 // written to a compact edge buffer first and synchronised from there, so that no kernel reads
 // a value another block of the same launch overwrites.
+
+#include "swm_ctx.h"
 
 #include "laplace_sbp42_narrow.h"
 #include "laplace_sbp63_narrow.h"
@@ -566,13 +568,25 @@ __global__ void hd_vsync(HdGeo g, const double *__restrict__ E2, double dt, cons
 
 // ------------------------------------------------------------------------------------------------
 // Host side
-namespace {
+namespace swm_host {
 
 struct HdWork {
     double *b1 = nullptr, *b2 = nullptr;          // 3 planes each
     double *WA = nullptr, *WB = nullptr;          // 4 fields each (h, Vx, Vy, Vz)
     double *E = nullptr, *E2 = nullptr;           // 4 x ns, 2 x ns edge values
 };
+
+void free_hd_work(HdWork *w) {
+    if (!w) return;
+    void *ptrs[] = {w->b1, w->b2, w->WA, w->WB, w->E, w->E2};
+    for (void *p : ptrs)
+        if (p) (void)hipFree(p);
+    delete w;
+}
+
+}  // namespace swm_host
+
+namespace {
 
 // closure rows of both panel edges disjoint: N+1 >= 12 (sbp42), 18 (sbp63); sbp21 has one-point
 // closures (any context size)
@@ -700,14 +714,6 @@ int enqueue_diff(swm_ctx *c, int uv_order, int h_order, const double *yin, const
     hipLaunchKernelGGL(swm::hd_vsync, dim3((ns + 255) / 256), blk, 0, c->stream, g, (const double *)w->E2, dt, y0, yo);
     HIP_TRY(hipGetLastError());
     return SWM_OK;
-}
-
-void free_hd_work(HdWork *w) {
-    if (!w) return;
-    void *ptrs[] = {w->b1, w->b2, w->WA, w->WB, w->E, w->E2};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
-    delete w;
 }
 
 }  // namespace

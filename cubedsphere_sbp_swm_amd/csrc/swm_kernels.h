@@ -257,6 +257,14 @@ __device__ __forceinline__ T sbp_row(int t, int n, const G &get) {
     return sbp_right_dispatch<ORD, T>(t - (n - S::NE), n, get, std::make_integer_sequence<int, S::NE>{});
 }
 
+// slot of a panel-edge point in a panel's compact edge buffer (4 (n-1) slots)
+__device__ __forceinline__ int edge_slot(int n, int i, int j) {
+    if (j == 0) return i;
+    if (j == n - 1) return n + i;
+    if (i == 0) return 2 * n + j - 1;
+    return 3 * n + j - 3;
+}
+
 // Vector halo convention: neighbour components (a,b) -> local (u,v)
 template <typename T>
 __device__ __forceinline__ void map_vec(int code, T a, T b, T &u, T &v) {
