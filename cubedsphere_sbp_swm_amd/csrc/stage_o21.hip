@@ -25,6 +25,21 @@ struct Pt21 {
     T K, Ud, Vd, Uc, Vc, J;
 };
 
+// Raw d21 gradient (gx, gy before the edge syncs) of the neighbour panel ed at the position k of the
+// shared edge: d0(kk) is K at tangential position kk on the edge line, dn(d) at depth d of position k.
+template <typename T, typename D0, typename DN>
+__device__ __forceinline__ void neighbour_grad21(const DevGeo<T> &g, const EdgeDesc &ed, int k, const D0 &d0,
+                                                 const DN &dn, T &gx, T &gy) {
+    const int n = g.n, a0 = ed.a_base + ed.s * k;
+    const T nK = sbp_row<21, T>(ed.tnu, n, [&](int a) {
+        const int d = ed.tnu == 0 ? a : n - 1 - a;
+        return d == 0 ? d0(k) : dn(d);
+    });
+    const T tK = sbp_row<21, T>(a0, n, [&](int a) { return d0(k + ed.s * (a - a0)); });
+    gx = (ed.nu_x ? nK : tK) / g.hxs;
+    gy = (ed.nu_x ? tK : nK) / g.hxs;
+}
+
 template <bool OTF, typename T>
 __device__ __forceinline__ Pt21<T> point21(const DevGeo<T> &g, const T *y, const T *hs, int p, int i, int j) {
     const long long id = pidx(g, p, i, j);
@@ -114,17 +129,10 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
                 const int e = slot < 2 ? slot : ey;
                 const int *ei = g.einfo + (p * 4 + e) * 8;
                 const int k0 = (slot < 2 ? ty0 : tx0) - 1;
-                auto d0 = [&](int kk, int f) -> T {
-                    if (f == 5) return T(1);
-                    if (f != 0) return T(0);
-                    return slot < 2 ? sm.gx[slot][0][kk - k0][0] : sm.gy[0][kk - k0][0];
-                };
-                auto dn = [&](int d, int f3) -> T {
-                    if (f3 != 0) return T(0);
-                    return slot < 2 ? sm.gx[slot][d][k - k0][0] : sm.gy[d][k - k0][0];
-                };
-                T r[4];
-                neighbour_raw<21, T>(g, edge_desc(ei), k, d0, dn, r);
+                auto d0 = [&](int kk) -> T { return slot < 2 ? sm.gx[slot][0][kk - k0][0] : sm.gy[0][kk - k0][0]; };
+                auto dn = [&](int d) -> T { return slot < 2 ? sm.gx[slot][d][k - k0][0] : sm.gy[d][k - k0][0]; };
+                T r[2];
+                neighbour_grad21<T>(g, edge_desc(ei), k, d0, dn, r[0], r[1]);
                 if (slot < 2) { sm.nrx[slot][kloc][0] = r[0]; sm.nrx[slot][kloc][1] = r[1]; }
                 else { sm.nry[kloc][0] = r[0]; sm.nry[kloc][1] = r[1]; }
             }
@@ -250,8 +258,10 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
     } else {
         q11 = g.Qi11[id]; q12 = g.Qi12[id]; q22 = g.Qi22[id];
     }
-    finish_point<T, MODE>(g, a, id, a.y[id], a.y[id + g.fs], a.y[id + 2 * g.fs], sm.J[ly][lx], q11, q12, q22, gx, gy, dv,
-                          cu, prefetch_point<T, MODE>(g, a, id));
+    const T h = a.y[id], u = a.y[id + g.fs], v = a.y[id + 2 * g.fs];
+    const unsigned off = point_off(g, i, j);
+    finish_point<T, MODE>(g, a, p, off, h, u, v, h * (q11 * u + q12 * v), h * (q12 * u + q22 * v), sm.J[ly][lx], gx, gy,
+                          dv, cu, prefetch_point<T, MODE>(g, a, p, off));
 }
 
 template <typename T, int TY, bool OTF>

@@ -85,10 +85,11 @@ int ens_build_tables(swm_ens *e) {
     // concatenated: every XCD then gets about the same mix of member sizes (the same for an
     // ensemble of 8 k members of each size) instead of the smallest members on the first XCDs
     // and the largest on the last.
+    const int reach = e->order == 42 ? swm::Sbp<42>::REACH : e->order == 43 ? swm::Sbp<43>::REACH : swm::Sbp<63>::REACH;
     std::vector<int> cnt(M), order(M);
     for (size_t k = 0; k < M; ++k) {
         const int n = e->m[k]->n;
-        cnt[k] = 6 * swm::tiles_along(n, e->tx) * swm::tiles_along(n, e->ty) + swm::edge_segs(n, true);
+        cnt[k] = 6 * swm::tiles_along(n, e->tx) * swm::tiles_along(n, e->ty) + swm::edge_segs(n, reach);
         order[k] = (int)k;
     }
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cnt[a] > cnt[b]; });

@@ -20,9 +20,45 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "sbp_tables.h"
 
 namespace swm {
+
+// ----------------------------------------------------------------------------------------
+// Division a / b by a denominator that several quotients share: the reciprocal is refined once
+// (hardware approximation and Newton steps), each quotient is then a product corrected by its exact
+// residual a - b q (Markstein's method: with a reciprocal good to the last place the corrected
+// quotient is the correctly rounded one), and v_div_fixup keeps zeros, infinities and NaN as IEEE
+// division gives them.  FP64: 5 + 4 instructions for the first quotient and 4 for each further one,
+// against 11 for each division on its own.  Same bits as a / b unless the quotient or the residual
+// falls into the subnormal range.
+template <typename T>
+struct Rcp {
+    T b, r;
+};
+__device__ __forceinline__ Rcp<double> rcp_of(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
+    return {b, r};
+}
+__device__ __forceinline__ Rcp<float> rcp_of(float b) {
+    float r = __builtin_amdgcn_rcpf(b);
+    r = fmaf(fmaf(-b, r, 1.0f), r, r);
+    return {b, r};
+}
+__device__ __forceinline__ double operator/(double a, const Rcp<double> &d) {
+    const double q = a * d.r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-d.b, q, a), d.r, q), d.b, a);
+}
+__device__ __forceinline__ float operator/(float a, const Rcp<float> &d) {
+    float q = a * d.r;
+    q = fmaf(fmaf(-d.b, q, a), d.r, q);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d.b, q, a), d.r, q), d.b, a);
+}
 
 // ----------------------------------------------------------------------------------------
 // Geometry and per-launch arguments
@@ -37,7 +73,7 @@ struct DevGeo {
     const double *tanA;                    // tan(alpha_i), i = 0..n-1 (metric evaluated on the fly)
     int n, pitch;
     long long fs;                          // elements per field (6*n*pitch)
-    T hxs;                                 // hx*scale
+    T hxs, rhxs;                           // hx*scale and its reciprocal, correctly rounded
     T hx, scale, grav;
 };
 
@@ -71,22 +107,14 @@ SWM_HD constexpr bool tile_shape_ok(int tx, int ty) {
 // tiles_along(n, t) tiles of t points, the b-th starting at point 1 + b*t.
 SWM_HD constexpr int tiles_along(int n, int t) { return (n - 2 + t - 1) / t; }
 
-// The panel-edge points are computed by edge segments of edge_seg_len(n) consecutive points:
-// per panel the x-edges (i = 0 and i = n-1, positions j = 0..n-1, cube corners included) and
-// the y-edges (j = 0 and j = n-1, positions i = 1..n-2).  A single cube with small panels
-// takes shorter segments, i.e. more blocks for the same edge work; the persistent ensemble
-// loop, where every task costs a fixed overhead, keeps the longest.
-constexpr int EDGE_SEG = 64;  // longest segment (LDS sizing)
-SWM_HD constexpr int edge_seg_len(int n, bool persist = false) { return (persist || n > 256) ? EDGE_SEG : 48; }
-SWM_HD constexpr int edge_segs_x(int n, bool persist = false) {
-    return (n + edge_seg_len(n, persist) - 1) / edge_seg_len(n, persist);
-}
-SWM_HD constexpr int edge_segs_y(int n, bool persist = false) {
-    return (n - 2 + edge_seg_len(n, persist) - 1) / edge_seg_len(n, persist);
-}
-SWM_HD constexpr int edge_segs(int n, bool persist = false) {
-    return 6 * 2 * (edge_segs_x(n, persist) + edge_segs_y(n, persist));
-}
+// The panel-edge points are computed by edge segments of consecutive points: per panel the
+// x-edges (i = 0 and i = n-1, positions j = 0..n-1, cube corners included) and the y-edges (j = 0
+// and j = n-1, positions i = 1..n-2).  A segment and the REACH points its tangential rows read on
+// either side fill the 64 lanes of a wave.
+SWM_HD constexpr int edge_seg_len(int reach) { return 64 - 2 * reach; }
+SWM_HD constexpr int edge_segs_x(int n, int reach) { return (n + edge_seg_len(reach) - 1) / edge_seg_len(reach); }
+SWM_HD constexpr int edge_segs_y(int n, int reach) { return (n - 2 + edge_seg_len(reach) - 1) / edge_seg_len(reach); }
+SWM_HD constexpr int edge_segs(int n, int reach) { return 6 * 2 * (edge_segs_x(n, reach) + edge_segs_y(n, reach)); }
 
 template <typename T>
 struct EnsMember {
@@ -104,8 +132,7 @@ struct Derived {
     T hu, hv;  // h*ut, h*vt (kept in registers for the point's own output)
 };
 
-// WHICH: 0 all five inputs, 2 only those of the y-derivative (K, J*hv, J*(-u/J))
-template <typename T, int WHICH = 0>
+template <typename T>
 __device__ __forceinline__ Derived<T> make_derived(T h, T u, T v, T J, T q11, T q12, T q22, T hsv, T grav) {
     Derived<T> d;
     const T ut = q11 * u + q12 * v;
@@ -114,15 +141,14 @@ __device__ __forceinline__ Derived<T> make_derived(T h, T u, T v, T J, T q11, T 
     const T hv = h * vt;
     T K = (u * ut + v * vt) / T(2);
     K = K + grav * h + grav * hsv;
+    const Rcp<T> rJ = rcp_of(J);
     d.K = K;
     d.hu = hu;
     d.hv = hv;
-    if constexpr (WHICH != 2) {
-        d.Gxd = J * hu;
-        d.Gxc = J * (v / J);
-    }
+    d.Gxd = J * hu;
+    d.Gxc = J * (v / rJ);
     d.Gyd = J * hv;
-    d.Gyc = J * (-u / J);
+    d.Gyc = J * (-u / rJ);
     return d;
 }
 
@@ -152,24 +178,26 @@ __device__ __forceinline__ Metric metric_otf(const double *tanA, int i, int j) {
     return m;
 }
 
-template <bool OTF, typename T>
-__device__ __forceinline__ T metric_J(const DevGeo<T> &g, int p, int i, int j) {
-    if constexpr (OTF) return metric_otf(g.tanA, i, j).J;
-    else return g.J[midx(g, p, i, j)];
+// Element at a byte offset from a uniform base: the offset stays a 32-bit vector register beside a
+// scalar base (a panel of the largest grid is 0.54 GB).
+template <typename T>
+__device__ __forceinline__ T &at_byte(T *base, unsigned off) {
+    return *reinterpret_cast<T *>(reinterpret_cast<std::conditional_t<std::is_const_v<T>, const char, char> *>(base) + off);
 }
 
-template <bool OTF, typename T, int WHICH = 0>
-__device__ __forceinline__ Derived<T> derived_global(const DevGeo<T> &g, const T *y, const T *hs, int p, int i, int j) {
-    const long long id = pidx(g, p, i, j);
-    if constexpr (OTF) {
-        const Metric m = metric_otf(g.tanA, i, j);
-        return make_derived<T, WHICH>(y[id], y[id + g.fs], y[id + 2 * g.fs], (T)m.J, (T)m.Qi11, (T)m.Qi12,
-                                      (T)m.Qi22, hs ? hs[id] : T(0), g.grav);
-    } else {
-        const long long mid = midx(g, p, i, j);
-        return make_derived<T, WHICH>(y[id], y[id + g.fs], y[id + 2 * g.fs], g.J[mid], g.Qi11[mid], g.Qi12[mid],
-                                      g.Qi22[mid], hs ? hs[id] : T(0), g.grav);
-    }
+// One panel of the inputs of a stage: state, orography and metric, and the byte offset of a point
+template <typename T>
+struct PanelIn {
+    const T *h, *u, *v, *hs, *J, *q11, *q12, *q22;
+};
+template <typename T>
+__device__ __forceinline__ PanelIn<T> panel_in(const DevGeo<T> &g, const T *y, const T *hs, int p) {
+    const long long o = (long long)p * g.n * g.pitch, m = (long long)p * g.mps;
+    return {y + o, y + g.fs + o, y + 2 * g.fs + o, hs ? hs + o : nullptr, g.J + m, g.Qi11 + m, g.Qi12 + m, g.Qi22 + m};
+}
+template <typename T>
+__device__ __forceinline__ unsigned point_off(const DevGeo<T> &g, int i, int j) {
+    return (__umul24((unsigned)j, (unsigned)g.pitch) + (unsigned)i) * (unsigned)sizeof(T);
 }
 
 // Raw inputs of one point (state, metric, orography) and the derived stencil inputs formed
@@ -180,26 +208,25 @@ struct RawPoint {
 };
 
 template <bool OTF, typename T>
-__device__ __forceinline__ RawPoint<T> load_point(const DevGeo<T> &g, const T *y, const T *hs, int p, int i, int j) {
-    const long long id = pidx(g, p, i, j);
+__device__ __forceinline__ RawPoint<T> load_point(const DevGeo<T> &g, const PanelIn<T> &in, int i, int j) {
+    const unsigned o = point_off(g, i, j);
     RawPoint<T> r;
-    r.h = y[id];
-    r.u = y[id + g.fs];
-    r.v = y[id + 2 * g.fs];
+    r.h = at_byte(in.h, o);
+    r.u = at_byte(in.u, o);
+    r.v = at_byte(in.v, o);
     if constexpr (OTF) {
         const Metric m = metric_otf(g.tanA, i, j);
         r.J = (T)m.J; r.q11 = (T)m.Qi11; r.q12 = (T)m.Qi12; r.q22 = (T)m.Qi22;
     } else {
-        const long long mid = midx(g, p, i, j);
-        r.J = g.J[mid]; r.q11 = g.Qi11[mid]; r.q12 = g.Qi12[mid]; r.q22 = g.Qi22[mid];
+        r.J = at_byte(in.J, o); r.q11 = at_byte(in.q11, o); r.q12 = at_byte(in.q12, o); r.q22 = at_byte(in.q22, o);
     }
-    r.hs = hs ? hs[id] : T(0);
+    r.hs = in.hs ? at_byte(in.hs, o) : T(0);
     return r;
 }
 
-template <typename T, int WHICH = 0>
+template <typename T>
 __device__ __forceinline__ Derived<T> derived_of(const DevGeo<T> &g, const RawPoint<T> &r) {
-    return make_derived<T, WHICH>(r.h, r.u, r.v, r.J, r.q11, r.q12, r.q22, r.hs, g.grav);
+    return make_derived<T>(r.h, r.u, r.v, r.J, r.q11, r.q12, r.q22, r.hs, g.grav);
 }
 
 // ----------------------------------------------------------------------------------------
@@ -255,6 +282,65 @@ __device__ __forceinline__ T sbp_row(int t, int n, const G &get) {
     if (t >= S::NE && t < n - S::NE) return sbp_row_in<ORD, T>(t, get);
     if (t < S::NE) return sbp_left_dispatch<ORD, T>(t, get, std::make_integer_sequence<int, S::NE>{});
     return sbp_right_dispatch<ORD, T>(t - (n - S::NE), n, get, std::make_integer_sequence<int, S::NE>{});
+}
+
+// The rows of the first derivative as a table: classes 0 .. NE-1 the left closure rows, NE the
+// interior row, NE+1 .. 2 NE the right closure rows.  Kernels whose points mix the classes read the
+// weights from an LDS copy: one code path for every point of a wave, where the rows written out
+// with constant weights (sbp_row) take a branch and its code per closure row.
+template <int ORD>
+struct RowWeights {
+    using S = Sbp<ORD>;
+    static constexpr int NC = 2 * S::NE + 1, NW = S::NW > S::WIN ? S::NW : S::WIN, SIZE = NC * NW;
+    double w[SIZE];
+    constexpr RowWeights() : w() {
+        for (int r = 0; r < S::NE; ++r)
+            for (int m = 0; m < S::last[r]; ++m) {
+                w[r * NW + m] = S::Ql[r][m];
+                w[(2 * S::NE - r) * NW + m] = -1.0 * S::Ql[r][S::last[r] - 1 - m];
+            }
+        for (int m = 0; m < S::WIN; ++m) w[S::NE * NW + m] = S::Qin[m];
+    }
+    static constexpr unsigned packed_last() {
+        unsigned v = 0;
+        for (int r = 0; r < S::NE; ++r) v |= (unsigned)S::last[r] << (4 * r);
+        return v;
+    }
+};
+template <int ORD>
+__device__ const RowWeights<ORD> row_weights = RowWeights<ORD>();
+
+// The row of output index t on a line of n points: first input index, number of inputs, class
+struct RowAt {
+    int base, cnt, cls;
+};
+template <int ORD>
+__device__ __forceinline__ RowAt row_at(int t, int n) {
+    using S = Sbp<ORD>;
+    constexpr unsigned LASTS = RowWeights<ORD>::packed_last();
+    if (t < S::NE) return {0, (int)((LASTS >> (4 * t)) & 15u), t};
+    if (t < n - S::NE) return {t + S::INSHIFT, S::WIN, S::NE};
+    const int c = (int)((LASTS >> (4 * (n - 1 - t))) & 15u);
+    return {n - c, c, 2 * S::NE - (n - 1 - t)};
+}
+// the row applied to three fields, f(m, a, b, c) giving their inputs at index base + m
+template <int ORD, typename T, typename F>
+__device__ __forceinline__ void row_apply3(const T *__restrict__ tab, const RowAt &r, const F &f, T &a, T &b, T &c) {
+    constexpr int NW = RowWeights<ORD>::NW;
+    const T *w = tab + r.cls * NW;
+    T x, y, z;
+    f(0, x, y, z);
+    a = w[0] * x;
+    b = w[0] * y;
+    c = w[0] * z;
+#pragma unroll
+    for (int m = 1; m < NW; ++m)
+        if (m < r.cnt) {
+            f(m, x, y, z);
+            a = a + w[m] * x;
+            b = b + w[m] * y;
+            c = c + w[m] * z;
+        }
 }
 
 // slot of a panel-edge point in a panel's compact edge buffer (4 (n-1) slots)

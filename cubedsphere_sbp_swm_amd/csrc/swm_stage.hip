@@ -7,52 +7,44 @@
 namespace swm {
 
 
-// Tile of TX x TY output points per workgroup of TX*TY threads (one point per thread).  Every
-// tiling has 512 threads: 64 x 8, 32 x 16 or 16 x 32 points.
-template <int ORD, typename T, int TX, int TY>
-struct Tile {
-    static constexpr int R = Sbp<ORD>::REACH;    // halo of the stencil inputs
-    static constexpr int D = Sbp<ORD>::last[0];  // points of the boundary row 0 (normal depth)
-    static constexpr int LX = TX + 2 * R;
-    static constexpr int LY = TY + 2 * R;
-    static constexpr int NT = TX * TY;
-};
-
-// LDS of one tile.  K lives on the cross-shaped region; the x-derivative inputs only on the
-// tile rows, the y-derivative inputs only on the tile columns.
-template <int ORD, typename T, int TX, int TY>
-struct TileSmem {
-    using C = Tile<ORD, T, TX, TY>;
-    static constexpr int R = C::R, LX = C::LX, LY = C::LY;
+// LDS of one tile of TX x TY output points (one point per thread) and its halo of R points.  K lives
+// on the cross-shaped region; the x-derivative inputs only on the tile rows, the y-derivative inputs
+// only on the tile columns.
+template <typename T, int TX, int TY, int R>
+struct TileFields {
+    static constexpr int LX = TX + 2 * R, LY = TY + 2 * R;
     T K[LY][LX];
     T Gxd[TY][LX], Gxc[TY][LX];
     T Gyd[LY][TX], Gyc[LY][TX];
 };
 
-// LDS of one edge segment: the stencil inputs along the edge of the own panel (side 0) and of
-// the neighbour across the edge (side 1), and at the cube corners the neighbour across the
-// other edge (slot 0: position 0, slot 1: position n-1).
+// halo of a tile: what the interior rows read (tiles of interior rows only), or what any row reads
+template <int ORD, bool INNER>
+constexpr int tile_halo() { return INNER ? -Sbp<ORD>::INSHIFT : Sbp<ORD>::REACH; }
+
+// LDS of one edge segment, lane l of a wave at position k0 - REACH + l along the edge: the stencil
+// inputs of the own panel (side 0) and of the neighbour across the edge (side 1), and at the cube
+// corners of the neighbour across the other edge (slot 0: position 0, slot 1: position n-1).
 template <int ORD, typename T>
-struct EdgeSmem {
+struct EdgeFields {
     static constexpr int R = Sbp<ORD>::REACH, D = Sbp<ORD>::last[0];
-    T e0[2][EDGE_SEG + 2 * R][6];   // depth 0: K, Gxd, Gyd, Gxc, Gyc, J
-    T en[2][D - 1][EDGE_SEG][3];    // depth >= 1: K and the two inputs along the normal axis
-    T c0[2][2 * R + 1][6];
-    T cn[2][D - 1][3];
+    T tan[2][3][64];          // depth 0: K and the two inputs of the rows along the edge
+    T nrm[2][D][3][64];       // depths 0..D-1: K and the two inputs of the rows across it
+    T J[2][64];
+    T ctan[2][3][2 * R + 1], cnrm[2][D][3], cJ[2];
+    T raw[3][4][64];          // gx, gy, div, curl before the syncs: own, neighbour, corner (lane = slot)
 };
 
 template <int ORD, typename T, int TX, int TY>
-union Smem {
-    TileSmem<ORD, T, TX, TY> t;
-    EdgeSmem<ORD, T> e;
+struct Smem {
+    T tab[RowWeights<ORD>::SIZE];   // derivative rows (edge segments and tiles with closure rows)
+    union {
+        TileFields<T, TX, TY, tile_halo<ORD, true>()> in;
+        TileFields<T, TX, TY, tile_halo<ORD, false>()> t;
+        EdgeFields<ORD, T> e;
+    };
 };
 
-// Raw values (gx, gy, div, curl before the edge syncs) of a panel at the point k of one of
-// its edges, from strips of stencil inputs along that edge.  ei describes the edge in the
-// neighbour-table form (panel, normal axis is x, normal index, tangential base and step); for
-// a neighbour panel it maps the local position k to the neighbour's tangential index.
-// d0(kk, f) returns field f (0 K, 1 Gxd, 2 Gyd, 3 Gxc, 4 Gyc, 5 J) at tangential index kk,
-// depth 0; dn(d, f3) the normal-axis inputs (0 K, 1 Gnd, 2 Gnc) at depth d >= 1.
 // One panel edge in neighbour-table form: panel, normal axis is x, normal index of the edge
 // line, tangential index = a_base + s * (local position), component code of the vector halo.
 struct EdgeDesc {
@@ -60,51 +52,23 @@ struct EdgeDesc {
 };
 __device__ __forceinline__ EdgeDesc edge_desc(const int *ei) { return {ei[0], ei[1], ei[2], ei[3], ei[4], ei[5]}; }
 
-template <int ORD, typename T, typename D0, typename DN>
-__device__ __forceinline__ void neighbour_raw(const DevGeo<T> &g, const EdgeDesc &ed, int k, const D0 &d0,
-                                              const DN &dn, T out[4]) {
-    const int n = g.n;
-    const int nu_x = ed.nu_x, tnu = ed.tnu, a0 = ed.a_base + ed.s * k, s = ed.s;
-    auto nu_get = [&](int fld3, int a) {  // along the normal axis of the neighbour
-        const int d = tnu == 0 ? a : n - 1 - a;
-        if (d == 0) return d0(k, fld3 == 0 ? 0 : (nu_x ? (fld3 == 1 ? 1 : 3) : (fld3 == 1 ? 2 : 4)));
-        return dn(d, fld3);
-    };
-    auto tau_get = [&](int fld, int a) { return d0(k + s * (a - a0), fld); };
-    const T nK = sbp_row<ORD, T>(tnu, n, [&](int a) { return nu_get(0, a); });
-    const T nD = sbp_row<ORD, T>(tnu, n, [&](int a) { return nu_get(1, a); });
-    const T nC = sbp_row<ORD, T>(tnu, n, [&](int a) { return nu_get(2, a); });
-    const int fD = nu_x ? 2 : 1, fC = nu_x ? 4 : 3;  // inputs along the tangential axis
-    const T tK = sbp_row<ORD, T>(a0, n, [&](int a) { return tau_get(0, a); });
-    const T tD = sbp_row<ORD, T>(a0, n, [&](int a) { return tau_get(fD, a); });
-    const T tC = sbp_row<ORD, T>(a0, n, [&](int a) { return tau_get(fC, a); });
-    const T dxK = nu_x ? nK : tK, dyK = nu_x ? tK : nK;
-    const T dxD = nu_x ? nD : tD, dyD = nu_x ? tD : nD;
-    const T dxC = nu_x ? nC : tC, dyC = nu_x ? tC : nC;
-    const T Jd = d0(k, 5) * g.hx * g.scale;
-    out[0] = dxK / g.hxs;
-    out[1] = dyK / g.hxs;
-    out[2] = (dxD + dyD) / Jd;
-    out[3] = (dxC + dyC) / Jd;
-}
-
 // Values of the output point that only the final combination reads (Coriolis parameter, RK
-// stage vectors); loaded at the start of the tile so that their latency overlaps the stencil
-// phases.
+// stage vectors); loaded ahead of it so that their latency overlaps the stencil phases.
 template <typename T>
 struct OutPre {
     T f, v0[3], acc[3];
 };
 
 template <typename T, int MODE>
-__device__ __forceinline__ OutPre<T> prefetch_point(const DevGeo<T> &g, const StageArgs<T> &a, long long id) {
+__device__ __forceinline__ OutPre<T> prefetch_point(const DevGeo<T> &g, const StageArgs<T> &a, int p, unsigned off) {
     OutPre<T> o{};
     if constexpr (MODE == MODE_CURL) return o;
-    o.f = g.f[id];
+    const long long pb = (long long)p * g.n * g.pitch;
+    o.f = at_byte(g.f + pb, off);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        if constexpr (MODE == MODE_STAGE23) o.v0[k] = a.v0[id + k * g.fs];
-        if constexpr (MODE == MODE_STAGE23 || MODE == MODE_STAGE4) o.acc[k] = a.acc[id + k * g.fs];
+        if constexpr (MODE == MODE_STAGE23) o.v0[k] = at_byte(a.v0 + (pb + k * g.fs), off);
+        if constexpr (MODE == MODE_STAGE23 || MODE == MODE_STAGE4) o.acc[k] = at_byte((const T *)a.acc + (pb + k * g.fs), off);
     }
     return o;
 }
@@ -113,102 +77,99 @@ __device__ __forceinline__ OutPre<T> prefetch_point(const DevGeo<T> &g, const St
 // (coriolis_colocated_mod.f90:97-98, operator_swm_mod.f90:95-101, rk4_mod.f90:28-40)
 // hu = h*ut, hv = h*vt: the mass fluxes of the point (u, v are read by stage 1 only)
 template <typename T, int MODE>
-__device__ __forceinline__ void finish_point_hv(const DevGeo<T> &g, const StageArgs<T> &a, long long id, T h, T u, T v,
-                                                T hu, T hv, T Jv, T gx, T gy, T dv, T cu, const OutPre<T> &pre) {
+__device__ __forceinline__ void finish_point(const DevGeo<T> &g, const StageArgs<T> &a, int p, unsigned off, T h, T u,
+                                             T v, T hu, T hv, T Jv, T gx, T gy, T dv, T cu, const OutPre<T> &pre) {
+    const long long pb = (long long)p * g.n * g.pitch;
+    T *out = a.out + pb;
     if constexpr (MODE == MODE_CURL) {
-        a.out[id] = cu;
+        at_byte(out, off) = cu;
         return;
     }
-    if (a.zeta) a.zeta[id] = cu;
+    if (a.zeta) at_byte(a.zeta + pb, off) = cu;
     const T fz = pre.f + cu;
-    const T cor_u = fz * hv / h * Jv;
-    const T cor_v = -(fz * hu / h * Jv);
-    const T kh = -dv;
-    const T ku = -gx + cor_u;
-    const T kv = -gy + cor_v;
-
-    if constexpr (MODE == MODE_RHS) {
-        a.out[id] = kh;
-        a.out[id + g.fs] = ku;
-        a.out[id + 2 * g.fs] = kv;
-    } else if constexpr (MODE == MODE_STAGE1) {
-        a.out[id] = h + a.cy * kh;
-        a.out[id + g.fs] = u + a.cy * ku;
-        a.out[id + 2 * g.fs] = v + a.cy * kv;
-        a.acc[id] = h + a.cacc * kh;
-        a.acc[id + g.fs] = u + a.cacc * ku;
-        a.acc[id + 2 * g.fs] = v + a.cacc * kv;
-    } else if constexpr (MODE == MODE_STAGE23) {
-        a.out[id] = pre.v0[0] + a.cy * kh;
-        a.out[id + g.fs] = pre.v0[1] + a.cy * ku;
-        a.out[id + 2 * g.fs] = pre.v0[2] + a.cy * kv;
-        a.acc[id] = pre.acc[0] + a.cacc * kh;
-        a.acc[id + g.fs] = pre.acc[1] + a.cacc * ku;
-        a.acc[id + 2 * g.fs] = pre.acc[2] + a.cacc * kv;
-    } else if constexpr (MODE == MODE_STAGE4) {
-        a.out[id] = pre.acc[0] + a.cy * kh;
-        a.out[id + g.fs] = pre.acc[1] + a.cy * ku;
-        a.out[id + 2 * g.fs] = pre.acc[2] + a.cy * kv;
+    const Rcp<T> rh = rcp_of(h);
+    const T cor_u = fz * hv / rh * Jv;
+    const T cor_v = -(fz * hu / rh * Jv);
+    const T k[3] = {-dv, -gx + cor_u, -gy + cor_v}, y[3] = {h, u, v};
+    T *acc = a.acc + pb;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const long long fc = c * g.fs;
+        if constexpr (MODE == MODE_RHS) {
+            at_byte(out + fc, off) = k[c];
+        } else if constexpr (MODE == MODE_STAGE1) {
+            at_byte(out + fc, off) = y[c] + a.cy * k[c];
+            at_byte(acc + fc, off) = y[c] + a.cacc * k[c];
+        } else if constexpr (MODE == MODE_STAGE23) {
+            at_byte(out + fc, off) = pre.v0[c] + a.cy * k[c];
+            at_byte(acc + fc, off) = pre.acc[c] + a.cacc * k[c];
+        } else if constexpr (MODE == MODE_STAGE4) {
+            at_byte(out + fc, off) = pre.acc[c] + a.cy * k[c];
+        }
     }
 }
 
-template <typename T, int MODE>
-__device__ __forceinline__ void finish_point(const DevGeo<T> &g, const StageArgs<T> &a, long long id, T h, T u, T v,
-                                             T Jv, T q11, T q12, T q22, T gx, T gy, T dv, T cu, const OutPre<T> &pre) {
-    const T ut = q11 * u + q12 * v;
-    const T vt = q12 * u + q22 * v;
-    finish_point_hv<T, MODE>(g, a, id, h, u, v, h * ut, h * vt, Jv, gx, gy, dv, cu, pre);
+// the derivative rows from memory into LDS; the caller's barrier follows
+template <int ORD, typename T>
+__device__ __forceinline__ void load_rows(T *tab, int tid, int nthreads) {
+    for (int c = tid; c < RowWeights<ORD>::SIZE; c += nthreads) tab[c] = (T)row_weights<ORD>.w[c];
 }
 
 // One TX x TY tile of panel p starting at (tx0, ty0) >= (1, 1): the whole RHS + RK stage update
 // of its points off the panel edges (the panel-edge points belong to the edge segments).
-// INNER: the tile lies inside NE <= i, j < n - NE (inner_tile), so every point of it and of its
-// halo exists, none is on a panel edge and every derivative row is an interior one; its guards
-// and closure branches are then known at compile time.
-template <int ORD, typename T, int MODE, int TX, int TY, bool OTF, bool PERSIST = false, bool INNER = false>
+// INNER (inner_tile): every derivative row of the tile is an interior one, so every point of it and
+// of its halo exists and none is on a panel edge; its halo is the REACH of the interior row (2 points
+// for sbp42 and sbp43, 3 for sbp63, against 3, 5, 5 for the closure rows), its guards vanish and its
+// rows have constant weights.  The other tiles take their rows from the table.
+// At C384 sbp42 FP64 (64 x 8, metric read) an RK4 step takes 83 us in a long run, 20.7 us per stage: the
+// kernel moves about 135 MB per stage 2/3 at the 7 TB/s that a copy of cache-resident buffers of this
+// size reaches.  Wider halos, a branch and its code per closure row, 11-instruction divisions, 64-bit
+// offsets and panel-major tile order (metric read once per panel) took 24-25 us.
+template <int ORD, typename T, int MODE, int TX, int TY, bool OTF, bool PERSIST, bool INNER>
 __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T> &a, int p, int tx0, int ty0,
-                                           TileSmem<ORD, T, TX, TY> &sm) {
-    using C = Tile<ORD, T, TX, TY>;
-    constexpr int R = C::R, NT = C::NT;
+                                           TileFields<T, TX, TY, tile_halo<ORD, INNER>()> &sm, T *tab) {
+    constexpr int R = tile_halo<ORD, INNER>(), NT = TX * TY;
     const int n = g.n;
     // in the persistent ensemble loop the thread index is made opaque per tile, so that the
     // thread-index arithmetic is recomputed per tile instead of being hoisted out of the loop
     // and held in registers
     int tid = threadIdx.x;
     if constexpr (PERSIST) asm volatile("" : "+v"(tid));
-    const T *y = a.y;
-    OutPre<T> pre{};
+    const PanelIn<T> in = panel_in(g, a.y, a.hs, p);
 
     // ---- load phase: every thread loads its own tile point (kept in registers for the output
-    // phase), plus at most NXH points of the x-halo columns and NYH points of the y-halo rows;
-    // all global loads are issued before any derived value is formed, so that they are in flight
-    // together. ----
-    constexpr int NXH = (2 * R * TY + NT - 1) / NT, NYH = (2 * R * TX + NT - 1) / NT;
+    // phase), plus at most NH halo points, the y-halo rows first (whole waves), then the x-halo
+    // columns; all global loads are issued before any derived value is formed, so that they are in
+    // flight together. ----
+    constexpr int NYH = 2 * R * TX, NXH = 2 * R * TY, NH = (NYH + NXH + NT - 1) / NT;
     const int tx = tid % TX, ty = tid / TX;
     const int i = tx0 + tx, j = ty0 + ty;
     const bool own_ok = INNER || (i < n && j < n);
     RawPoint<T> own{};
-    if (own_ok) own = load_point<OTF>(g, y, a.hs, p, i, j);
-    RawPoint<T> rx[NXH], ry[NYH];
-    bool okx[NXH], oky[NYH];
+    if (own_ok) own = load_point<OTF>(g, in, i, j);
+    RawPoint<T> rh[NH];
+    int hc[NH], hr[NH];   // tile column and row of the halo point, relative to (tx0, ty0)
+    bool okh[NH];
 #pragma unroll
-    for (int k = 0; k < NXH; ++k) {
+    for (int k = 0; k < NH; ++k) {
         const int c = tid + k * NT;
-        const int r = c / (2 * R), q = c - r * (2 * R);
-        const int lx = q < R ? q : q + TX;
-        const int xi = tx0 - R + lx, xj = ty0 + r;
-        okx[k] = c < 2 * R * TY && (INNER || (xi >= 0 && xi < n && xj < n));
-        if (okx[k]) rx[k] = load_point<OTF>(g, y, a.hs, p, xi, xj);
+        if (c < NYH) {
+            const int r = c / TX;
+            hc[k] = c - r * TX;
+            hr[k] = r < R ? r - R : r - R + TY;
+        } else {
+            const int q = c - NYH, r = q / (2 * R), x = q - r * (2 * R);
+            hr[k] = r;
+            hc[k] = x < R ? x - R : x - R + TX;
+        }
+        okh[k] = c < NYH + NXH;
+        if constexpr (!INNER) {
+            const int hi = tx0 + hc[k], hj = ty0 + hr[k];
+            okh[k] = okh[k] && hi >= 0 && hj >= 0 && hi < n && hj < n;
+        }
+        if (okh[k]) rh[k] = load_point<OTF>(g, in, tx0 + hc[k], ty0 + hr[k]);
     }
-#pragma unroll
-    for (int k = 0; k < NYH; ++k) {
-        const int c = tid + k * NT;
-        const int r = c / TX, cx = c - r * TX;
-        const int ly = r < R ? r : r + TY;
-        const int yi = tx0 + cx, yj = ty0 - R + ly;
-        oky[k] = c < 2 * R * TX && (INNER || (yi < n && yj >= 0 && yj < n));
-        if (oky[k]) ry[k] = load_point<OTF>(g, y, a.hs, p, yi, yj);
-    }
+    if constexpr (!INNER) load_rows<ORD, T>(tab, tid, NT);
     // of the own point only h, u, v, J and the mass fluxes h*ut, h*vt stay live for the output
     // phase (the same products the Coriolis term forms)
     T own_hu = T(0), own_hv = T(0);
@@ -223,69 +184,73 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
         sm.Gyc[ty + R][tx] = d.Gyc;
     }
 #pragma unroll
-    for (int k = 0; k < NXH; ++k) {
-        if (!okx[k]) continue;
-        const int c = tid + k * NT;
-        const int r = c / (2 * R), q = c - r * (2 * R);
-        const int lx = q < R ? q : q + TX;
-        const Derived<T> d = derived_of(g, rx[k]);
-        sm.K[r + R][lx] = d.K;
-        sm.Gxd[r][lx] = d.Gxd;
-        sm.Gxc[r][lx] = d.Gxc;
-    }
-#pragma unroll
-    for (int k = 0; k < NYH; ++k) {
-        if (!oky[k]) continue;
-        const int c = tid + k * NT;
-        const int r = c / TX, cx = c - r * TX;
-        const int ly = r < R ? r : r + TY;
-        const Derived<T> d = derived_of<T, 2>(g, ry[k]);
-        sm.K[ly][cx + R] = d.K;
-        sm.Gyd[ly][cx] = d.Gyd;
-        sm.Gyc[ly][cx] = d.Gyc;
+    for (int k = 0; k < NH; ++k) {
+        if (!okh[k]) continue;
+        const Derived<T> d = derived_of(g, rh[k]);
+        sm.K[hr[k] + R][hc[k] + R] = d.K;
+        if (tid + k * NT < NYH) {
+            sm.Gyd[hr[k] + R][hc[k]] = d.Gyd;
+            sm.Gyc[hr[k] + R][hc[k]] = d.Gyc;
+        } else {
+            sm.Gxd[hr[k]][hc[k] + R] = d.Gxd;
+            sm.Gxc[hr[k]][hc[k] + R] = d.Gxc;
+        }
     }
     // the output point's Coriolis parameter and RK vectors: issued after the load phase (issued
-    // with it, they raised its register peak from 74 to 88 VGPRs at FP64, one wave per SIMD
-    // less), in flight across the barrier and the stencil phase
-    if (INNER || (i > 0 && j > 0 && i < n - 1 && j < n - 1)) pre = prefetch_point<T, MODE>(g, a, pidx(g, p, i, j));
+    // with it, they raised its register peak by 14 VGPRs at FP64), in flight across the barrier and
+    // the stencil phase
+    const bool out_ok = INNER || (i < n - 1 && j < n - 1);
+    const unsigned off = point_off(g, i, j);
+    OutPre<T> pre{};
+    if (out_ok) pre = prefetch_point<T, MODE>(g, a, p, off);
     __syncthreads();
 
     // ---- output phase: the thread's own point ----
-    if (!INNER && (i <= 0 || j <= 0 || i >= n - 1 || j >= n - 1)) return;
+    if (!out_ok) return;
     const int lx = tx + R, ly = ty + R;
-    auto d1 = [&](int t, const auto &get) {
-        if constexpr (INNER) return sbp_row_in<ORD, T>(t, get);
-        else return sbp_row<ORD, T>(t, n, get);
-    };
-    const T dxK = d1(i, [&](int ai) { return sm.K[ly][ai - tx0 + R]; });
-    const T dyK = d1(j, [&](int aj) { return sm.K[aj - ty0 + R][lx]; });
-    const T dxD = d1(i, [&](int ai) { return sm.Gxd[ty][ai - tx0 + R]; });
-    const T dyD = d1(j, [&](int aj) { return sm.Gyd[aj - ty0 + R][tx]; });
-    const T dxC = d1(i, [&](int ai) { return sm.Gxc[ty][ai - tx0 + R]; });
-    const T dyC = d1(j, [&](int aj) { return sm.Gyc[aj - ty0 + R][tx]; });
-    const long long id = pidx(g, p, i, j);
-    const T Jd = own.J * g.hx * g.scale;
-    const T gx = dxK / g.hxs;
-    const T gy = dyK / g.hxs;
-    const T dv = (dxD + dyD) / Jd;
-    const T cu = (dxC + dyC) / Jd;
-
-    finish_point_hv<T, MODE>(g, a, id, own.h, own.u, own.v, own_hu, own_hv, own.J, gx, gy, dv, cu, pre);
+    T dxK, dyK, dxD, dyD, dxC, dyC;
+    if constexpr (INNER) {
+        dxK = sbp_row_in<ORD, T>(lx, [&](int q) { return sm.K[ly][q]; });
+        dyK = sbp_row_in<ORD, T>(ly, [&](int q) { return sm.K[q][lx]; });
+        dxD = sbp_row_in<ORD, T>(lx, [&](int q) { return sm.Gxd[ty][q]; });
+        dyD = sbp_row_in<ORD, T>(ly, [&](int q) { return sm.Gyd[q][tx]; });
+        dxC = sbp_row_in<ORD, T>(lx, [&](int q) { return sm.Gxc[ty][q]; });
+        dyC = sbp_row_in<ORD, T>(ly, [&](int q) { return sm.Gyc[q][tx]; });
+    } else {
+        const RowAt rx = row_at<ORD>(i, n), ry = row_at<ORD>(j, n);
+        const int bx = rx.base - tx0 + R, by = ry.base - ty0 + R;
+        row_apply3<ORD, T>(tab, rx, [&](int m, T &x, T &y, T &z) {
+            x = sm.K[ly][bx + m]; y = sm.Gxd[ty][bx + m]; z = sm.Gxc[ty][bx + m];
+        }, dxK, dxD, dxC);
+        row_apply3<ORD, T>(tab, ry, [&](int m, T &x, T &y, T &z) {
+            x = sm.K[by + m][lx]; y = sm.Gyd[by + m][tx]; z = sm.Gyc[by + m][tx];
+        }, dyK, dyD, dyC);
+    }
+    const Rcp<T> rhxs{g.hxs, g.rhxs}, rJd = rcp_of(own.J * g.hx * g.scale);
+    finish_point<T, MODE>(g, a, p, off, own.h, own.u, own.v, own_hu, own_hv, own.J, dxK / rhxs, dyK / rhxs,
+                          (dxD + dyD) / rJd, (dxC + dyC) / rJd, pre);
 }
 
-// Edge segment `seg` of the cube (edge_segs(n, PERSIST) per cube): positions k0..k1-1 of one
-// panel edge, at most edge_seg_len(n, PERSIST) points.  The own panel's and the neighbour's stencil inputs along the edge go to LDS; each
-// point then forms both panels' raw values, applies the scalar and covariant vector edge syncs
-// (ecs_Ah_vec_sync_mod.f90:77-124 with (U, V) = (gy, gx), halo_Ah_scalar_sync_mod.f90:52-93,
-// in the reference's operand order) and the RK stage update.
+// Edge segment `seg` of the cube (edge_segs(n, REACH) per cube): positions k0..k1-1 of one panel
+// edge, at most 64 - 2 REACH points.  Both panels' stencil inputs along the edge go to LDS, one line of
+// one depth per wave; then one wave per panel forms the raw values of its side's one-sided rows (a
+// third those of the corners' third panel), and the first wave applies the scalar and covariant
+// vector edge syncs (ecs_Ah_vec_sync_mod.f90:77-124 with (U, V) = (gy, gx),
+// halo_Ah_scalar_sync_mod.f90:52-93, in the reference's operand order) and the RK stage update.
+// These blocks are the longest chains of a launch on small panels, and most of such a chain is
+// fetching its instructions, which no earlier wave has brought in: every phase therefore has one
+// copy of its code, for all depths, sides and closure rows.  The kernel is 14 KB (sbp42) / 17 KB (sbp63)
+// instead of 71 / 147 KB with the rows written out per side; a C95 sbp63 step went from 34 to 19 us and the
+// 16-member ensemble (C48-C192) from 342 to 239 us.
 template <int ORD, typename T, int MODE, bool OTF, bool PERSIST = false>
-__device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T> &a, int seg, EdgeSmem<ORD, T> &sm,
-                                           int nthreads) {
-    constexpr int R = Sbp<ORD>::REACH, D = Sbp<ORD>::last[0];
-    const int n = g.n, S = edge_seg_len(n, PERSIST);
+__device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T> &a, int seg, EdgeFields<ORD, T> &sm,
+                                           T *tab, int nthreads) {
+    constexpr int R = Sbp<ORD>::REACH, D = Sbp<ORD>::last[0], S = edge_seg_len(R);
+    constexpr int NE = Sbp<ORD>::NE, NW = RowWeights<ORD>::NW;
+    const int n = g.n;
     int tid = threadIdx.x;
     if constexpr (PERSIST) asm volatile("" : "+v"(tid));
-    const int nsx = edge_segs_x(n, PERSIST), nsy = edge_segs_y(n, PERSIST), per = 2 * (nsx + nsy);
+    const int nsx = edge_segs_x(n, R), nsy = edge_segs_y(n, R), per = 2 * (nsx + nsy);
     const int p = seg / per, r = seg - p * per;
     int e, si;
     if (r < 2 * nsx) { e = r / nsx; si = r - e * nsx; }
@@ -298,146 +263,184 @@ __device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T
     // cube corners of the x-edges: the neighbour across the y-edge at i = 0 / n-1
     const bool c0 = e < 2 && k0 == 0, c1 = e < 2 && k1 == n;
     const int ci = e == 0 ? 0 : n - 1;
-    const T *y = a.y;
 
-    const int k = k0 + tid;
-    const bool act = tid < k1 - k0;
+    const int lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), nwaves = nthreads / 64;
+    const int k = k0 - R + lane;
+    const bool act = k >= k0 && k < k1;
+    const int i = e < 2 ? ci : k, j = e < 2 ? k : (e == 2 ? 0 : n - 1);
+    const unsigned off = point_off(g, i, j);
+    OutPre<T> pre{};
+    T q = T(0);          // sync weight of the own point; at a corner the x-edge's, qc the y-edge's
+    T qc = T(0);
+    if (wave == 0 && act) {
+        pre = prefetch_point<T, MODE>(g, a, p, off);
+        q = e == 0 ? g.ql[k] : e == 1 ? g.qr[k] : e == 2 ? g.qb[k] : g.qt[k];
+        if (e < 2 && k == 0) qc = g.qb[i];
+        if (e < 2 && k == n - 1) qc = g.qt[i];
+    }
 
-    // ---- strips: per side S + 2R positions at depth 0, S positions at depths 1..D-1; at a
-    // corner 2R+1 positions at depth 0 and the corner position at depths 1..D-1 ----
-    const int N0 = S + 2 * R, NS = N0 + (D - 1) * S;
-    constexpr int NC = 2 * R + 1 + (D - 1);
-    const int total = 2 * NS + 2 * NC;
-    for (int c = tid; c < total; c += nthreads) {
-        EdgeDesc ei;
-        int d, kk, slot, side, idx;
-        if (c < 2 * NS) {
-            side = c / NS;
-            const int q = c - side * NS;
-            ei = side == 0 ? own : nbr;
-            slot = -1;
-            if (q < N0) { d = 0; idx = q; kk = k0 - R + q; }
-            else { d = 1 + (q - N0) / S; idx = (q - N0) % S; kk = k0 + idx; if (kk >= k1) continue; }
-        } else {
-            const int q = c - 2 * NS;
-            slot = q / NC;
-            if (!(slot == 0 ? c0 : c1)) continue;
-            const int w = q - slot * NC;
-            ei = edge_desc(g.einfo + (p * 4 + (slot == 0 ? 2 : 3)) * 8);
-            side = 0;
-            if (w < 2 * R + 1) { d = 0; idx = w; kk = ci - R + w; }
-            else { d = 1 + (w - (2 * R + 1)); idx = 0; kk = ci; }
+    // ---- inputs: line w of the list (side 0 depths 0..D-1, side 1 likewise, corner slots 0, 1) ----
+    RawPoint<T> mine{};
+    T hu = T(0), hv = T(0);
+#pragma unroll 1
+    for (int w = wave; w < 2 * D + 2; w += nwaves) {
+        const bool corner = w >= 2 * D;
+        const int side = corner ? w - 2 * D : (w >= D ? 1 : 0);   // or corner slot
+        EdgeDesc ei = side ? nbr : own;
+        int d = w - side * D, kk = k;
+        bool ok = kk >= 0 && kk < n && (d == 0 || act);
+        if (corner) {
+            if (!(side == 0 ? c0 : c1)) continue;
+            ei = edge_desc(g.einfo + (p * 4 + 2 + side) * 8);
+            d = lane <= 2 * R ? 0 : lane - 2 * R;
+            kk = lane <= 2 * R ? ci - R + lane : ci;
+            ok = kk >= 0 && kk < n && d < D;
         }
-        if (kk < 0 || kk >= n) continue;
+        if (!ok) continue;
         const int nidx = ei.tnu == 0 ? d : n - 1 - d, tidx = ei.a_base + ei.s * kk;
-        const int qi = ei.nu_x ? nidx : tidx, qj = ei.nu_x ? tidx : nidx;
-        const Derived<T> dv = derived_global<OTF>(g, y, a.hs, ei.q, qi, qj);
-        if (d == 0) {
-            T *dst = slot < 0 ? sm.e0[side][idx] : sm.c0[slot][idx];
-            dst[0] = dv.K; dst[1] = dv.Gxd; dst[2] = dv.Gyd; dst[3] = dv.Gxc; dst[4] = dv.Gyc;
-            dst[5] = metric_J<OTF>(g, ei.q, qi, qj);
+        const PanelIn<T> in = panel_in(g, a.y, a.hs, ei.q);
+        const RawPoint<T> rp = load_point<OTF>(g, in, ei.nu_x ? nidx : tidx, ei.nu_x ? tidx : nidx);
+        const Derived<T> dv = derived_of(g, rp);
+        const T nD = ei.nu_x ? dv.Gxd : dv.Gyd, nC = ei.nu_x ? dv.Gxc : dv.Gyc;
+        const T tD = ei.nu_x ? dv.Gyd : dv.Gxd, tC = ei.nu_x ? dv.Gyc : dv.Gxc;
+        if (!corner) {
+            sm.nrm[side][d][0][lane] = dv.K;
+            sm.nrm[side][d][1][lane] = nD;
+            sm.nrm[side][d][2][lane] = nC;
+            if (d == 0) {
+                sm.tan[side][0][lane] = dv.K;
+                sm.tan[side][1][lane] = tD;
+                sm.tan[side][2][lane] = tC;
+                sm.J[side][lane] = rp.J;
+            }
+            if (w == 0) {      // the first wave's first line: its lanes' output points
+                mine = rp;
+                hu = dv.hu;
+                hv = dv.hv;
+            }
         } else {
-            const bool nu_x = ei.nu_x != 0;
-            T *dst = slot < 0 ? sm.en[side][d - 1][idx] : sm.cn[slot][d - 1];
-            dst[0] = dv.K;
-            dst[1] = nu_x ? dv.Gxd : dv.Gyd;
-            dst[2] = nu_x ? dv.Gxc : dv.Gyc;
+            if (kk == ci) {
+                sm.cnrm[side][d][0] = dv.K;
+                sm.cnrm[side][d][1] = nD;
+                sm.cnrm[side][d][2] = nC;
+                if (d == 0) sm.cJ[side] = rp.J;
+            }
+            if (d == 0) {
+                sm.ctan[side][0][lane] = dv.K;
+                sm.ctan[side][1][lane] = tD;
+                sm.ctan[side][2][lane] = tC;
+            }
         }
     }
+    load_rows<ORD, T>(tab, tid, nthreads);
     __syncthreads();
-    if (!act) return;
-    int i, j;
-    if (e < 2) { i = e == 0 ? 0 : n - 1; j = k; }
-    else { i = k; j = e == 2 ? 0 : n - 1; }
-    const long long id = pidx(g, p, i, j);
-    const OutPre<T> pre = prefetch_point<T, MODE>(g, a, id);
 
-    T ro[4], rn[4];
-    neighbour_raw<ORD, T>(g, own, k, [&](int kk, int f) { return sm.e0[0][kk - (k0 - R)][f]; },
-                          [&](int d, int f3) { return sm.en[0][d - 1][k - k0][f3]; }, ro);
-    neighbour_raw<ORD, T>(g, nbr, k, [&](int kk, int f) { return sm.e0[1][kk - (k0 - R)][f]; },
-                          [&](int d, int f3) { return sm.en[1][d - 1][k - k0][f3]; }, rn);
-    T gx = ro[0], gy = ro[1], dv = ro[2], cu = ro[3];
+    // ---- raw values: wave 0 the own panel's, wave 1 the neighbour's, wave 2 lanes 0, 1 the corners' ----
+    if (wave < 2 ? act : (wave == 2 && lane < 2 && (lane == 0 ? c0 : c1))) {
+        const bool corner = wave == 2;
+        EdgeDesc ed = wave ? nbr : own;
+        int kk = k, ns = 64, ts = 64;
+        const T *nb = &sm.nrm[wave & 1][0][0][lane], *tb = &sm.tan[wave & 1][0][lane], *Jb = &sm.J[wave & 1][lane];
+        if (corner) {
+            ed = edge_desc(g.einfo + (p * 4 + 2 + lane) * 8);
+            kk = ci;
+            ns = 1;
+            ts = 2 * R + 1;
+            nb = sm.cnrm[lane][0];
+            tb = &sm.ctan[lane][0][R];
+            Jb = &sm.cJ[lane];
+        }
+        // across the edge: row 0 by depth, or the last row, whose inputs run from depth D-1 to 0
+        const bool low = ed.tnu == 0;
+        T nK, nD, nC, tK, tD, tC;
+        row_apply3<ORD, T>(tab, RowAt{0, D, low ? 0 : 2 * NE}, [&](int m, T &x, T &y, T &z) {
+            const T *q = nb + (low ? m : D - 1 - m) * 3 * ns;
+            x = q[0]; y = q[ns]; z = q[2 * ns];
+        }, nK, nD, nC);
+        // along it: index b of the panel lies s (b - a0) lanes away
+        const int a0 = ed.a_base + ed.s * kk;
+        const RowAt rt = row_at<ORD>(a0, n);
+        row_apply3<ORD, T>(tab, rt, [&](int m, T &x, T &y, T &z) {
+            const T *q = tb + ed.s * (rt.base + m - a0);
+            x = q[0]; y = q[ts]; z = q[2 * ts];
+        }, tK, tD, tC);
+        const Rcp<T> rhxs{g.hxs, g.rhxs}, rJd = rcp_of(*Jb * g.hx * g.scale);
+        // x before y in the sums: the operands commute, so the order does not matter
+        sm.raw[wave][0][lane] = (ed.nu_x ? nK : tK) / rhxs;
+        sm.raw[wave][1][lane] = (ed.nu_x ? tK : nK) / rhxs;
+        sm.raw[wave][2][lane] = (nD + tD) / rJd;
+        sm.raw[wave][3][lane] = (nC + tC) / rJd;
+    }
+    __syncthreads();
+    if (wave != 0 || !act) return;
+
+    T gx = sm.raw[0][0][lane], gy = sm.raw[0][1][lane], dv = sm.raw[0][2][lane], cu = sm.raw[0][3][lane];
     const T U = gy, V = gx;
     // the neighbour's raw values mapped to this panel's components (vector halo convention)
     T Vn, Un;
-    map_vec(nbr.code, rn[0], rn[1], Vn, Un);
-    const T Dn = rn[2], Cn = rn[3];
-    const bool corner = e < 2 && (k == 0 || k == n - 1);
-    if (corner) {
+    map_vec(nbr.code, sm.raw[1][0][lane], sm.raw[1][1][lane], Vn, Un);
+    const T Dn = sm.raw[1][2][lane], Cn = sm.raw[1][3][lane];
+    if (e < 2 && (k == 0 || k == n - 1)) {
         const int slot = k == 0 ? 0 : 1;
-        const EdgeDesc ec = edge_desc(g.einfo + (p * 4 + (slot == 0 ? 2 : 3)) * 8);
-        T rc[4];
-        neighbour_raw<ORD, T>(g, ec, ci, [&](int kk, int f) { return sm.c0[slot][kk - (ci - R)][f]; },
-                              [&](int d, int f3) { return sm.cn[slot][d - 1][f3]; }, rc);
         T Vy, Uy;
-        map_vec(ec.code, rc[0], rc[1], Vy, Uy);
-        const T qy = slot == 0 ? g.qb[i] : g.qt[i];
-        const T qx = e == 0 ? g.ql[j] : g.qr[j];
-        dv = (dv + Dn + rc[2]) / T(3);
-        cu = (cu + Cn + rc[3]) / T(3);
-        gy = (U + Un + Uy + qy * Vy) / T(3);
-        gx = (V + Vn + Vy + qx * Un) / T(3);
-    } else if (e == 0) {
-        dv = T(0.5) * (Dn + dv);
-        cu = T(0.5) * (Cn + cu);
-        gy = T(0.5) * (Un + U);
-        gx = T(0.5) * (V + Vn + g.ql[j] * Un);
-    } else if (e == 1) {
-        dv = T(0.5) * (dv + Dn);
-        cu = T(0.5) * (cu + Cn);
-        gy = T(0.5) * (U + Un);
-        gx = T(0.5) * (V + Vn + g.qr[j] * Un);
-    } else if (e == 2) {
-        dv = T(0.5) * (dv + Dn);
-        cu = T(0.5) * (cu + Cn);
-        gx = T(0.5) * (Vn + V);
-        gy = T(0.5) * (U + Un + g.qb[i] * Vn);
+        map_vec(g.einfo[(p * 4 + 2 + slot) * 8 + 5], sm.raw[2][0][slot], sm.raw[2][1][slot], Vy, Uy);
+        dv = (dv + Dn + sm.raw[2][2][slot]) / T(3);
+        cu = (cu + Cn + sm.raw[2][3][slot]) / T(3);
+        gy = (U + Un + Uy + qc * Vy) / T(3);
+        gx = (V + Vn + Vy + q * Un) / T(3);
     } else {
+        // the component along the edge is averaged, the one across it takes the weight q
         dv = T(0.5) * (dv + Dn);
         cu = T(0.5) * (cu + Cn);
-        gx = T(0.5) * (V + Vn);
-        gy = T(0.5) * (U + Un + g.qt[i] * Vn);
+        if (e < 2) {
+            gy = T(0.5) * (U + Un);
+            gx = T(0.5) * (V + Vn + q * Un);
+        } else {
+            gx = T(0.5) * (V + Vn);
+            gy = T(0.5) * (U + Un + q * Vn);
+        }
     }
-    T Jv, q11, q12, q22;
-    if constexpr (OTF) {
-        const Metric m = metric_otf(g.tanA, i, j);
-        Jv = (T)m.J; q11 = (T)m.Qi11; q12 = (T)m.Qi12; q22 = (T)m.Qi22;
-    } else {
-        const long long mid = midx(g, p, i, j);
-        Jv = g.J[mid]; q11 = g.Qi11[mid]; q12 = g.Qi12[mid]; q22 = g.Qi22[mid];
-    }
-    finish_point<T, MODE>(g, a, id, y[id], y[id + g.fs], y[id + 2 * g.fs], Jv, q11, q12, q22, gx, gy, dv, cu, pre);
+    finish_point<T, MODE>(g, a, p, off, mine.h, mine.u, mine.v, hu, hv, mine.J, gx, gy, dv, cu, pre);
 }
 
-// a tile starting at (tx0, ty0) whose derivative rows are all interior ones (NE <= i, j < n - NE)
-// and whose halo of REACH points lies inside the panel: M <= i, j < n - M with M the larger
+// a tile starting at (tx0, ty0) whose derivative rows are all interior ones (NE <= i, j < n - NE; the
+// interior row's reach is at most NE, so its halo lies inside the panel)
 template <int ORD, int TX, int TY>
 __device__ __forceinline__ bool inner_tile(int tx0, int ty0, int n) {
-    constexpr int NE = Sbp<ORD>::NE, RE = Sbp<ORD>::REACH, M = NE > RE ? NE : RE;
-    return tx0 >= M && tx0 + TX <= n - M && ty0 >= M && ty0 + TY <= n - M;
+    constexpr int NE = Sbp<ORD>::NE;
+    static_assert(tile_halo<ORD, true>() <= NE, "the halo of an inner tile lies inside the panel");
+    return tx0 >= NE && tx0 + TX <= n - NE && ty0 >= NE && ty0 + TY <= n - NE;
+}
+
+// Tile t of a cube: row strips outermost, then panels, then the columns of a strip.  An XCD's
+// contiguous range (xcd_tile) is then a band of rows of all six panels, which read the same metric
+// planes there: an eighth of them per XCD, which stays in its L2 from panel to panel.
+template <int ORD, typename T, int MODE, int TX, int TY, bool OTF, bool PERSIST>
+__device__ __forceinline__ void stage_any_tile(const DevGeo<T> &g, const StageArgs<T> &a, int t,
+                                               Smem<ORD, T, TX, TY> &sm) {
+    const int ntx = tiles_along(g.n, TX);
+    const int strip = t / (6 * ntx), rem = t - strip * 6 * ntx, p = rem / ntx;
+    const int tx0 = 1 + (rem - p * ntx) * TX, ty0 = 1 + strip * TY;
+    if (inner_tile<ORD, TX, TY>(tx0, ty0, g.n))
+        stage_tile<ORD, T, MODE, TX, TY, OTF, PERSIST, true>(g, a, p, tx0, ty0, sm.in, sm.tab);
+    else
+        stage_tile<ORD, T, MODE, TX, TY, OTF, PERSIST, false>(g, a, p, tx0, ty0, sm.t, sm.tab);
 }
 
 // edge blocks first (a multiple of 8, so that the tiles keep their XCD-contiguous mapping)
-SWM_HD constexpr int edge_blocks(int n) { return (edge_segs(n) + 7) / 8 * 8; }
+SWM_HD constexpr int edge_blocks(int n, int reach) { return (edge_segs(n, reach) + 7) / 8 * 8; }
 
 template <int ORD, typename T, int MODE, int TX, int TY, bool OTF>
 __global__ void __launch_bounds__(TX * TY) stage_kernel(DevGeo<T> g, StageArgs<T> a) {
     __shared__ Smem<ORD, T, TX, TY> sm;
-    const int ne = edge_blocks(g.n);
+    const int ne = edge_blocks(g.n, Sbp<ORD>::REACH);
     if ((int)blockIdx.x < ne) {
-        if ((int)blockIdx.x < edge_segs(g.n)) stage_edge<ORD, T, MODE, OTF>(g, a, blockIdx.x, sm.e, TX * TY);
+        if ((int)blockIdx.x < edge_segs(g.n, Sbp<ORD>::REACH))
+            stage_edge<ORD, T, MODE, OTF>(g, a, blockIdx.x, sm.e, sm.tab, TX * TY);
         return;
     }
-    const int ntx = tiles_along(g.n, TX), nty = tiles_along(g.n, TY);
-    const int tile = xcd_tile(blockIdx.x - ne, 6 * ntx * nty);
-    const int p = tile / (ntx * nty);
-    const int rem = tile - p * ntx * nty;
-    const int tx0 = 1 + (rem % ntx) * TX, ty0 = 1 + (rem / ntx) * TY;
-    if (inner_tile<ORD, TX, TY>(tx0, ty0, g.n))
-        stage_tile<ORD, T, MODE, TX, TY, OTF, false, true>(g, a, p, tx0, ty0, sm.t);
-    else
-        stage_tile<ORD, T, MODE, TX, TY, OTF>(g, a, p, tx0, ty0, sm.t);
+    const int ntiles = 6 * tiles_along(g.n, TX) * tiles_along(g.n, TY);
+    stage_any_tile<ORD, T, MODE, TX, TY, OTF, false>(g, a, xcd_tile(blockIdx.x - ne, ntiles), sm);
 }
 
 // Copy of a block-uniform struct into scalar registers (word by word through readfirstlane):
@@ -455,7 +458,7 @@ __device__ __forceinline__ S uniform_copy(const S *src) {
 }
 
 // Ensemble of cubes of different sizes in one launch: the blocks walk the concatenated task list
-// of all members (per member its 6*ntx*nty tiles (tiles_along), then its edge_segs(n, true) edge
+// of all members (per member its 6*ntx*nty tiles (tiles_along), then its edge_segs(n, REACH) edge
 // segments), XCD-contiguous; a persistent grid loops over it, a grid of one block per task runs
 // each block once.  tasks[t] = (member, task index within the
 // member): one load gives a block its member, whose geometry and stage arguments it then takes
@@ -471,19 +474,12 @@ __global__ void __launch_bounds__(TX * TY) ens_stage_kernel(const EnsMember<T> *
         const int lt = __builtin_amdgcn_readfirstlane(tk.y);
         const DevGeo<T> g = uniform_copy(&members[m].g);
         const StageArgs<T> a = uniform_copy(&members[m].a);
-        const int ntx = tiles_along(g.n, TX), nty = tiles_along(g.n, TY);
+        const int ncell = 6 * tiles_along(g.n, TX) * tiles_along(g.n, TY);
         __syncthreads();  // the previous task's LDS reads are done
-        if (lt >= 6 * ntx * nty) {
-            stage_edge<ORD, T, MODE, OTF, true>(g, a, lt - 6 * ntx * nty, sm.e, TX * TY);
-            continue;
-        }
-        const int p = lt / (ntx * nty);
-        const int rem = lt - p * ntx * nty;
-        const int tx0 = 1 + (rem % ntx) * TX, ty0 = 1 + (rem / ntx) * TY;
-        if (inner_tile<ORD, TX, TY>(tx0, ty0, g.n))
-            stage_tile<ORD, T, MODE, TX, TY, OTF, true, true>(g, a, p, tx0, ty0, sm.t);
+        if (lt >= ncell)
+            stage_edge<ORD, T, MODE, OTF, true>(g, a, lt - ncell, sm.e, sm.tab, TX * TY);
         else
-            stage_tile<ORD, T, MODE, TX, TY, OTF, true>(g, a, p, tx0, ty0, sm.t);
+            stage_any_tile<ORD, T, MODE, TX, TY, OTF, true>(g, a, lt, sm);
     }
 }
 
@@ -494,7 +490,7 @@ namespace swm {
 template <int ORD, typename T, int TX, int TY, bool OTF>
 hipError_t launch_one(int mode, const DevGeo<T> &g, const StageArgs<T> &a, hipStream_t s) {
     const int ntx = tiles_along(g.n, TX), nty = tiles_along(g.n, TY);
-    const dim3 grid(edge_blocks(g.n) + 6 * ntx * nty), block(TX * TY);
+    const dim3 grid(edge_blocks(g.n, Sbp<ORD>::REACH) + 6 * ntx * nty), block(TX * TY);
     switch (mode) {
     case MODE_RHS: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_RHS, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_STAGE1: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_STAGE1, TX, TY, OTF>), grid, block, 0, s, g, a); break;
