@@ -15,18 +15,15 @@ struct swm_cctx {
     double scale = 1, omega = 1, grav = 1, hx = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
-    double *geo = nullptr;  // one panel plane each of Jo, Jx, Jy, Jq, Qi12o, Qi11x, Qi22y, then fo (6 panels)
+    double *geo = nullptr;  // one panel plane each of Jo, Jx, Jy, Jq, Qi12o, Qi11x, Qi22y, Jo Qi12o, then fo (6 panels)
     double *hs = nullptr;
     // cube-edge neighbour lists (swmc::CGeo): vsrc, fsrc, osrc, qnb; signs vsg, fsg
     long long *lists = nullptr;
     signed char *signs = nullptr;
     long long *vsrc = nullptr, *fsrc = nullptr, *osrc = nullptr, *qnb = nullptr;
     signed char *vsg = nullptr, *fsg = nullptr;
-    // groups of the q-point edge sync (k_qsync_edges)
-    long long *qpairs = nullptr, *qcorners = nullptr;
-    int nqpairs = 0, nqcorners = 0;
-    // work fields: G (pair), KEu, KEv, KE, W, cup, cvp, RK tendencies k0..k2, stage inputs yA, yB,
-    // A, B (J Qi12-weighted components at o points), fu, fv (the synced curl at x and y points)
+    // work fields: the fluxes G (pair), the potential KE, the raw curl W, the RK accumulator and the stage
+    // inputs yA, yB (a state each)
     double *work = nullptr;
     // diagnostics: quadrature weights A_centers (1..N) and A_interfaces (1..N+1) per index, block
     // partial sums (10 per block) and the 6 results

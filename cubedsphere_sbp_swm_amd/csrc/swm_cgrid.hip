@@ -15,13 +15,17 @@
 //     sbp_operator_mod.f90:344-413),
 //   - the O-point halo of the kinetic-energy potential (gradient, grad_c_sbp42_mod.f90:53-139),
 //   - the corner sync of the curl (halo_Ah_scalar_sync_mod.f90:52-93),
-// the first three read on the fly through precomputed neighbour lists by the threads on the panel
-// edges, the sync one small launch over the shared points.  One RHS is eight launches of memory-bound stencil sweeps with one thread per output point (16 x 16
-// thread blocks, coalesced along i); the RK4 stage updates are applied by the kernels that produce
-// the tendencies.  Intermediate values at another point type (the J Qi12-weighted components at o
-// points, the curl at x and y points) are stored once and read by the next kernel: recomputing
-// them inside the consumer (4-6 nested stencil rows per output) measured slower than the extra
-// field traffic.  The RK4 step is captured into a HIP graph.
+// all read on the fly through precomputed neighbour lists by the tiles on the panel edges.
+//
+// One RHS is two launches over tiles of TX x TY cells.  k_flux forms the fluxes J hu, J hv, the
+// kinetic-energy potential and the raw curl of a tile from the state, k_tend the synced curl, the
+// Coriolis terms, the divergence, the gradient, the tendencies and the RK4 stage update from those.
+// Every intermediate at another point type (the J Qi12-weighted components and the potential's halves
+// in k_flux; the curl at x and y points and the Coriolis terms at o points in k_tend) lives in LDS on
+// the tile and the halo that the next stencil reads; only the four fields that need the neighbour
+// panels' values go through memory between the two.  Eight launches with the intermediates in
+// memory move 140 field passes per step more and leave each launch near its latency floor.  The RK4
+// step is captured into a HIP graph.
 //
 // Every expression keeps the reference's operation order with no fused multiply-adds
 // (-ffp-contract=off), so results match an FP64 CPU evaluation of the same algorithm bit for bit.
@@ -36,7 +40,7 @@
 
 namespace swmc {
 
-constexpr int BX = 16, BY = 16;
+constexpr int BX = 16, BY = 16;   // blocks of the diagnostics
 
 // ---- staggered SBP42 operators, sbp_operators_collection_mod.f90:110-191 ----
 // W42 interpolation interfaces -> centres, optimised weights (W42_staggered_i2c_opt1)
@@ -130,6 +134,114 @@ __device__ __forceinline__ double sop(int i, int nsrc, const double *__restrict_
     return sopf<O>(i, nsrc, [&](int k) { return f0[(long long)k * s]; });
 }
 
+// ---- the same rows from tables ----
+// Classes 0 .. NE-1 the left closure rows, NE the interior row, NE+1 .. 2 NE the right closure rows, NW
+// weights each; a tile that holds closure rows reads them from LDS, one code path for all its points.
+template <class O>
+struct Rows {
+    static constexpr int NW = O::NW, NC = 2 * O::NE + 1, SIZE = NC * NW;
+    static constexpr void fill(double *w) {
+        for (int c = 0; c < SIZE; ++c) w[c] = 0.0;
+        for (int r = 0; r < O::NE; ++r)
+            for (int m = 0; m < O::last[r]; ++m) {
+                w[r * NW + m] = O::Ql[r][m];
+                w[(2 * O::NE - r) * NW + m] = O::SIGN * O::Ql[r][O::last[r] - 1 - m];
+            }
+        for (int m = 0; m < 4; ++m) w[O::NE * NW + m] = O::Qin[m];
+    }
+    static constexpr unsigned packed_last() {
+        unsigned v = 0;
+        for (int r = 0; r < O::NE; ++r) v |= (unsigned)O::last[r] << (4 * r);
+        return v;
+    }
+    static constexpr int min_last() {
+        int m = 4;
+        for (int r = 0; r < O::NE; ++r) m = O::last[r] < m ? O::last[r] : m;
+        return m;
+    }
+    static constexpr int MINLAST = min_last();
+};
+// the tables of the four operators one after the other
+constexpr int ROW_I2C = 0, ROW_C2I = ROW_I2C + Rows<W42i2c>::SIZE, ROW_DC2I = ROW_C2I + Rows<W42c2i>::SIZE,
+              ROW_DI2C = ROW_DC2I + Rows<D42c2i>::SIZE, ROW_SIZE = ROW_DI2C + Rows<D42i2c>::SIZE;
+template <class O> constexpr int row_start();
+template <> constexpr int row_start<W42i2c>() { return ROW_I2C; }
+template <> constexpr int row_start<W42c2i>() { return ROW_C2I; }
+template <> constexpr int row_start<D42c2i>() { return ROW_DC2I; }
+template <> constexpr int row_start<D42i2c>() { return ROW_DI2C; }
+struct RowTab {
+    double w[ROW_SIZE];
+    constexpr RowTab() : w() {
+        Rows<W42i2c>::fill(w + ROW_I2C);
+        Rows<W42c2i>::fill(w + ROW_C2I);
+        Rows<D42c2i>::fill(w + ROW_DC2I);
+        Rows<D42i2c>::fill(w + ROW_DI2C);
+    }
+};
+__device__ const RowTab row_tab = RowTab();
+
+// output row i (1-based) of operator O on a line of nsrc inputs f(k): the interior row with constant
+// weights (INNER at compile time, or `inner` for a tile whose rows along this line all are), or any row
+// from the table
+template <class O, bool INNER, class F>
+__device__ __forceinline__ double trow(const double *tab, bool inner, int i, int nsrc, const F &f) {
+    if (INNER || inner) {
+        const int b = i + O::INSHIFT;
+        double r = O::Qin[0] * f(b);
+        r = r + O::Qin[1] * f(b + 1);
+        r = r + O::Qin[2] * f(b + 2);
+        return r + O::Qin[3] * f(b + 3);
+    } else {
+        constexpr unsigned LASTS = Rows<O>::packed_last();
+        const int ntarg = nsrc + O::DNX;
+        int b = i + O::INSHIFT, cnt = 4, cls = O::NE;
+        if (i <= O::NE) {
+            b = 1;
+            cnt = (int)((LASTS >> (4 * (i - 1))) & 15u);
+            cls = i - 1;
+        } else if (i > ntarg - O::NE) {
+            cnt = (int)((LASTS >> (4 * (ntarg - i))) & 15u);
+            b = nsrc + 1 - cnt;
+            cls = 2 * O::NE - (ntarg - i);
+        }
+        const double *w = tab + row_start<O>() + cls * O::NW;
+        // all inputs are read at once (the last one again beyond the row's end) and the sum stops at cnt: a
+        // branch per input would wait for LDS input by input
+        double x[O::NW];
+#pragma unroll
+        for (int m = 0; m < O::NW; ++m) x[m] = f(b + (m < Rows<O>::MINLAST ? m : min(m, cnt - 1)));
+        double r = w[0] * x[0];
+#pragma unroll
+        for (int m = 1; m < O::NW; ++m) {
+            const double z = r + w[m] * x[m];
+            r = m < Rows<O>::MINLAST || m < cnt ? z : r;
+        }
+        return r;
+    }
+}
+
+// range lo .. hi of points along a line, and the inputs that the rows of a range read (closure rows:
+// at most 6 (i2c) / 5 (c2i) points from the end)
+struct Rng {
+    int lo, hi;
+};
+template <class O>
+__device__ __forceinline__ Rng rng_in(const Rng &r, int nsrc) {
+    if (r.lo > r.hi) return {1 << 30, -(1 << 30)};
+    const int ntarg = nsrc + O::DNX;
+    int lo = r.lo + O::INSHIFT, hi = r.hi + O::INSHIFT + 3;
+    if (r.lo <= O::NE) {
+        lo = 1;
+        hi = max(hi, O::NW);
+    }
+    if (r.hi > ntarg - O::NE) {
+        hi = nsrc;
+        lo = min(lo, nsrc + 1 - O::NW);
+    }
+    return {max(lo, 1), min(hi, nsrc)};
+}
+__device__ __forceinline__ Rng hull(const Rng &a, const Rng &b) { return {min(a.lo, b.lo), max(a.hi, b.hi)}; }
+
 // metric terms J, Qi at the four point types depend on (alpha, beta) only: one panel plane each,
 // read for every panel at the point's offset within its panel (mid); f differs per panel.
 // Cube-edge neighbour lists (offsets in the stored layout, signs +-1), indexed by panel p, edge
@@ -141,7 +253,7 @@ __device__ __forceinline__ double sop(int i, int nsrc, const double *__restrict_
 //   osrc      O points, [((p*4+e)*3 + d-1)*N + k-1]
 //   qnb       q points on an edge: the neighbour's copy, [(p*4+e)*(N+1) + k-1]
 struct CGeo {
-    const double *Jo, *Jx, *Jy, *Jq, *Qi12o, *Qi11x, *Qi22y, *fo;
+    const double *Jo, *Jx, *Jy, *Jq, *Qi12o, *Qi11x, *Qi22y, *JQo, *fo;  // JQo = Jo Qi12o
     const double *hs;  // orography at o points, or NULL
     const long long *vsrc, *fsrc, *osrc, *qnb;
     const signed char *vsg, *fsg;
@@ -171,32 +283,35 @@ __device__ __forceinline__ double ohalo(const CGeo &g, const double *f, int p, i
     return f[g.osrc[(((long long)p * 4 + e) * 3 + (d - 1)) * g.N + (k - 1)]];
 }
 
-// RK4 stage handling of the kernels that produce the tendencies (rk4_mod.f90:20-42):
-// RK_RHS writes the tendency k; RK_STAGE writes k and the next stage input 1.0*v0 + b*k
-// (stvec_swm_t%assign); RK_FINAL writes v0 = (v0 + c2 k0 + c3 k1) + c3 k2 + c2 k (k = the last
-// stage's tendency, not stored)
-enum { RK_RHS = 0, RK_STAGE = 1, RK_FINAL = 2 };
+// RK4 stage handling of the tendencies k (rk4_mod.f90:20-42; stage inputs as stvec_swm_t%assign forms
+// them): RK_RHS writes k; RK_S1 the next stage input 1.0*v0 + b*k and acc = v0 + c*k; RK_S23 the next
+// stage input and acc = acc + c*k; RK_S4 the new state acc + c*k (the reference's sum
+// v0 + c2 k0 + c3 k1 + c3 k2 + c2 k3 added up from the left as the stages produce its terms).
+enum { RK_RHS = 0, RK_S1 = 1, RK_S23 = 2, RK_S4 = 3 };
 struct RkArgs {
-    double *k;          // tendency out (RK_RHS, RK_STAGE)
-    const double *v0;   // stage-1 state (RK_STAGE, RK_FINAL)
-    double *yn;         // next stage input (RK_STAGE)
-    double *v0w;        // state written (RK_FINAL; the same buffer as v0)
-    const double *k0, *k1, *k2;
-    double b, c2, c3;
+    double *out;        // k (RK_RHS), the next stage input, or the new state (RK_S4)
+    const double *v0;   // stage-1 state (RK_S1, RK_S23)
+    double *acc;
+    double b, c;
 };
-
+struct RkPre {
+    double v0, acc;
+};
 template <int RKM>
-__device__ __forceinline__ void rk_out(const RkArgs &r, long long off, double k) {
-    if (RKM == RK_RHS) {
-        r.k[off] = k;
-    } else if (RKM == RK_STAGE) {
-        r.k[off] = k;
-        r.yn[off] = 1.0 * r.v0[off] + r.b * k;
-    } else {
-        double v = r.v0[off] + r.c2 * r.k0[off] + r.c3 * r.k1[off];
-        v = v + r.c3 * r.k2[off] + r.c2 * k;
-        r.v0w[off] = v;
+__device__ __forceinline__ RkPre rk_pre(const RkArgs &r, long long base, unsigned off) {
+    RkPre q{0.0, 0.0};
+    if (RKM == RK_S1 || RKM == RK_S23) q.v0 = swm::at_byte(r.v0 + base, off);
+    if (RKM == RK_S23 || RKM == RK_S4) q.acc = swm::at_byte((const double *)r.acc + base, off);
+    return q;
+}
+template <int RKM>
+__device__ __forceinline__ void rk_out(const RkArgs &r, long long base, unsigned off, const RkPre &q, double k) {
+    if (RKM == RK_RHS) swm::at_byte(r.out + base, off) = k;
+    if (RKM == RK_S1 || RKM == RK_S23) {
+        swm::at_byte(r.out + base, off) = 1.0 * q.v0 + r.b * k;
+        swm::at_byte(r.acc + base, off) = (RKM == RK_S1 ? q.v0 : q.acc) + r.c * k;
     }
+    if (RKM == RK_S4) swm::at_byte(r.out + base, off) = q.acc + r.c * k;
 }
 
 // Block -> tile mapping: tiles of BX x BY points in the order (column strip fastest, row strip,
@@ -211,248 +326,501 @@ __device__ __forceinline__ void rk_out(const RkArgs &r, long long off, double k)
     const int j = ty_ * BY + threadIdx.y + 1;                          \
     const int p = tile_ / (g.nbx * g.nby);
 
-// co2contra_c_sbp42 first half (co2contra_Cgrid_mod.f90:361-378): at o points
-// a = J Qi12 * (v interpolated along y), b = J Qi12 * (u interpolated along x)
-__global__ void __launch_bounds__(256) k_contra_o(CGeo g, const double *__restrict__ u, const double *__restrict__ v,
-                                                  double *__restrict__ A, double *__restrict__ B) {
-    C_POINT
-    if (i > g.N || j > g.N) return;
-    const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
-    const double dy = sop<W42i2c>(j, g.N + 1, v + cid(g, p, i, 0), g.pitch);
-    const double dx = sop<W42i2c>(i, g.N + 1, u + cid(g, p, 0, j), 1);
-    A[id] = g.Jo[mid] * g.Qi12o[mid] * dy;
-    B[id] = g.Jo[mid] * g.Qi12o[mid] * dx;
-}
+// ---- tiles ----
+// extents of a tile's LDS boxes beyond its TX (TY) cells: faces that the cells' interpolations read (F),
+// o points that those faces read (O), o points that the own faces read (C), faces that the C points
+// read (Q).  Tiles with closure rows need a little more than tiles of interior rows; the widest over
+// every N and tile position (closure rows of the last points reach back over a narrow last tile).
+template <bool INNER> constexpr int EXT_F = INNER ? 3 : 5;
+template <bool INNER> constexpr int EXT_O = INNER ? 6 : 7;
+template <bool INNER> constexpr int EXT_C = INNER ? 3 : 4;
+template <bool INNER> constexpr int EXT_Q = INNER ? 6 : 8;
 
-// at x and y points: second half of co2contra (:370-398), massflux_c_sbp42
-// (massflux_Cgrid_mod.f90:330-355), the J-weighted fluxes of the divergence and Coriolis terms
-// (div_c_sbp42_mod.f90:101-130, coriolis_Cgrid_mod.f90:69-84) and the halves of KE_Cgrid
-// (KE_Cgrid_mod.f90:41-57): G = (J hu, J hv), KEu = J u ut / 2, KEv = J v vt / 2
-__global__ void __launch_bounds__(256) k_flux(CGeo g, const double *__restrict__ h, const double *__restrict__ u,
-                                              const double *__restrict__ v, const double *__restrict__ A,
-                                              const double *__restrict__ B, double *__restrict__ G,
-                                              double *__restrict__ KEu, double *__restrict__ KEv) {
-    C_POINT
-    const int N = g.N;
-    if (i <= N + 1 && j <= N) {
-        const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
-        const double t = sop<W42c2i>(i, N, A + cid(g, p, 0, j), 1);
-        const double ut = g.Qi11x[mid] * u[id] + t / g.Jx[mid];
-        const double hh = sop<W42c2i>(i, N, h + cid(g, p, 0, j), 1);
-        const double hu = ut * hh;
-        G[id] = g.Jx[mid] * hu;
-        KEu[id] = g.Jx[mid] * (u[id] * ut) / 2.0;
-    }
-    if (i <= N && j <= N + 1) {
-        const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
-        const double t = sop<W42c2i>(j, N, B + cid(g, p, i, 0), g.pitch);
-        const double vt = g.Qi22y[mid] * v[id] + t / g.Jy[mid];
-        const double hh = sop<W42c2i>(j, N, h + cid(g, p, i, 0), g.pitch);
-        const double hv = vt * hh;
-        G[g.fs + id] = g.Jy[mid] * hv;
-        KEv[id] = g.Jy[mid] * (v[id] * vt) / 2.0;
-    }
-}
-
-// at o points: KE = (I_x KEu + I_y KEv)/J + g h + g hs (KE_Cgrid_mod.f90:59-75 and the update of
-// operator_swm_mod.f90:85), and dh = -div(J hu, J hv) with the centre penalties
-// (div_c_sbp42_mod.f90:70-99, sbp_operator_mod.f90:344-413), the neighbour's copies of the shared
-// faces read through fsrc
-template <int RKM>
-__global__ void __launch_bounds__(256) k_ke_div(CGeo g, const double *__restrict__ h, const double *__restrict__ KEu,
-                                                const double *__restrict__ KEv, const double *__restrict__ G,
-                                                double *__restrict__ KE, RkArgs r) {
-    C_POINT
-    const int N = g.N;
-    if (i > N || j > N) return;
-    const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
-    const double kuh = sop<W42i2c>(i, N + 1, KEu + cid(g, p, 0, j), 1);
-    const double kvh = sop<W42i2c>(j, N + 1, KEv + cid(g, p, i, 0), g.pitch);
-    double ke = (kuh + kvh) / g.Jo[mid];
-    ke = ke + g.grav * h[id] + g.grav * (g.hs ? g.hs[id] : 0.0);
-    KE[id] = ke;
-    const double *Gu = G, *Gv = G + g.fs;
-    double dx = sop<D42i2c>(i, N + 1, Gu + cid(g, p, 0, j), 1);
-    if (i <= 3) {
-        const double df = Gu[cid(g, p, 1, j)] - fhalo(g, G, p, 0, j);
-        dx = dx + 0.5 * PEN_L[i - 1] * df;
-    }
-    if (i >= N - 2) {
-        const double df = fhalo(g, G, p, 1, j) - Gu[cid(g, p, N + 1, j)];
-        dx = dx + 0.5 * PEN_R[i - N + 2] * df;
-    }
-    double dy = sop<D42i2c>(j, N + 1, Gv + cid(g, p, i, 0), g.pitch);
-    if (j <= 3) {
-        const double df = Gv[cid(g, p, i, 1)] - fhalo(g, G, p, 2, i);
-        dy = dy + 0.5 * PEN_L[j - 1] * df;
-    }
-    if (j >= N - 2) {
-        const double df = fhalo(g, G, p, 3, i) - Gv[cid(g, p, i, N + 1)];
-        dy = dy + 0.5 * PEN_R[j - N + 2] * df;
-    }
-    const double div = (dx + dy) / (g.Jo[mid] * g.hx * g.scale);
-    rk_out<RKM>(r, id, -1.0 * div);
-}
-
-// curl_c_sbp42 at q points before the corner sync (curl_c_sbp_mod.f90:73-118): staggered
-// differences of v along x and u along y with the interface penalties, the neighbour's
-// tangential components read through vsrc
-__global__ void __launch_bounds__(256) k_curl(CGeo g, const double *__restrict__ u, double *__restrict__ W) {
-    C_POINT
-    const int N = g.N, n = N + 1;
-    if (i > n || j > n) return;
-    const double *v = u + g.fs;
-    const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
-    double dvx = sop<D42c2i>(i, N, v + cid(g, p, 0, j), 1);
-    if (i == 1) {
-        double dv = 0.0;
-        for (int k = 1; k <= 3; ++k) dv = dv + PROJ[k - 1] * (v[cid(g, p, k, j)] - vhalo(g, u, p, 0, k, j));
-        dvx = dvx + 0.5 * dv / A_IF1;
-    }
-    if (i == n) {
-        double dv = 0.0;
-        for (int t = 0; t <= 2; ++t) dv = dv + PROJ[t] * (vhalo(g, u, p, 1, t + 1, j) - v[cid(g, p, n - t - 1, j)]);
-        dvx = dvx + 0.5 * dv / A_IF1;
-    }
-    double duy = sop<D42c2i>(j, N, u + cid(g, p, i, 0), g.pitch);
-    if (j == 1) {
-        double du = 0.0;
-        for (int k = 1; k <= 3; ++k) du = du + PROJ[k - 1] * (u[cid(g, p, i, k)] - vhalo(g, u, p, 2, k, i));
-        duy = duy + 0.5 * du / A_IF1;
-    }
-    if (j == n) {
-        double du = 0.0;
-        for (int t = 0; t <= 2; ++t) du = du + PROJ[t] * (vhalo(g, u, p, 3, t + 1, i) - u[cid(g, p, i, n - t - 1)]);
-        duy = duy + 0.5 * du / A_IF1;
-    }
-    W[id] = (dvx - duy) / (g.Jq[mid] * g.hx * g.scale);
-}
-
-// halo_Ah_scalar_sync of the curl at q points (halo_Ah_scalar_sync_mod.f90:52-93), in place on
-// the panel-edge points only.  Every shared point is one group handled by one thread: a point on
-// a cube edge has two copies whose mean 0.5 (a + b) is the same value on both panels; a cube
-// corner has three copies, copy c = (own + first neighbour + second neighbour) / 3 in the
-// order of its own panel's formula.  pairs[2k], pairs[2k+1]: offsets of the two copies;
-// corners[6g..6g+2]: offsets of the three copies, corners[6g+3+c]: the neighbour order of copy
-// c packed as 3 * first + second.
-__global__ void __launch_bounds__(256) k_qsync_edges(int npairs, int ncorners, const long long *__restrict__ pairs,
-                                                     const long long *__restrict__ corners, double *W) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < npairs) {
-        const long long a = pairs[2 * k], b = pairs[2 * k + 1];
-        const double v = 0.5 * (W[a] + W[b]);
-        W[a] = v;
-        W[b] = v;
-    } else if (k < npairs + ncorners) {
-        const long long *cg = corners + 6 * (k - npairs);
-        const double r[3] = {W[cg[0]], W[cg[1]], W[cg[2]]};
-        double v[3];
-        for (int c = 0; c < 3; ++c) {
-            const int ord = (int)cg[3 + c];
-            v[c] = (r[c] + r[ord / 3] + r[ord % 3]) / 3.0;
-        }
-        for (int c = 0; c < 3; ++c) W[cg[c]] = v[c];
-    }
-}
-
-// interpolator_w2h first half (interpolator_w2h_mod.f90:50-68): the synced curl at x points
-// (interpolated along y) and at y points (along x)
-__global__ void __launch_bounds__(256) k_w2uv(CGeo g, const double *__restrict__ W, double *__restrict__ fu,
-                                              double *__restrict__ fv) {
-    C_POINT
-    const int N = g.N;
-    if (i <= N + 1 && j <= N) fu[cid(g, p, i, j)] = sop<W42i2c>(j, N + 1, W + cid(g, p, i, 0), g.pitch);
-    if (i <= N && j <= N + 1) fv[cid(g, p, i, j)] = sop<W42i2c>(i, N + 1, W + cid(g, p, 0, j), 1);
-}
-
-// at o points: curl_p = (I_x fu + I_y fv)/2 (interpolator_w2h_mod.f90:40-46), the fluxes J hu, J hv
-// interpolated to o points, and the vector-invariant Coriolis terms (coriolis_Cgrid_mod.f90:86-103)
-__global__ void __launch_bounds__(256) k_cor_o(CGeo g, const double *__restrict__ h, const double *__restrict__ fu,
-                                               const double *__restrict__ fv, const double *__restrict__ G,
-                                               double *__restrict__ cup, double *__restrict__ cvp) {
-    C_POINT
-    const int N = g.N;
-    if (i > N || j > N) return;
-    const long long id = cid(g, p, i, j);
-    const double fuh = sop<W42i2c>(i, N + 1, fu + cid(g, p, 0, j), 1);
-    const double fvh = sop<W42i2c>(j, N + 1, fv + cid(g, p, i, 0), g.pitch);
-    const double ghup = sop<W42i2c>(i, N + 1, G + cid(g, p, 0, j), 1);
-    const double ghvp = sop<W42i2c>(j, N + 1, G + g.fs + cid(g, p, i, 0), g.pitch);
-    const double cp = 0.5 * fuh + 0.5 * fvh;
-    cup[id] = (g.fo[id] + cp) * ghvp / h[id];
-    cvp[id] = -(g.fo[id] + cp) * ghup / h[id];
-}
-
-// gradient_c_sbp42 along one line (grad_c_sbp42_mod.f90:61-139), F(k) for k = -2..N+3
-template <class F>
-__device__ __forceinline__ double grad_line(int i, int N, F &&Fv, double dx1) {
-    constexpr double dedge[4][5] = {{-2.0, 3.0, -1.0, 0.0, 0.0},
-                                    {-1.0, 1.0, 0.0, 0.0, 0.0},
-                                    {1.0 / 24.0, -9.0 / 8.0, 9.0 / 8.0, -1.0 / 24.0, 0.0},
-                                    {-1.0 / 71.0, 6.0 / 71.0, -83.0 / 71.0, 81.0 / 71.0, -3.0 / 71.0}};
-    constexpr int dlast[4] = {3, 2, 4, 5};
+// a tile of panel p: cells x0..x1 x y0..y1, own faces (and q points) up to fx1, fy1: the last tile of a
+// line holds the face N+1 too
+struct CTile {
+    int p, x0, y0, x1, y1, fx1, fy1;
+};
+// gradient_c_sbp42 along one line at face i (grad_c_sbp42_mod.f90:61-139) of the values F(k): the rows of
+// D42c2i, the right closure rows summed from the edge inwards, and on the panel edges the interface
+// penalty with the neighbour's values nb[depth]
+template <bool INNER, class F>
+__device__ __forceinline__ double grad_row(const double *tab, bool inner, int i, int N, double dx1, const F &Fv,
+                                           const double (&nb)[3]) {
     constexpr double din[4] = {1.0 / 24.0, -9.0 / 8.0, 9.0 / 8.0, -1.0 / 24.0};
-    const int n = N + 1;
-    double r;
-    if (i <= 4) {
-        r = dedge[i - 1][0] * Fv(1);
-#pragma unroll
-        for (int m = 2; m <= 5; ++m)
-            if (m <= dlast[i - 1]) r = r + dedge[i - 1][m - 1] * Fv(m);
-        r = r * dx1;
-        if (i == 1) {
-            const double dh = (PROJ[0] * (Fv(1) - Fv(0)) + PROJ[1] * (Fv(2) - Fv(-1)) + PROJ[2] * (Fv(3) - Fv(-2))) * dx1;
-            r = r + 0.5 * dh / A_IF1;
-        }
-    } else if (i <= N + 1 - 4) {
-        r = Fv(i - 2) * din[0];
+    if (INNER || inner) {
+        double r = Fv(i - 2) * din[0];
         r = r + Fv(i - 1) * din[1];
         r = r + Fv(i) * din[2];
         r = r + Fv(i + 1) * din[3];
-        r = r * dx1;
+        return r * dx1;
     } else {
-        const int i2 = n - i + 1, i1 = dlast[i2 - 1];
-        double t = dedge[i2 - 1][0] * Fv(n - 1);
+        constexpr unsigned LASTS = Rows<D42c2i>::packed_last();
+        const int n = N + 1;
+        const bool right = i > n - 4;
+        int b = i - 2, s = 1, cnt = 4, cls = 4;
+        if (i <= 4) { b = 1; cls = i - 1; }
+        else if (right) { b = n - 1; s = -1; cls = n - i; }
+        if (cls < 4) cnt = (int)((LASTS >> (4 * cls)) & 15u);
+        const double *w = tab + ROW_DC2I + cls * D42c2i::NW;
+        double x[D42c2i::NW];
 #pragma unroll
-        for (int m = 2; m <= 5; ++m)
-            if (m <= i1) t = t + dedge[i2 - 1][m - 1] * Fv(n - m);
-        r = -t * dx1;
-        if (i == n) {
-            const double dh =
-                (PROJ[0] * (Fv(n) - Fv(n - 1)) + PROJ[1] * (Fv(n + 1) - Fv(n - 2)) + PROJ[2] * (Fv(n + 2) - Fv(n - 3))) * dx1;
-            r = r + 0.5 * dh / A_IF1;
+        for (int m = 0; m < D42c2i::NW; ++m) x[m] = Fv(b + s * (m < 2 ? m : min(m, cnt - 1)));
+        double r = w[0] * x[0];
+#pragma unroll
+        for (int m = 1; m < D42c2i::NW; ++m) {
+            const double z = r + w[m] * x[m];
+            r = m < 2 || m < cnt ? z : r;
         }
+        r = (s < 0 ? -r : r) * dx1;
+        if (i == 1 || i == n) {
+            double dh = 0.0;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                const double own = Fv(i == 1 ? 1 + m : N - m);
+                const double x = PROJ[m] * (i == 1 ? own - nb[m] : nb[m] - own);
+                dh = m ? dh + x : x;
+            }
+            r = r + 0.5 * (dh * dx1) / A_IF1;
+        }
+        return r;
     }
-    return r;
 }
 
-// momentum tendencies at x and y points: du = -grad_x(KE) + cor_u, dv = -grad_y(KE) + cor_v with
-// cor interpolated from o points (interp2d_pvec2uv_C_sbp42, interpolator_p2uv_mod.f90:90-113;
-// operator_swm_mod.f90:94-95); KE beyond the panel edges read through osrc
+// the synced curl (halo_Ah_scalar_sync_mod.f90:52-93) of the q point (i, j): on a cube edge the mean of
+// the two panels' raw values, at a cube corner of the three
+__device__ __forceinline__ double curl_at(const CGeo &g, const double *__restrict__ W, int p, int i, int j) {
+    const int n = g.N + 1;
+    const double w = W[cid(g, p, i, j)];
+    const bool ex = i == 1 || i == n, ey = j == 1 || j == n;
+    if (!ex && !ey) return w;
+    const double a = ex ? W[g.qnb[((long long)p * 4 + (i == 1 ? 0 : 1)) * n + j - 1]] : 0.0;
+    const double b = ey ? W[g.qnb[((long long)p * 4 + (j == 1 ? 2 : 3)) * n + i - 1]] : 0.0;
+    if (ex && ey) return (w + a + b) / 3.0;
+    return 0.5 * (w + (ex ? a : b));
+}
+
+// One tile configuration: TX x TY cells, NT threads
+template <int TX, int TY, int NT>
+struct CTiles {
+static constexpr int X = TX, Y = TY, THREADS = NT;
+
+// every point (column c, row r, pass k) of a W x R box dealt to the NT threads, the first to thread FROM
+template <int W, int R, int FROM = 0, class F>
+static __device__ __forceinline__ void each(int tid, const F &f) {
+    static_assert((NT & (NT - 1)) == 0, "power of two");
+#pragma unroll
+    for (int k = 0; k < (W * R + NT - 1) / NT; ++k) {
+        const int q = ((tid + NT - FROM) & (NT - 1)) + k * NT;
+        if ((k + 1) * NT <= W * R || q < W * R) f(k, q % W, q / W);
+    }
+}
+template <int W, int R> static constexpr int passes() { return (W * R + NT - 1) / NT; }
+
+static __device__ __forceinline__ CTile c_tile(const CGeo &g, int t) {
+    const int ntx = (g.N + TX - 1) / TX, strip = t / (6 * ntx), rem = t - strip * 6 * ntx;
+    CTile c;
+    c.p = rem / ntx;
+    c.x0 = (rem - c.p * ntx) * TX + 1;
+    c.y0 = strip * TY + 1;
+    c.x1 = min(c.x0 + TX - 1, g.N);
+    c.y1 = min(c.y0 + TY - 1, g.N);
+    c.fx1 = c.x1 + (c.x1 == g.N);
+    c.fy1 = c.y1 + (c.y1 == g.N);
+    return c;
+}
+// full tiles all of whose rows are interior ones
+static __device__ __forceinline__ bool c_inner(const CGeo &g, const CTile &c) {
+    return c.x0 >= 7 && c.y0 >= 7 && c.x1 <= g.N - 5 && c.y1 <= g.N - 5 && c.x1 - c.x0 == TX - 1 && c.y1 - c.y0 == TY - 1;
+}
+static __device__ __forceinline__ unsigned c_off(const CGeo &g, int i, int j) {
+    return (__umul24((unsigned)(j - 1 + H), (unsigned)g.pitch) + (unsigned)(i - 1 + H)) * 8u;
+}
+static __device__ __forceinline__ void load_row_tab(double *tab, int tid) {
+    for (int c = tid; c < ROW_SIZE; c += NT) tab[c] = row_tab.w[c];
+}
+
+template <bool INNER>
+struct FluxSmem {
+    static constexpr int F = EXT_F<INNER>, O = EXT_O<INNER>, C = EXT_C<INNER>;
+    double u[TY + O][TX + F], v[TY + F][TX + O], h[TY + C][TX + C];
+    double A[TY][TX + O], B[TY + O][TX];         // J Qi12-weighted components at o points
+    double ku[TY][TX + F], kv[TY + F][TX];       // halves of the potential at x and y points
+};
+
+// co2contra_c_sbp42 (co2contra_Cgrid_mod.f90:361-398), massflux_c_sbp42 (massflux_Cgrid_mod.f90:330-355),
+// the J-weighted fluxes G = (J hu, J hv) of the divergence and Coriolis terms (div_c_sbp42_mod.f90:
+// 101-130, coriolis_Cgrid_mod.f90:69-84), KE_Cgrid (KE_Cgrid_mod.f90:41-75) with the update of
+// operator_swm_mod.f90:85, and curl_c_sbp42 before the corner sync (curl_c_sbp_mod.f90:73-118)
+template <bool INNER>
+static __device__ __forceinline__ void flux_tile(const CGeo &g, const double *__restrict__ y, double *__restrict__ G,
+                                          double *__restrict__ KE, double *__restrict__ W, const CTile &t,
+                                          FluxSmem<INNER> &sm, double *tab) {
+    constexpr int F = EXT_F<INNER>, O = EXT_O<INNER>, C = EXT_C<INNER>;
+    const int N = g.N, tid = threadIdx.x, x0 = t.x0, y0 = t.y0, x1 = t.x1, y1 = t.y1;
+    const bool inx = INNER || (x0 >= 7 && x1 <= N - 5), iny = INNER || (y0 >= 7 && y1 <= N - 5);
+    Rng FX{x0 - 1, x1 + 2}, FY{y0 - 1, y1 + 2}, OX{x0 - 3, x1 + 3}, OY{y0 - 3, y1 + 3}, CX{x0 - 2, x1 + 1}, CY{y0 - 2, y1 + 1};
+    if constexpr (!INNER) {
+        const Rng fx{x0, t.fx1}, fy{y0, t.fy1};
+        FX = hull(rng_in<W42i2c>({x0, x1}, N + 1), fx);
+        FY = hull(rng_in<W42i2c>({y0, y1}, N + 1), fy);
+        OX = rng_in<W42c2i>(FX, N);
+        OY = rng_in<W42c2i>(FY, N);
+        CX = rng_in<W42c2i>(fx, N);
+        CY = rng_in<W42c2i>(fy, N);
+    }
+    const long long pb = (long long)t.p * g.plane;
+    const double *h = y + pb, *u = y + g.fs + pb, *v = y + 2 * g.fs + pb;
+    auto in = [&](int i, int j, const Rng &X, const Rng &Y) { return INNER || (i <= X.hi && j <= Y.hi); };
+
+    // the state on the boxes and the metric at the points where the later phases use it, all in flight
+    // together
+    double ru[passes<TX + F, TY + O>()], rv[passes<TX + O, TY + F>()], rh[passes<TX + C, TY + C>()];
+    double mA[passes<TX + O, TY>()], mB[passes<TX, TY + O>()];
+    double q11[passes<TX + F, TY>()], jx[passes<TX + F, TY>()], q22[passes<TX, TY + F>()], jy[passes<TX, TY + F>()];
+    each<TX + F, TY + O>(tid, [&](int k, int c, int r) {
+        if (in(FX.lo + c, OY.lo + r, FX, OY)) ru[k] = swm::at_byte(u, c_off(g, FX.lo + c, OY.lo + r));
+    });
+    each<TX + O, TY + F>(tid, [&](int k, int c, int r) {
+        if (in(OX.lo + c, FY.lo + r, OX, FY)) rv[k] = swm::at_byte(v, c_off(g, OX.lo + c, FY.lo + r));
+    });
+    each<TX + C, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, CY.lo + r, CX, CY)) rh[k] = swm::at_byte(h, c_off(g, CX.lo + c, CY.lo + r));
+    });
+    const Rng cx{x0, x1}, cy{y0, y1};
+    each<TX + O, TY>(tid, [&](int k, int c, int r) {
+        if (in(OX.lo + c, y0 + r, OX, cy)) mA[k] = swm::at_byte(g.JQo, c_off(g, OX.lo + c, y0 + r));
+    });
+    each<TX, TY + O>(tid, [&](int k, int c, int r) {
+        if (in(x0 + c, OY.lo + r, cx, OY)) mB[k] = swm::at_byte(g.JQo, c_off(g, x0 + c, OY.lo + r));
+    });
+    each<TX + F, TY>(tid, [&](int k, int c, int r) {
+        if (in(FX.lo + c, y0 + r, FX, cy)) {
+            const unsigned o = c_off(g, FX.lo + c, y0 + r);
+            q11[k] = swm::at_byte(g.Qi11x, o);
+            jx[k] = swm::at_byte(g.Jx, o);
+        }
+    });
+    each<TX, TY + F>(tid, [&](int k, int c, int r) {
+        if (in(x0 + c, FY.lo + r, cx, FY)) {
+            const unsigned o = c_off(g, x0 + c, FY.lo + r);
+            q22[k] = swm::at_byte(g.Qi22y, o);
+            jy[k] = swm::at_byte(g.Jy, o);
+        }
+    });
+    // the neighbour's tangential components beyond the panel edges, for the curl's penalties
+    double nx[3], ny[3];
+    if constexpr (!INNER) {
+        static_assert((TX + 1) * (TY + 1) <= NT, "one q point per thread");
+        each<TX + 1, TY + 1, NT - TX * TY>(tid, [&](int, int c, int r) {
+            const int i = x0 + c, j = y0 + r;
+            if (i > t.fx1 || j > t.fy1) return;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (i == 1 || i == N + 1) nx[k] = vhalo(g, y + g.fs, t.p, i == 1 ? 0 : 1, k + 1, j);
+                if (j == 1 || j == N + 1) ny[k] = vhalo(g, y + g.fs, t.p, j == 1 ? 2 : 3, k + 1, i);
+            }
+        });
+    }
+    each<TX + F, TY + O>(tid, [&](int k, int c, int r) {
+        if (in(FX.lo + c, OY.lo + r, FX, OY)) sm.u[r][c] = ru[k];
+    });
+    each<TX + O, TY + F>(tid, [&](int k, int c, int r) {
+        if (in(OX.lo + c, FY.lo + r, OX, FY)) sm.v[r][c] = rv[k];
+    });
+    each<TX + C, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, CY.lo + r, CX, CY)) sm.h[r][c] = rh[k];
+    });
+    if constexpr (!INNER) load_row_tab(tab, tid);
+    __syncthreads();
+
+    each<TX + O, TY>(tid, [&](int k, int c, int r) {
+        const int j = y0 + r;
+        if (in(OX.lo + c, j, OX, cy))
+            sm.A[r][c] = mA[k] * trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.v[q - FY.lo][c]; });
+    });
+    each<TX, TY + O>(tid, [&](int k, int c, int r) {
+        const int i = x0 + c;
+        if (in(i, OY.lo + r, cx, OY))
+            sm.B[r][c] = mB[k] * trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.u[r][q - FX.lo]; });
+    });
+    __syncthreads();
+
+    each<TX + F, TY>(tid, [&](int k, int c, int r) {
+        const int i = FX.lo + c, j = y0 + r;
+        if (!in(i, j, FX, cy)) return;
+        const double tt = trow<W42c2i, INNER>(tab, inx, i, N, [&](int q) { return sm.A[r][q - OX.lo]; });
+        const double uu = sm.u[j - OY.lo][c], ut = q11[k] * uu + tt / swm::rcp_of(jx[k]);
+        sm.ku[r][c] = jx[k] * (uu * ut) / 2.0;
+        if (i >= x0 && i <= t.fx1) {
+            const double hh = trow<W42c2i, INNER>(tab, inx, i, N, [&](int q) { return sm.h[j - CY.lo][q - CX.lo]; });
+            const double hu = ut * hh;
+            swm::at_byte(G + pb, c_off(g, i, j)) = jx[k] * hu;
+        }
+    });
+    each<TX, TY + F>(tid, [&](int k, int c, int r) {
+        const int i = x0 + c, j = FY.lo + r;
+        if (!in(i, j, cx, FY)) return;
+        const double tt = trow<W42c2i, INNER>(tab, iny, j, N, [&](int q) { return sm.B[q - OY.lo][c]; });
+        const double vv = sm.v[r][i - OX.lo], vt = q22[k] * vv + tt / swm::rcp_of(jy[k]);
+        sm.kv[r][c] = jy[k] * (vv * vt) / 2.0;
+        if (j >= y0 && j <= t.fy1) {
+            const double hh = trow<W42c2i, INNER>(tab, iny, j, N, [&](int q) { return sm.h[q - CY.lo][i - CX.lo]; });
+            const double hv = vt * hh;
+            swm::at_byte(G + g.fs + pb, c_off(g, i, j)) = jy[k] * hv;
+        }
+    });
+    __syncthreads();
+
+    each<TX, TY>(tid, [&](int, int c, int r) {
+        const int i = x0 + c, j = y0 + r;
+        if (!in(i, j, cx, cy)) return;
+        const unsigned o = c_off(g, i, j);
+        const double kuh = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.ku[r][q - FX.lo]; });
+        const double kvh = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.kv[q - FY.lo][c]; });
+        double ke = (kuh + kvh) / swm::rcp_of(swm::at_byte(g.Jo, o));
+        ke = ke + g.grav * sm.h[j - CY.lo][i - CX.lo] + g.grav * (g.hs ? swm::at_byte(g.hs + pb, o) : 0.0);
+        swm::at_byte(KE + pb, o) = ke;
+    });
+    // curl: staggered differences of v along x and u along y with the interface penalties, the
+    // neighbour's tangential components read through vsrc
+    each<INNER ? TX : TX + 1, INNER ? TY : TY + 1, NT - TX * TY>(tid, [&](int, int c, int r) {
+        const int i = x0 + c, j = y0 + r, n = N + 1;
+        if (!INNER && (i > t.fx1 || j > t.fy1)) return;
+        const unsigned o = c_off(g, i, j);
+        auto vx = [&](int q) { return sm.v[j - FY.lo][q - OX.lo]; };
+        auto uy = [&](int q) { return sm.u[q - OY.lo][i - FX.lo]; };
+        double dvx = trow<D42c2i, INNER>(tab, inx, i, N, vx);
+        double duy = trow<D42c2i, INNER>(tab, iny, j, N, uy);
+        if constexpr (!INNER) {
+            if (i == 1 || i == n) {
+                double d = 0.0;
+#pragma unroll
+                for (int k = 1; k <= 3; ++k) d = d + PROJ[k - 1] * (i == 1 ? vx(k) - nx[k - 1] : nx[k - 1] - vx(n - k));
+                dvx = dvx + 0.5 * d / A_IF1;
+            }
+            if (j == 1 || j == n) {
+                double d = 0.0;
+#pragma unroll
+                for (int k = 1; k <= 3; ++k) d = d + PROJ[k - 1] * (j == 1 ? uy(k) - ny[k - 1] : ny[k - 1] - uy(n - k));
+                duy = duy + 0.5 * d / A_IF1;
+            }
+        }
+        swm::at_byte(W + pb, o) = (dvx - duy) / swm::rcp_of(swm::at_byte(g.Jq, o) * g.hx * g.scale);
+    });
+}
+
+template <bool INNER>
+struct TendSmem {
+    static constexpr int F = EXT_F<INNER>, C = EXT_C<INNER>, Q = EXT_Q<INNER>;
+    double W[TY + Q][TX + Q], gu[TY + C][TX + F], gv[TY + F][TX + C], ke[TY + C][TX + C];
+    double fu[TY + C][TX + Q], fv[TY + Q][TX + C];   // the synced curl at x and y points
+    double cu[TY][TX + C], cv[TY + C][TX];           // Coriolis terms at o points
+};
+
+// interpolator_w2h of the synced curl (interpolator_w2h_mod.f90:40-68), the vector-invariant Coriolis
+// terms (coriolis_Cgrid_mod.f90:86-103) and their interpolation to faces (interpolator_p2uv_mod.f90:
+// 90-113), dh = -div(J hu, J hv) with the centre penalties (div_c_sbp42_mod.f90:70-99,
+// sbp_operator_mod.f90:344-413), du = -grad_x(KE) + cor_u, dv = -grad_y(KE) + cor_v
+// (operator_swm_mod.f90:94-95), and the RK4 stage update
+template <int RKM, bool INNER>
+static __device__ __forceinline__ void tend_tile(const CGeo &g, const double *__restrict__ h, const double *__restrict__ G,
+                                          const double *__restrict__ KE, const double *__restrict__ W,
+                                          const RkArgs &rk, const CTile &t, TendSmem<INNER> &sm, double *tab) {
+    constexpr int F = EXT_F<INNER>, C = EXT_C<INNER>, Q = EXT_Q<INNER>;
+    const int N = g.N, tid = threadIdx.x, x0 = t.x0, y0 = t.y0, x1 = t.x1, y1 = t.y1;
+    const bool inx = INNER || (x0 >= 7 && x1 <= N - 5), iny = INNER || (y0 >= 7 && y1 <= N - 5);
+    Rng GX{x0 - 1, x1 + 2}, GY{y0 - 1, y1 + 2}, CX{x0 - 2, x1 + 1}, CY{y0 - 2, y1 + 1}, QX{x0 - 3, x1 + 3}, QY{y0 - 3, y1 + 3};
+    const Rng cx{x0, x1}, cy{y0, y1};
+    if constexpr (!INNER) {
+        GX = rng_in<W42i2c>(cx, N + 1);
+        GY = rng_in<W42i2c>(cy, N + 1);
+        CX = hull(rng_in<W42c2i>({x0, t.fx1}, N), cx);
+        CY = hull(rng_in<W42c2i>({y0, t.fy1}, N), cy);
+        QX = rng_in<W42i2c>(CX, N + 1);
+        QY = rng_in<W42i2c>(CY, N + 1);
+    }
+    const long long pb = (long long)t.p * g.plane;
+    auto in = [&](int i, int j, const Rng &X, const Rng &Y) { return INNER || (i <= X.hi && j <= Y.hi); };
+
+    // the four fields on the boxes, and the own points' stage vectors and the o points' f and h, all in
+    // flight together
+    double rw[passes<TX + Q, TY + Q>()], ru[passes<TX + F, TY + C>()], rv[passes<TX + C, TY + F>()], re[passes<TX + C, TY + C>()];
+    double fa[passes<TX + C, TY>()], ha[passes<TX + C, TY>()], fb[passes<TX, TY + C>()], hb[passes<TX, TY + C>()];
+    each<TX + Q, TY + Q>(tid, [&](int k, int c, int r) {
+        const int i = QX.lo + c, j = QY.lo + r;
+        if (INNER) rw[k] = swm::at_byte(W + pb, c_off(g, i, j));
+        else if (in(i, j, QX, QY)) rw[k] = curl_at(g, W, t.p, i, j);
+    });
+    each<TX + F, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(GX.lo + c, CY.lo + r, GX, CY)) ru[k] = swm::at_byte(G + pb, c_off(g, GX.lo + c, CY.lo + r));
+    });
+    each<TX + C, TY + F>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, GY.lo + r, CX, GY)) rv[k] = swm::at_byte(G + g.fs + pb, c_off(g, CX.lo + c, GY.lo + r));
+    });
+    each<TX + C, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, CY.lo + r, CX, CY)) re[k] = swm::at_byte(KE + pb, c_off(g, CX.lo + c, CY.lo + r));
+    });
+    each<TX + C, TY>(tid, [&](int k, int c, int r) {
+        if (!in(CX.lo + c, y0 + r, CX, cy)) return;
+        const unsigned o = c_off(g, CX.lo + c, y0 + r);
+        fa[k] = swm::at_byte(g.fo + pb, o);
+        ha[k] = swm::at_byte(h + pb, o);
+    });
+    each<TX, TY + C>(tid, [&](int k, int c, int r) {
+        if (!in(x0 + c, CY.lo + r, cx, CY)) return;
+        const unsigned o = c_off(g, x0 + c, CY.lo + r);
+        fb[k] = swm::at_byte(g.fo + pb, o);
+        hb[k] = swm::at_byte(h + pb, o);
+    });
+    // the neighbours' values that the penalties of the own points read: copies of the shared faces (nx, ny),
+    // the potential beyond the x edges (ex) and the y edges (ey)
+    double nx = 0.0, ny = 0.0, ex[3], ey[3];
+    if constexpr (!INNER) {
+        static_assert((TX + 1) * (TY + 1) <= NT, "one point of each type per thread");
+        each<TX, TY>(tid, [&](int, int c, int r) {
+            const int i = x0 + c, j = y0 + r;
+            if (!in(i, j, cx, cy)) return;
+            if (i <= 3 || i >= N - 2) nx = fhalo(g, G, t.p, i <= 3 ? 0 : 1, j);
+            if (j <= 3 || j >= N - 2) ny = fhalo(g, G, t.p, j <= 3 ? 2 : 3, i);
+        });
+        each<TX + 1, TY, NT - TX * TY>(tid, [&](int, int c, int r) {
+            const int i = x0 + c, j = y0 + r;
+            if ((i == 1 || i == N + 1) && j <= y1)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) ex[k] = ohalo(g, KE, t.p, i == 1 ? 0 : 1, k + 1, j);
+        });
+        each<TX, TY + 1>(tid, [&](int, int c, int r) {
+            const int i = x0 + c, j = y0 + r;
+            if ((j == 1 || j == N + 1) && i <= x1)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) ey[k] = ohalo(g, KE, t.p, j == 1 ? 2 : 3, k + 1, i);
+        });
+    }
+    each<TX + Q, TY + Q>(tid, [&](int k, int c, int r) {
+        if (in(QX.lo + c, QY.lo + r, QX, QY)) sm.W[r][c] = rw[k];
+    });
+    each<TX + F, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(GX.lo + c, CY.lo + r, GX, CY)) sm.gu[r][c] = ru[k];
+    });
+    each<TX + C, TY + F>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, GY.lo + r, CX, GY)) sm.gv[r][c] = rv[k];
+    });
+    each<TX + C, TY + C>(tid, [&](int k, int c, int r) {
+        if (in(CX.lo + c, CY.lo + r, CX, CY)) sm.ke[r][c] = re[k];
+    });
+    if constexpr (!INNER) load_row_tab(tab, tid);
+    __syncthreads();
+
+    each<TX + Q, TY + C>(tid, [&](int, int c, int r) {
+        const int j = CY.lo + r;
+        if (in(QX.lo + c, j, QX, CY))
+            sm.fu[r][c] = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.W[q - QY.lo][c]; });
+    });
+    each<TX + C, TY + Q>(tid, [&](int, int c, int r) {
+        const int i = CX.lo + c;
+        if (in(i, QY.lo + r, CX, QY))
+            sm.fv[r][c] = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.W[r][q - QX.lo]; });
+    });
+    __syncthreads();
+
+    // curl_p = (I_x fu + I_y fv)/2 at the o point (i, j)
+    auto curl_p = [&](int i, int j) {
+        const double fuh = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.fu[j - CY.lo][q - QX.lo]; });
+        const double fvh = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.fv[q - QY.lo][i - CX.lo]; });
+        return 0.5 * fuh + 0.5 * fvh;
+    };
+    each<TX + C, TY>(tid, [&](int k, int c, int r) {
+        const int i = CX.lo + c, j = y0 + r;
+        if (!in(i, j, CX, cy)) return;
+        const double gv = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.gv[q - GY.lo][c]; });
+        sm.cu[r][c] = (fa[k] + curl_p(i, j)) * gv / swm::rcp_of(ha[k]);
+    });
+    each<TX, TY + C>(tid, [&](int k, int c, int r) {
+        const int i = x0 + c, j = CY.lo + r;
+        if (!in(i, j, cx, CY)) return;
+        const double gu = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.gu[r][q - GX.lo]; });
+        sm.cv[r][c] = -(fb[k] + curl_p(i, j)) * gu / swm::rcp_of(hb[k]);
+    });
+    // the stage vectors of the own points, in flight across the barrier (tiles of interior rows: one
+    // point of each field per thread)
+    RkPre qh{}, qu{}, qv{};
+    if constexpr (INNER) {
+        const int m = tid & (TX * TY - 1);   // the own point, as the loops below deal them
+        const unsigned o = c_off(g, x0 + m % TX, y0 + m / TX);
+        if (tid < TX * TY) {
+            qh = rk_pre<RKM>(rk, pb, o);
+            qv = rk_pre<RKM>(rk, 2 * g.fs + pb, o);
+        }
+        if (tid >= NT - TX * TY) qu = rk_pre<RKM>(rk, g.fs + pb, o);
+    }
+    __syncthreads();
+
+    each<TX, TY>(tid, [&](int, int c, int r) {
+        const int i = x0 + c, j = y0 + r;
+        if (!in(i, j, cx, cy)) return;
+        const unsigned o = c_off(g, i, j);
+        auto gx = [&](int q) { return sm.gu[j - CY.lo][q - GX.lo]; };
+        auto gy = [&](int q) { return sm.gv[q - GY.lo][i - CX.lo]; };
+        double dx = trow<D42i2c, INNER>(tab, inx, i, N + 1, gx);
+        double dy = trow<D42i2c, INNER>(tab, iny, j, N + 1, gy);
+        if constexpr (!INNER) {
+            if (i <= 3) dx = dx + 0.5 * PEN_L[i - 1] * (gx(1) - nx);
+            if (i >= N - 2) dx = dx + 0.5 * PEN_R[i - N + 2] * (nx - gx(N + 1));
+            if (j <= 3) dy = dy + 0.5 * PEN_L[j - 1] * (gy(1) - ny);
+            if (j >= N - 2) dy = dy + 0.5 * PEN_R[j - N + 2] * (ny - gy(N + 1));
+            qh = rk_pre<RKM>(rk, pb, o);
+        }
+        const double div = (dx + dy) / swm::rcp_of(swm::at_byte(g.Jo, o) * g.hx * g.scale);
+        rk_out<RKM>(rk, pb, o, qh, -1.0 * div);
+    });
+    each<INNER ? TX : TX + 1, TY, NT - TX * TY>(tid, [&](int, int c, int r) {
+        const int i = x0 + c, j = y0 + r;
+        if (!INNER && (i > t.fx1 || j > y1)) return;
+        const unsigned o = c_off(g, i, j);
+        const double gx = grad_row<INNER>(tab, inx, i, N, g.dx1, [&](int q) { return sm.ke[j - CY.lo][q - CX.lo]; }, ex);
+        const double cu = trow<W42c2i, INNER>(tab, inx, i, N, [&](int q) { return sm.cu[r][q - CX.lo]; });
+        if constexpr (!INNER) qu = rk_pre<RKM>(rk, g.fs + pb, o);
+        rk_out<RKM>(rk, g.fs + pb, o, qu, -1.0 * gx + 1.0 * cu);
+    });
+    each<TX, INNER ? TY : TY + 1>(tid, [&](int, int c, int r) {
+        const int i = x0 + c, j = y0 + r;
+        if (!INNER && (i > x1 || j > t.fy1)) return;
+        const unsigned o = c_off(g, i, j);
+        const double gy = grad_row<INNER>(tab, iny, j, N, g.dx1, [&](int q) { return sm.ke[q - CY.lo][i - CX.lo]; }, ey);
+        const double cv = trow<W42c2i, INNER>(tab, iny, j, N, [&](int q) { return sm.cv[q - CY.lo][c]; });
+        if constexpr (!INNER) qv = rk_pre<RKM>(rk, 2 * g.fs + pb, o);
+        rk_out<RKM>(rk, 2 * g.fs + pb, o, qv, -1.0 * gy + 1.0 * cv);
+    });
+}
+
+};
+
+// 16 x 8 cells and two threads per cell: the phases of a tile have 1.3 to 3 tasks per cell, a block is a
+// chain of load, three LDS phases and stores whose length is what a launch of few tiles takes, and 8 such
+// blocks fit a CU.  RK4 step (8 launches), C90 / C384 / C512: 73 / 241 / 361 us; 8 x 8 cells 75 / 342 / 537,
+// 32 x 4 69 / 273 / 406, 32 x 8 with 512 threads 85 / 306 / 460, with 256 124 / 287 / 383; the
+// eight-launch form with its intermediates in memory 140 / 391 us.
+using Tiles = CTiles<16, 8, 256>;
+
+__global__ void __launch_bounds__(Tiles::THREADS) k_flux(CGeo g, const double *__restrict__ y, double *__restrict__ G,
+                                                         double *__restrict__ KE, double *__restrict__ W, int ntiles) {
+    __shared__ union { Tiles::FluxSmem<true> in; Tiles::FluxSmem<false> any; } sm;
+    __shared__ double tab[ROW_SIZE];
+    const CTile t = Tiles::c_tile(g, swm::xcd_tile(blockIdx.x, ntiles));
+    if (Tiles::c_inner(g, t)) Tiles::flux_tile<true>(g, y, G, KE, W, t, sm.in, tab);
+    else Tiles::flux_tile<false>(g, y, G, KE, W, t, sm.any, tab);
+}
+
 template <int RKM>
-__global__ void __launch_bounds__(256) k_mom(CGeo g, const double *__restrict__ KE, const double *__restrict__ cup,
-                                             const double *__restrict__ cvp, RkArgs r) {
-    C_POINT
-    const int N = g.N;
-    if (i <= N + 1 && j <= N) {
-        const long long id = cid(g, p, i, j);
-        const double *row = KE + cid(g, p, 0, j);
-        const double gx = grad_line(i, N, [&](int k) {
-            return k < 1 ? ohalo(g, KE, p, 0, 1 - k, j) : k > N ? ohalo(g, KE, p, 1, k - N, j) : row[k];
-        }, g.dx1);
-        const double cu = sop<W42c2i>(i, N, cup + cid(g, p, 0, j), 1);
-        rk_out<RKM>(r, g.fs + id, -1.0 * gx + 1.0 * cu);
-    }
-    if (i <= N && j <= N + 1) {
-        const long long id = cid(g, p, i, j);
-        const double *col = KE + cid(g, p, i, 0);
-        const double gy = grad_line(j, N, [&](int k) {
-            return k < 1 ? ohalo(g, KE, p, 2, 1 - k, i) : k > N ? ohalo(g, KE, p, 3, k - N, i)
-                                                               : col[(long long)k * g.pitch];
-        }, g.dx1);
-        const double cv = sop<W42c2i>(j, N, cvp + cid(g, p, i, 0), g.pitch);
-        rk_out<RKM>(r, 2 * g.fs + id, -1.0 * gy + 1.0 * cv);
-    }
+__global__ void __launch_bounds__(Tiles::THREADS) k_tend(CGeo g, const double *__restrict__ h, const double *__restrict__ G,
+                                                            const double *__restrict__ KE, const double *__restrict__ W,
+                                                            RkArgs r, int ntiles) {
+    __shared__ union { Tiles::TendSmem<true> in; Tiles::TendSmem<false> any; } sm;
+    __shared__ double tab[ROW_SIZE];
+    const CTile t = Tiles::c_tile(g, swm::xcd_tile(blockIdx.x, ntiles));
+    if (Tiles::c_inner(g, t)) Tiles::tend_tile<RKM, true>(g, h, G, KE, W, r, t, sm.in, tab);
+    else Tiles::tend_tile<RKM, false>(g, h, G, KE, W, r, t, sm.any, tab);
 }
 
 // ---- get_diagnostics on the C grid (operator_swm_mod.f90:115-155, calc_energy :211-236) ----
@@ -552,9 +920,7 @@ __global__ void __launch_bounds__(swm::FINAL_THREADS) k_cdiag_final(const double
 // ------------------------------------------------------------------------------------------------
 namespace {
 
-constexpr int CW_G = 0 /* and 1 */, CW_KEU = 2, CW_KEV = 3, CW_KE = 4, CW_W = 5, CW_CUP = 6, CW_CVP = 7,
-              CW_K = 8 /* 3 stages x 3 fields */, CW_YA = 17, CW_YB = 20, CW_A = 23, CW_B = 24, CW_FU = 25,
-              CW_FV = 26, CW_COUNT = 27;
+constexpr int CW_G = 0 /* and 1 */, CW_KE = 2, CW_W = 3, CW_ACC = 4, CW_YA = 7, CW_YB = 10, CW_COUNT = 13;
 
 swmc::CGeo make_cgeo(const swm_cctx *c) {
     swmc::CGeo g;
@@ -567,7 +933,8 @@ swmc::CGeo make_cgeo(const swm_cctx *c) {
     g.Qi12o = G + 4 * P;
     g.Qi11x = G + 5 * P;
     g.Qi22y = G + 6 * P;
-    g.fo = G + 7 * P;
+    g.JQo = G + 7 * P;
+    g.fo = G + 8 * P;
     g.hs = c->hs;
     g.vsrc = c->vsrc;
     g.fsrc = c->fsrc;
@@ -590,56 +957,31 @@ swmc::CGeo make_cgeo(const swm_cctx *c) {
     return g;
 }
 
-// operator_swm_t%apply on the C grid for the input y (h, u, v), eight launches; the tendencies go
-// where RKM says (RK_RHS: r.k; RK_STAGE: r.k and the next stage input; RK_FINAL: the state)
+// operator_swm_t%apply on the C grid for the input y (h, u, v), two launches; the tendencies go
+// where RKM says
 template <int RKM>
 int c_enqueue_rhs(swm_cctx *c, const double *y, const swmc::RkArgs &r) {
+    using K = swmc::Tiles;
     const swmc::CGeo g = make_cgeo(c);
-    const dim3 blk(swmc::BX, swmc::BY), grd(8 * g.per);
-    const size_t F = (size_t)c->fs;
-    const double *h = y, *u = y + F, *v = y + 2 * F;
-    hipLaunchKernelGGL(swmc::k_contra_o, grd, blk, 0, c->stream, g, u, v, c->wf(CW_A), c->wf(CW_B));
-    hipLaunchKernelGGL(swmc::k_flux, grd, blk, 0, c->stream, g, h, u, v, c->wf(CW_A), c->wf(CW_B), c->wf(CW_G),
-                       c->wf(CW_KEU), c->wf(CW_KEV));
-    hipLaunchKernelGGL(swmc::k_ke_div<RKM>, grd, blk, 0, c->stream, g, h, c->wf(CW_KEU), c->wf(CW_KEV), c->wf(CW_G),
-                       c->wf(CW_KE), r);
-    hipLaunchKernelGGL(swmc::k_curl, grd, blk, 0, c->stream, g, u, c->wf(CW_W));
-    const int nsync = c->nqpairs + c->nqcorners;
-    hipLaunchKernelGGL(swmc::k_qsync_edges, dim3((nsync + 255) / 256), dim3(256), 0, c->stream, c->nqpairs,
-                       c->nqcorners, c->qpairs, c->qcorners, c->wf(CW_W));
-    hipLaunchKernelGGL(swmc::k_w2uv, grd, blk, 0, c->stream, g, c->wf(CW_W), c->wf(CW_FU), c->wf(CW_FV));
-    hipLaunchKernelGGL(swmc::k_cor_o, grd, blk, 0, c->stream, g, h, c->wf(CW_FU), c->wf(CW_FV), c->wf(CW_G),
-                       c->wf(CW_CUP), c->wf(CW_CVP));
-    hipLaunchKernelGGL(swmc::k_mom<RKM>, grd, blk, 0, c->stream, g, c->wf(CW_KE), c->wf(CW_CUP), c->wf(CW_CVP), r);
+    const int ntiles = 6 * ((c->N + K::X - 1) / K::X) * ((c->N + K::Y - 1) / K::Y);
+    const dim3 blk(K::THREADS), grd(ntiles);
+    hipLaunchKernelGGL(swmc::k_flux, grd, blk, 0, c->stream, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W), ntiles);
+    hipLaunchKernelGGL(swmc::k_tend<RKM>, grd, blk, 0, c->stream, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W), r,
+                       ntiles);
     HIP_TRY(hipGetLastError());
     return SWM_OK;
 }
 
-// rk4_t%step (rk4_mod.f90:20-42): stage inputs state -> yA -> yB -> yA, the stage updates and the
-// final combination inside the tendency kernels
+// rk4_t%step (rk4_mod.f90:20-42): stage inputs state -> yA -> yB -> yA, the stage updates inside the
+// tendency kernel; no stage writes a buffer that it reads at other points
 int c_enqueue_rk4_step(swm_cctx *c, double *state, double dt) {
-    double *k[3] = {c->wf(CW_K), c->wf(CW_K + 3), c->wf(CW_K + 6)};
-    const double *in[4] = {state, c->wf(CW_YA), c->wf(CW_YB), c->wf(CW_YA)};
-    double *next[3] = {c->wf(CW_YA), c->wf(CW_YB), c->wf(CW_YA)};
-    const double b[3] = {0.5 * dt, 0.5 * dt, dt};
+    const double c1 = 0.5 * dt, c2 = dt / 6.0, c3 = dt / 3.0;
+    double *acc = c->wf(CW_ACC), *yA = c->wf(CW_YA), *yB = c->wf(CW_YB);
     int rc;
-    for (int s = 0; s < 3; ++s) {
-        swmc::RkArgs r{};
-        r.k = k[s];
-        r.v0 = state;
-        r.yn = next[s];
-        r.b = b[s];
-        if ((rc = c_enqueue_rhs<swmc::RK_STAGE>(c, in[s], r))) return rc;
-    }
-    swmc::RkArgs r{};
-    r.v0 = state;
-    r.v0w = state;
-    r.k0 = k[0];
-    r.k1 = k[1];
-    r.k2 = k[2];
-    r.c2 = dt / 6.0;
-    r.c3 = dt / 3.0;
-    return c_enqueue_rhs<swmc::RK_FINAL>(c, in[3], r);
+    if ((rc = c_enqueue_rhs<swmc::RK_S1>(c, state, {yA, state, acc, c1, c2}))) return rc;
+    if ((rc = c_enqueue_rhs<swmc::RK_S23>(c, yA, {yB, state, acc, c1, c3}))) return rc;
+    if ((rc = c_enqueue_rhs<swmc::RK_S23>(c, yB, {yA, state, acc, dt, c3}))) return rc;
+    return c_enqueue_rhs<swmc::RK_S4>(c, yA, {state, nullptr, acc, 0.0, c2});
 }
 
 void c_drop_graphs(swm_cctx *c) {
@@ -652,7 +994,7 @@ void c_free(swm_cctx *c) {
     if (!c) return;
     c_drop_graphs(c);
     for (void *p : {(void *)c->geo, (void *)c->hs, (void *)c->lists, (void *)c->signs, (void *)c->work, (void *)c->qw,
-                    (void *)c->dpart, (void *)c->qpairs, (void *)c->ecs_src, (void *)c->ecs_sign,
+                    (void *)c->dpart, (void *)c->ecs_src, (void *)c->ecs_sign,
                     (void *)c->ecs_strips, (void *)c->ecs_ow, (void *)c->ecs_oind, (void *)c->ecs_vt,
                     (void *)c->ecs_vti, (void *)c->ecs_ext})
         if (p) (void)hipFree(p);
@@ -727,9 +1069,9 @@ extern "C" int swm_c_create(swm_cctx **out, int N, const char *div, const char *
     swmh_c_geometry(N, 2, swmc::H, c->rows, c->pitch, omega, axis, G + 2 * F, nullptr, nullptr, G + 6 * F, nullptr);
     swmh_c_geometry(N, 3, swmc::H, c->rows, c->pitch, omega, axis, G + 3 * F, nullptr, nullptr, nullptr, nullptr);
     // device copy: panel 0 of the seven metric planes (every panel holds the same values, checked
-    // here bit for bit), then f on all six panels
+    // here bit for bit), the product J Qi12 at o points, then f on all six panels
     const size_t P = (size_t)c->plane;
-    std::vector<double> dgeo(7 * P + F);
+    std::vector<double> dgeo(8 * P + F);
     for (int w = 0; w < 7; ++w) {
         const double *m = G + (size_t)w * F;
         for (int p = 1; p < 6; ++p)
@@ -737,7 +1079,8 @@ extern "C" int swm_c_create(swm_cctx **out, int N, const char *div, const char *
                 return bail(fail(SWM_EARG, "C-grid metric differs between panels"));
         std::copy(m, m + P, dgeo.begin() + (size_t)w * P);
     }
-    std::copy(G + 7 * F, G + 8 * F, dgeo.begin() + 7 * P);
+    for (size_t k = 0; k < P; ++k) dgeo[7 * P + k] = dgeo[k] * dgeo[4 * P + k];
+    std::copy(G + 7 * F, G + 8 * F, dgeo.begin() + 8 * P);
     if (hipMalloc((void **)&c->geo, dgeo.size() * sizeof(double)) != hipSuccess ||
         hipMemcpy(c->geo, dgeo.data(), dgeo.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(SWM_EHIP, "C-grid geometry upload failed"));
@@ -779,68 +1122,6 @@ extern "C" int swm_c_create(swm_cctx **out, int N, const char *div, const char *
     c->qnb = c->osrc + mo;
     c->vsg = c->signs;
     c->fsg = c->signs + mv;
-    {
-        // q-point sync groups from the neighbour copies qn[(p*4+e)*(N+1) + k-1] of edge point k of
-        // edge e (0: i = 1, 1: i = N+1, 2: j = 1, 3: j = N+1) of panel p
-        const int n = N + 1;
-        auto own = [&](int p, int i, int j) { return ((long long)p * c->rows + (j - 1 + swmc::H)) * c->pitch + (i - 1 + swmc::H); };
-        auto nb = [&](int p, int e, int k) { return qn[((size_t)p * 4 + e) * n + (k - 1)]; };
-        std::vector<long long> pairs, corners;
-        for (int p = 0; p < 6; ++p)
-            for (int e = 0; e < 4; ++e)
-                for (int k = 2; k <= n - 1; ++k) {
-                    const int i = e == 0 ? 1 : e == 1 ? n : k, j = e == 2 ? 1 : e == 3 ? n : k;
-                    const long long a = own(p, i, j), b = nb(p, e, k);
-                    if (a < b) { pairs.push_back(a); pairs.push_back(b); }
-                }
-        // corner copies: (own, first, second) in the order of halo_Ah_scalar_sync_mod.f90:56-72
-        struct Copy { long long o, a, b; };
-        std::vector<Copy> cps;
-        for (int p = 0; p < 6; ++p) {
-            cps.push_back({own(p, 1, 1), nb(p, 0, 1), nb(p, 2, 1)});
-            cps.push_back({own(p, 1, n), nb(p, 0, n), nb(p, 3, 1)});
-            cps.push_back({own(p, n, 1), nb(p, 1, 1), nb(p, 2, n)});
-            cps.push_back({own(p, n, n), nb(p, 1, n), nb(p, 3, n)});
-        }
-        std::vector<bool> used(cps.size(), false);
-        for (size_t x = 0; x < cps.size(); ++x) {
-            if (used[x]) continue;
-            long long g3[3] = {cps[x].o, cps[x].a, cps[x].b};
-            size_t idx[3] = {x, 0, 0};
-            for (int m = 1; m < 3; ++m) {
-                idx[m] = cps.size();
-                for (size_t y = 0; y < cps.size(); ++y)
-                    if (cps[y].o == g3[m]) idx[m] = y;
-                if (idx[m] == cps.size()) return bail(fail(SWM_EARG, "cube corner copies do not form a group"));
-            }
-            long long ords[3];
-            for (int m = 0; m < 3; ++m) {
-                const Copy &cp = cps[idx[m]];
-                int fa = -1, fb = -1;
-                for (int t = 0; t < 3; ++t) {
-                    if (g3[t] == cp.a) fa = t;
-                    if (g3[t] == cp.b) fb = t;
-                }
-                if (fa < 0 || fb < 0 || fa == m || fb == m || fa == fb)
-                    return bail(fail(SWM_EARG, "cube corner copies do not form a group"));
-                used[idx[m]] = true;
-                ords[m] = 3 * fa + fb;
-            }
-            for (int m = 0; m < 3; ++m) corners.push_back(g3[m]);
-            for (int m = 0; m < 3; ++m) corners.push_back(ords[m]);
-        }
-        if (pairs.size() != (size_t)2 * 12 * (n - 2) || corners.size() != (size_t)6 * 8)
-            return bail(fail(SWM_EARG, "q-point sync groups do not match the cube topology"));
-        c->nqpairs = (int)(pairs.size() / 2);
-        c->nqcorners = (int)(corners.size() / 6);
-        std::vector<long long> Q(pairs);
-        Q.insert(Q.end(), corners.begin(), corners.end());
-        if (hipMalloc((void **)&c->qpairs, Q.size() * sizeof(long long)) != hipSuccess ||
-            hipMemcpy(c->qpairs, Q.data(), Q.size() * sizeof(long long), hipMemcpyHostToDevice) != hipSuccess)
-            return bail(fail(SWM_EHIP, "q-point sync group upload failed"));
-        c->qcorners = c->qpairs + pairs.size();
-    }
-
     {
         // create_mass_coefficients (quadrature_factory_mod.f90:156-175): A_centers (13/12, 7/8,
         // 25/24, 1, ...) and A_interfaces (7/18, 9/8, 1, 71/72, 1, ...) from both ends
@@ -949,9 +1230,7 @@ extern "C" int swm_c_set_orography(swm_cctx *c, const double *hs, int hw) {
 extern "C" int swm_c_rhs(swm_cctx *c, const void *vin, void *vout) {
     if (!c || !vin || !vout) return fail(SWM_EARG, "NULL argument");
     if (vin == vout) return fail(SWM_EARG, "vin and vout must differ");
-    swmc::RkArgs r{};
-    r.k = (double *)vout;
-    return c_enqueue_rhs<swmc::RK_RHS>(c, (const double *)vin, r);
+    return c_enqueue_rhs<swmc::RK_RHS>(c, (const double *)vin, {(double *)vout, nullptr, nullptr, 0.0, 0.0});
 }
 
 extern "C" int swm_c_rk4_steps(swm_cctx *c, void *state, double dt, int nsteps) {
