@@ -106,8 +106,8 @@ __device__ __forceinline__ V3 sbp_col_T(int c, int n, const G &get) {
 struct AdjGeo {
     const double *J, *Qi11, *Qi12, *Qi22, *f;
     int n, pitch, es;
-    long long fs;
-    double hxs, grav;
+    long long fs, mps;   // elements per field; panel stride of J, Qi (0 where all panels hold the same values)
+    double hxs, rhxs, grav;
 };
 
 // One launch for the pointwise seeds and the transposed edge syncs.  Blocks below nb_edge
@@ -293,136 +293,293 @@ __device__ __forceinline__ void adj_rows(int a0, int ae, int n, int &lo, int &hi
     }
 }
 
-template <int ORD, int MODE, int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) adj_tile(AdjGeo g, AdjArgs A, AdjEll ell) {
-    using Tl = AdjTile<ORD, TX, TY>;
-    __shared__ double box[4][Tl::LH][Tl::LW];
-    const int n = g.n, ns = 6 * g.es;
-    const int ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
-    const int tile = xcd_tile(blockIdx.x, 6 * ntx * nty);
-    const int p = tile / (ntx * nty), rem = tile - p * (ntx * nty);
-    const int x0 = (rem % ntx) * TX, y0 = (rem / ntx) * TY;
-    const int xe = x0 + TX < n ? x0 + TX : n, ye = y0 + TY < n ? y0 + TY : n;
-    int lx, hx, ly, hy;
-    adj_rows<ORD, TX, TY>(x0, xe, n, lx, hx);
-    adj_rows<ORD, TX, TY>(y0, ye, n, ly, hy);
-    const double alpha = A.alpha, hxs = g.hxs;
-    const double *__restrict__ y = A.y;
-    const double *__restrict__ M = A.M;
+// The columns of D as a table: classes 0 .. B-1 the left closure columns (weights of rows first .. first +
+// count - 1, ascending), B the interior column (rows c + R down to c - R); a right closure column is the
+// left one mirrored and negated.  One code path for all points of a tile with closure columns.
+template <int ORD>
+struct ColWeights {
+    using T = SbpT<ORD>;
+    static constexpr int B = T::B, NR = T::B + T::W;
+    static constexpr int first(int c) {
+        for (int r = 0; r < NR; ++r)
+            if (T::left(r, c) != 0.0) return r;
+        return 0;
+    }
+    static constexpr int count(int c) {
+        int last = 0;
+        for (int r = 0; r < NR; ++r)
+            if (T::left(r, c) != 0.0) last = r;
+        return last - first(c) + 1;
+    }
+    static constexpr int widest() {
+        int w = T::S::WIN;
+        for (int c = 0; c < B; ++c) w = count(c) > w ? count(c) : w;
+        return w;
+    }
+    static constexpr int NW = widest(), SIZE = (B + 1) * NW;
+    double w[SIZE];
+    constexpr ColWeights() : w() {
+        for (int c = 0; c < B; ++c)
+            for (int m = 0; m < count(c); ++m) w[c * NW + m] = T::left(first(c) + m, c);
+        for (int m = 0; m < T::S::WIN; ++m) w[B * NW + m] = T::S::Qin[m];
+    }
+    // 4-bit first rows and counts of the closure columns
+    static constexpr unsigned long long packed(bool cnt) {
+        unsigned long long v = 0;
+        for (int c = 0; c < B; ++c) v |= (unsigned long long)(cnt ? count(c) : first(c)) << (4 * c);
+        return v;
+    }
+};
+template <int ORD>
+__device__ const ColWeights<ORD> col_weights = ColWeights<ORD>();
 
-    // seeds at the point (px, py) of panel p into LDS
-    auto seed = [&](int px, int py) {
-        const long long o = ((long long)p * n + py) * g.pitch + px;
-        double w0, w1, w2, w3;
-        if (px == 0 || py == 0 || px == n - 1 || py == n - 1) {
-            const int sl = p * g.es + edge_slot(n, px, py);
-            int so[ELL_S], vx[ELL_V], vy[ELL_V];
-            double sw[ELL_S], wx[ELL_V], wy[ELL_V];
+// (D^T y)_c from the table, get(r) the three transported fields at row r; rows of weight zero do not
+// enter the sum
+template <int ORD, typename G>
+__device__ __forceinline__ V3 tab_col_T(const double *__restrict__ tab, int c, int n, const G &get) {
+    using C = ColWeights<ORD>;
+    constexpr unsigned long long FIRST = C::packed(false), COUNT = C::packed(true);
+    const bool right = c >= n - C::B;
+    const int k = right ? n - 1 - c : c;
+    int start = c + SbpT<ORD>::R, step = -1, cnt = Sbp<ORD>::WIN, cls = C::B;
+    if (k < C::B) {
+        start = (int)((FIRST >> (4 * k)) & 15u);
+        cnt = (int)((COUNT >> (4 * k)) & 15u);
+        cls = k;
+        step = right ? -1 : 1;
+        if (right) start = n - 1 - start;
+    }
+    const double *w = tab + cls * C::NW;
+    V3 s{0.0, 0.0, 0.0};
 #pragma unroll
-            for (int k = 0; k < ELL_S; ++k) {
-                so[k] = ell.s_off[k * ns + sl];
-                sw[k] = ell.s_w[k * ns + sl];
-            }
-#pragma unroll
-            for (int k = 0; k < ELL_V; ++k) {
-                vx[k] = ell.v_off[k * 2 * ns + sl];
-                wx[k] = ell.v_w[k * 2 * ns + sl];
-                vy[k] = ell.v_off[k * 2 * ns + ns + sl];
-                wy[k] = ell.v_w[k * 2 * ns + ns + sl];
-            }
-            double a = 0.0, b = 0.0;
-#pragma unroll
-            for (int k = 0; k < ELL_S; ++k) {
-                const long long q = so[k];
-                const double u = y[g.fs + q], v = y[2 * g.fs + q];
-                const double ut = g.Qi11[q] * u + g.Qi12[q] * v;
-                const double vt = g.Qi12[q] * u + g.Qi22[q] * v;
-                const double mh = alpha * M[q], mu = alpha * M[g.fs + q], mv = alpha * M[2 * g.fs + q];
-                const double z = g.J[q] * (vt * mu - ut * mv);
-                a += sw[k] * -mh;
-                b += sw[k] * z;
-            }
-            const double dnm = g.J[o] * hxs;
-            w0 = a / dnm;
-            w1 = b / dnm;
-            w2 = 0.0;
-            w3 = 0.0;
-#pragma unroll
-            for (int k = 0; k < ELL_V; ++k) {
-                w2 += wx[k] * (-(alpha * M[g.fs + vx[k]]) / hxs);
-                w3 += wy[k] * (-(alpha * M[g.fs + vy[k]]) / hxs);
-            }
-        } else {
-            const double u = y[g.fs + o], v = y[2 * g.fs + o];
-            const double Jv = g.J[o];
-            const double ut = g.Qi11[o] * u + g.Qi12[o] * v;
-            const double vt = g.Qi12[o] * u + g.Qi22[o] * v;
-            const double mh = alpha * M[o], mu = alpha * M[g.fs + o], mv = alpha * M[2 * g.fs + o];
-            const double z = Jv * (vt * mu - ut * mv);
-            const double dnm = Jv * hxs;
-            w0 = -mh / dnm;
-            w1 = z / dnm;
-            w2 = -mu / hxs;
-            w3 = -mv / hxs;
-        }
-        box[0][py - ly][px - lx] = w0;
-        box[1][py - ly][px - lx] = w1;
-        box[2][py - ly][px - lx] = w2;
-        box[3][py - ly][px - lx] = w3;
+    for (int m = 0; m < C::NW; ++m)
+        if (m < cnt && w[m] != 0.0) s = s + w[m] * get(start + m * step);
+    return right ? V3{-s.a, -s.b, -s.c} : s;
+}
+
+// state, metric and seed of one point
+struct AdjPoint {
+    double u, v, J, q11, q12, q22, mh, mu, mv;
+};
+
+// INNER: the tile holds no closure column and its box no panel-edge point, so the box is the tile +-R.
+// A block is a chain of loads, LDS, the columns and stores, and at C192 all blocks of a launch are
+// resident at once, so that chain is the launch's time.  It is kept short: the loads of the own and the
+// halo points are issued together, the own point stays in registers and what only the output reads is
+// in flight across the barrier; the closure columns come from the table (written out, they took a branch
+// with its code per column).  C192 sbp42, stages 3 and 2: 13.6 us, 3.2 TB/s over its 24 values per point;
+// 17.3 us with the halo, the edge gathers and the output's loads one after the other and the divisions
+// on their own.
+template <int ORD, int MODE, int TX, int TY, bool INNER>
+__device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, const AdjEll &ell, int p, int x0, int y0,
+                                             double (&box)[4][AdjTile<ORD, TX, TY>::LH][AdjTile<ORD, TX, TY>::LW],
+                                             double *tab) {
+    using Tl = AdjTile<ORD, TX, TY>;
+    constexpr int R = Tl::R, NT = Tl::NT;
+    const int n = g.n, ns = 6 * g.es;
+    const int xe = INNER ? x0 + TX : (x0 + TX < n ? x0 + TX : n), ye = INNER ? y0 + TY : (y0 + TY < n ? y0 + TY : n);
+    int lx = x0 - R, hx = xe + R, ly = y0 - R, hy = ye + R;
+    if constexpr (!INNER) {
+        adj_rows<ORD, TX, TY>(x0, xe, n, lx, hx);
+        adj_rows<ORD, TX, TY>(y0, ye, n, ly, hy);
+    }
+    const double alpha = A.alpha;
+    const Rcp<double> rhxs{g.hxs, g.rhxs};
+    const long long pb = (long long)p * n * g.pitch, mb = (long long)p * g.mps;
+    const double *yu = A.y + (pb + g.fs), *yv = yu + g.fs, *Mh = A.M + pb, *Mu = Mh + g.fs, *Mv = Mu + g.fs;
+    const double *J = g.J + mb, *Q11 = g.Qi11 + mb, *Q12 = g.Qi12 + mb, *Q22 = g.Qi22 + mb;
+    auto off = [&](int i, int j) { return (__umul24((unsigned)j, (unsigned)g.pitch) + (unsigned)i) * 8u; };
+    auto load = [&](int i, int j) {
+        const unsigned o = off(i, j);
+        return AdjPoint{at_byte(yu, o), at_byte(yv, o), at_byte(J, o), at_byte(Q11, o), at_byte(Q12, o), at_byte(Q22, o),
+                        at_byte(Mh, o), at_byte(Mu, o), at_byte(Mv, o)};
+    };
+    auto on_edge = [&](int i, int j) { return !INNER && (i == 0 || j == 0 || i == n - 1 || j == n - 1); };
+    auto put = [&](int i, int j, double w0, double w1, double w2, double w3) {
+        box[0][j - ly][i - lx] = w0;
+        box[1][j - ly][i - lx] = w1;
+        box[2][j - ly][i - lx] = w2;
+        box[3][j - ly][i - lx] = w3;
+    };
+    auto put_seed = [&](int i, int j, const AdjPoint &q) {
+        const double ut = q.q11 * q.u + q.q12 * q.v;
+        const double vt = q.q12 * q.u + q.q22 * q.v;
+        const double mh = alpha * q.mh, mu = alpha * q.mu, mv = alpha * q.mv;
+        const double z = q.J * (vt * mu - ut * mv);
+        const Rcp<double> rd = rcp_of(q.J * g.hxs);
+        put(i, j, -mh / rd, z / rd, -mu / rhxs, -mv / rhxs);
     };
 
+    // the halo points: tile rows outside [x0, xe), then tile columns outside [y0, ye)
+    constexpr int HALO = INNER ? 2 * R * (TX + TY) : (R + Tl::B - 1) * (TX + TY), NH = (HALO + NT - 1) / NT;
     const int tid = threadIdx.x;
     const int gx = x0 + tid % TX, gy = y0 + tid / TX;
-    const bool own = gx < n && gy < n;
-    if (own) seed(gx, gy);
-    // halo: tile rows outside [x0, xe), then tile columns outside [y0, ye)
-    const int xl = x0 - lx, xw = xl + (hx - xe), yl = y0 - ly, ncol = xe - x0;
-    const int nxh = (ye - y0) * xw, nyh = (y0 - ly + hy - ye) * ncol;
-    for (int q = tid; q < nxh + nyh; q += Tl::NT) {
-        if (q < nxh) {
-            const int r = q / xw, k = q - r * xw;
-            seed(k < xl ? lx + k : xe + (k - xl), y0 + r);
+    const bool own = INNER || (gx < n && gy < n);
+    const int xl = x0 - lx, xw = INNER ? 2 * R : xl + (hx - xe), yl = y0 - ly, ncol = INNER ? TX : xe - x0;
+    const int nyh = (INNER ? 2 * R : yl + hy - ye) * ncol, nxh = (INNER ? TY : ye - y0) * xw;
+    auto halo = [&](int q, int &i, int &j) {
+        if (q < nyh) {
+            const int r = q / ncol;
+            i = x0 + q - r * ncol;
+            j = r < yl ? ly + r : ye + (r - yl);
         } else {
-            const int q2 = q - nxh, r = q2 / ncol, k = q2 - r * ncol;
-            seed(x0 + k, r < yl ? ly + r : ye + (r - yl));
+            const int r = (q - nyh) / xw, k = q - nyh - r * xw;
+            i = k < xl ? lx + k : xe + (k - xl);
+            j = y0 + r;
+        }
+        return q < nyh + nxh;
+    };
+    // panel-edge points of the box hold the transposed edge syncs of the seeds, gathered through the tables:
+    // wave e takes the points of panel edge e (i = 0, i = n-1, j = 0, j = n-1; corners on the first two),
+    // its table loads ahead of everything else
+    int ei = 0, ej = 0;
+    bool e_in = false;
+    int so[ELL_S], vx[ELL_V], vy[ELL_V];
+    double sw[ELL_S], wx[ELL_V], wy[ELL_V], eJ = 1.0;
+    if constexpr (!INNER) {
+        static_assert(NT >= 256 && Tl::LW <= 64 && Tl::LH <= 64, "one wave per panel edge, one lane per point");
+        const int e = tid / 64, lane = tid % 64;
+        if (e < 4) {
+            ei = e == 0 ? 0 : e == 1 ? n - 1 : lx + lane;
+            ej = e == 2 ? 0 : e == 3 ? n - 1 : ly + lane;
+            e_in = ei >= lx && ei < hx && ej >= ly && ej < hy && ((ei >= x0 && ei < xe) || (ej >= y0 && ej < ye)) &&
+                   (e < 2 || (ei != 0 && ei != n - 1));
+        }
+        if (e_in) {
+            const int sl = p * g.es + edge_slot(n, ei, ej);
+#pragma unroll
+            for (int q = 0; q < ELL_S; ++q) {
+                so[q] = ell.s_off[q * ns + sl];
+                sw[q] = ell.s_w[q * ns + sl];
+            }
+#pragma unroll
+            for (int q = 0; q < ELL_V; ++q) {
+                vx[q] = ell.v_off[q * 2 * ns + sl];
+                wx[q] = ell.v_w[q * 2 * ns + sl];
+                vy[q] = ell.v_off[q * 2 * ns + ns + sl];
+                wy[q] = ell.v_w[q * 2 * ns + ns + sl];
+            }
+            eJ = at_byte(J, off(ei, ej));
+        }
+    }
+    AdjPoint me{};
+    if (own) me = load(gx, gy);
+    AdjPoint hp[NH];
+    int hi[NH], hj[NH];
+    bool ok[NH];
+#pragma unroll
+    for (int k = 0; k < NH; ++k) {
+        ok[k] = halo(tid + k * NT, hi[k], hj[k]);
+        if (ok[k] && !on_edge(hi[k], hj[k])) hp[k] = load(hi[k], hj[k]);
+    }
+    if constexpr (!INNER) {
+        for (int c = tid; c < ColWeights<ORD>::SIZE; c += NT) tab[c] = col_weights<ORD>.w[c];
+        if (e_in) {
+            double a = 0.0, b = 0.0;
+#pragma unroll
+            for (int q = 0; q < ELL_S; ++q) {
+                const int o = so[q];
+                const double u = A.y[g.fs + o], v = A.y[2 * g.fs + o];
+                const double ut = g.Qi11[o] * u + g.Qi12[o] * v;
+                const double vt = g.Qi12[o] * u + g.Qi22[o] * v;
+                const double mh = alpha * A.M[o], mu = alpha * A.M[g.fs + o], mv = alpha * A.M[2 * g.fs + o];
+                const double z = g.J[o] * (vt * mu - ut * mv);
+                a += sw[q] * -mh;
+                b += sw[q] * z;
+            }
+            const Rcp<double> rd = rcp_of(eJ * g.hxs);
+            double w2 = 0.0, w3 = 0.0;
+#pragma unroll
+            for (int q = 0; q < ELL_V; ++q) {
+                w2 += wx[q] * (-(alpha * A.M[g.fs + vx[q]]) / rhxs);
+                w3 += wy[q] * (-(alpha * A.M[g.fs + vy[q]]) / rhxs);
+            }
+            put(ei, ej, a / rd, b / rd, w2, w3);
+        }
+    }
+    if (own && !on_edge(gx, gy)) put_seed(gx, gy, me);
+#pragma unroll
+    for (int k = 0; k < NH; ++k)
+        if (ok[k] && !on_edge(hi[k], hj[k])) put_seed(hi[k], hj[k], hp[k]);
+    // what only the output reads
+    const unsigned o = off(gx, gy);
+    double h = 0.0, f = 0.0, zeta = 0.0, L[3], ACC[3];
+    if (own) {
+        h = at_byte(A.y + pb, o);
+        f = at_byte(g.f + pb, o);
+        zeta = at_byte(A.zeta + pb, o);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if constexpr (MODE == ADJ_S4 || MODE == ADJ_S32) L[k] = at_byte((const double *)A.L + (pb + k * g.fs), o);
+            if constexpr (MODE == ADJ_S32 || MODE == ADJ_S1) ACC[k] = at_byte((const double *)A.ACC + (pb + k * g.fs), o);
         }
     }
     __syncthreads();
     if (!own) return;
 
     const int cx = gx - lx, cy = gy - ly;
-    const V3 dx = sbp_col_T<ORD>(gx, n, [&](int r) { return V3{box[0][cy][r - lx], box[1][cy][r - lx], box[2][cy][r - lx]}; });
-    const V3 dy = sbp_col_T<ORD>(gy, n, [&](int r) { return V3{box[0][r - ly][cx], box[1][r - ly][cx], box[3][r - ly][cx]}; });
-    const long long o = ((long long)p * n + gy) * g.pitch + gx;
-    const double Jv = g.J[o];
+    V3 dx, dy;
+    if constexpr (INNER) {
+        using S = Sbp<ORD>;
+        dx = dy = V3{0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < S::WIN; ++k)
+            if (S::Qin[k] != 0.0) {
+                const int x = cx + R - k, y = cy + R - k;
+                dx = dx + S::Qin[k] * V3{box[0][cy][x], box[1][cy][x], box[2][cy][x]};
+                dy = dy + S::Qin[k] * V3{box[0][y][cx], box[1][y][cx], box[3][y][cx]};
+            }
+    } else {
+        dx = tab_col_T<ORD>(tab, gx, n, [&](int r) { return V3{box[0][cy][r - lx], box[1][cy][r - lx], box[2][cy][r - lx]}; });
+        dy = tab_col_T<ORD>(tab, gy, n, [&](int r) { return V3{box[0][r - ly][cx], box[1][r - ly][cx], box[3][r - ly][cx]}; });
+    }
+    const double Jv = me.J;
     const double lFx = Jv * dx.a, lFy = Jv * dy.a, lAx = Jv * dx.b, lAy = Jv * dy.b, lK = dx.c + dy.c;
-    const double h = y[o], u = y[g.fs + o], v = y[2 * g.fs + o];
-    const double q11 = g.Qi11[o], q12 = g.Qi12[o], q22 = g.Qi22[o];
+    const double u = me.u, v = me.v;
+    const double q11 = me.q11, q12 = me.q12, q22 = me.q22;
     const double ut = q11 * u + q12 * v, vt = q12 * u + q22 * v;
-    const double qz = g.f[o] + A.zeta[o];
-    const double mu = alpha * M[g.fs + o], mv = alpha * M[2 * g.fs + o];
+    const double qz = f + zeta;
+    const double mu = alpha * me.mu, mv = alpha * me.mv;
     const double lut = h * lFx - qz * Jv * mv;
     const double lvt = h * lFy + qz * Jv * mu;
     const double gh = ut * lFx + vt * lFy + g.grav * lK;
-    const double gu = ut * lK - lAy / Jv + q11 * lut + q12 * lvt;
-    const double gv = vt * lK + lAx / Jv + q12 * lut + q22 * lvt;
+    const Rcp<double> rJ = rcp_of(Jv);
+    const double gu = ut * lK - lAy / rJ + q11 * lut + q12 * lvt;
+    const double gv = vt * lK + lAx / rJ + q12 * lut + q22 * lvt;
     const double gg[3] = {gh, gu, gv};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const long long ok = k * g.fs + o;
+        const long long fk = pb + k * g.fs;
         if constexpr (MODE == ADJ_VJP) {
-            A.out[ok] = gg[k];
+            at_byte(A.out + fk, o) = gg[k];
         } else if constexpr (MODE == ADJ_S4) {
-            const double l = A.L[ok];
-            A.MU[ok] = A.a * l + A.b * gg[k];
-            A.ACC[ok] = l + gg[k];
+            at_byte(A.MU + fk, o) = A.a * L[k] + A.b * gg[k];
+            at_byte(A.ACC + fk, o) = L[k] + gg[k];
         } else if constexpr (MODE == ADJ_S32) {
-            A.MU[ok] = A.a * A.L[ok] + A.b * gg[k];
-            A.ACC[ok] = A.ACC[ok] + gg[k];
+            at_byte(A.MU + fk, o) = A.a * L[k] + A.b * gg[k];
+            at_byte(A.ACC + fk, o) = ACC[k] + gg[k];
         } else {
-            A.L[ok] = A.ACC[ok] + gg[k];
+            at_byte(A.L + fk, o) = ACC[k] + gg[k];
         }
     }
+}
+
+template <int ORD, int MODE, int TX, int TY>
+__global__ void __launch_bounds__(TX * TY) adj_tile(AdjGeo g, AdjArgs A, AdjEll ell) {
+    using Tl = AdjTile<ORD, TX, TY>;
+    __shared__ double box[4][Tl::LH][Tl::LW];
+    __shared__ double tab[ColWeights<ORD>::SIZE];
+    const int n = g.n, ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
+    // row strips outermost, then panels: an XCD's contiguous range is a band of all six panels, which share
+    // the metric
+    const int t = xcd_tile(blockIdx.x, 6 * ntx * nty);
+    const int strip = t / (6 * ntx), rem = t - strip * 6 * ntx, p = rem / ntx;
+    const int x0 = (rem - p * ntx) * TX, y0 = strip * TY;
+    constexpr int M = Tl::B > Tl::R ? Tl::B : Tl::R + 1;
+    if (x0 >= M && y0 >= M && x0 + TX <= n - M && y0 + TY <= n - M)
+        adj_tile_run<ORD, MODE, TX, TY, true>(g, A, ell, p, x0, y0, box, tab);
+    else
+        adj_tile_run<ORD, MODE, TX, TY, false>(g, A, ell, p, x0, y0, box, tab);
 }
 
 }  // namespace swm
@@ -581,7 +738,8 @@ swm::AdjGeo adj_geo(const swm_ctx *c) {
     swm::AdjGeo g;
     g.J = c->J64; g.Qi11 = c->Qi64[0]; g.Qi12 = c->Qi64[1]; g.Qi22 = c->Qi64[2]; g.f = c->f64;
     g.n = c->n; g.pitch = c->pitch; g.es = 4 * c->N; g.fs = c->fs;
-    g.hxs = c->hx * c->scale; g.grav = c->grav;
+    g.hxs = c->hx * c->scale; g.rhxs = 1.0 / g.hxs; g.grav = c->grav;
+    g.mps = c->metric_shared ? 0 : (long long)c->n * c->pitch;
     return g;
 }
 
