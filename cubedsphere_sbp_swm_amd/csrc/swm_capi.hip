@@ -145,8 +145,7 @@ int parse_names(swm_ctx *c, const char *div, const char *grad, const char *curl,
 }
 
 void drop_graphs(swm_ctx *c) {
-    if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
-    if (c->graph_multi) { (void)hipGraphExecDestroy(c->graph_multi); c->graph_multi = nullptr; }
+    c->graphs.drop();
     c->graph_state = nullptr;
 }
 
@@ -403,29 +402,9 @@ extern "C" int swm_rk4_steps(swm_ctx *c, void *state, double dt, int nsteps) {
     if (nsteps < 0) return fail(SWM_EARG, "nsteps must be >= 0");
     if (nsteps == 0) return SWM_OK;
     if (c->graph_state != state || c->graph_dt != dt) drop_graphs(c);
-    // whole runs of RK4_GRAPH_STEPS steps replay the multi-step graph (4 * RK4_GRAPH_STEPS
-    // kernel nodes, one graph launch), the rest the one-step graph
-    const int nmulti = nsteps / RK4_GRAPH_STEPS, nsingle = nsteps - nmulti * RK4_GRAPH_STEPS;
-    for (int which = 0; which < 2; ++which) {
-        hipGraphExec_t &ge = which == 0 ? c->graph : c->graph_multi;
-        const int per = which == 0 ? 1 : RK4_GRAPH_STEPS;
-        if (ge || (which == 0 ? nsingle : nmulti) == 0) continue;
-        hipGraph_t g = nullptr;
-        HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int rc = SWM_OK;
-        for (int k = 0; k < per && !rc; ++k) rc = enqueue_rk4_step(c, state, dt);
-        hipError_t e = hipStreamEndCapture(c->stream, &g);
-        if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-        if (e != hipSuccess) return fail(SWM_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
-        e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e != hipSuccess) { ge = nullptr; return fail(SWM_EHIP, std::string("graph instantiate: ") + hipGetErrorString(e)); }
-        c->graph_state = state;
-        c->graph_dt = dt;
-    }
-    for (int s = 0; s < nmulti; ++s) HIP_TRY(hipGraphLaunch(c->graph_multi, c->stream));
-    for (int s = 0; s < nsingle; ++s) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
-    return SWM_OK;
+    c->graph_state = state;
+    c->graph_dt = dt;
+    return c->graphs.run(c->stream, nsteps, [&] { return enqueue_rk4_step(c, state, dt); });
 }
 
 extern "C" int swm_ctx_set_tile_shape(swm_ctx *c, int tile_cols, int tile_rows, int metric_on_the_fly) {

@@ -29,7 +29,7 @@ struct swm_cctx {
     // partial sums (10 per block) and the 6 results
     double *qw = nullptr, *dpart = nullptr;
     long long dblocks = 0;
-    hipGraphExec_t graph = nullptr, graph_multi = nullptr;
+    StepGraphs graphs;  // captured RK4 steps of (graph_state, graph_dt)
     void *graph_state = nullptr;
     double graph_dt = 0.0;
     // ECS halos of the C grid (the vector halo and the ECS_O halo of gradient_c2_ecs and

@@ -985,8 +985,7 @@ int c_enqueue_rk4_step(swm_cctx *c, double *state, double dt) {
 }
 
 void c_drop_graphs(swm_cctx *c) {
-    if (c->graph) { (void)hipGraphExecDestroy(c->graph); c->graph = nullptr; }
-    if (c->graph_multi) { (void)hipGraphExecDestroy(c->graph_multi); c->graph_multi = nullptr; }
+    c->graphs.drop();
     c->graph_state = nullptr;
 }
 
@@ -1238,27 +1237,9 @@ extern "C" int swm_c_rk4_steps(swm_cctx *c, void *state, double dt, int nsteps) 
     if (nsteps < 0) return fail(SWM_EARG, "nsteps must be >= 0");
     if (nsteps == 0) return SWM_OK;
     if (c->graph_state != state || c->graph_dt != dt) c_drop_graphs(c);
-    const int nmulti = nsteps / RK4_GRAPH_STEPS, nsingle = nsteps - nmulti * RK4_GRAPH_STEPS;
-    for (int which = 0; which < 2; ++which) {
-        hipGraphExec_t &ge = which == 0 ? c->graph : c->graph_multi;
-        const int per = which == 0 ? 1 : RK4_GRAPH_STEPS;
-        if (ge || (which == 0 ? nsingle : nmulti) == 0) continue;
-        hipGraph_t gr = nullptr;
-        HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int rc = SWM_OK;
-        for (int k = 0; k < per && !rc; ++k) rc = c_enqueue_rk4_step(c, (double *)state, dt);
-        hipError_t e = hipStreamEndCapture(c->stream, &gr);
-        if (rc) { if (gr) (void)hipGraphDestroy(gr); return rc; }
-        if (e != hipSuccess) return fail(SWM_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
-        e = hipGraphInstantiate(&ge, gr, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(gr);
-        if (e != hipSuccess) { ge = nullptr; return fail(SWM_EHIP, std::string("graph instantiate: ") + hipGetErrorString(e)); }
-        c->graph_state = state;
-        c->graph_dt = dt;
-    }
-    for (int s = 0; s < nmulti; ++s) HIP_TRY(hipGraphLaunch(c->graph_multi, c->stream));
-    for (int s = 0; s < nsingle; ++s) HIP_TRY(hipGraphLaunch(c->graph, c->stream));
-    return SWM_OK;
+    c->graph_state = state;
+    c->graph_dt = dt;
+    return c->graphs.run(c->stream, nsteps, [&] { return c_enqueue_rk4_step(c, (double *)state, dt); });
 }
 
 extern "C" int swm_c_diagnostics(swm_cctx *c, const void *state, double out[7]) {

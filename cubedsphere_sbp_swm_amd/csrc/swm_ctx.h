@@ -12,8 +12,6 @@
 
 namespace swm_host {
 
-constexpr int RK4_GRAPH_STEPS = 50;  // steps per replay of the multi-step graph
-
 // sets the message of swm_last_error on this thread and returns `code`
 int fail(int code, const std::string &msg);
 
@@ -22,6 +20,67 @@ int fail(int code, const std::string &msg);
         hipError_t e_ = (expr);                                                              \
         if (e_ != hipSuccess) return fail(SWM_EHIP, std::string(#expr ": ") + hipGetErrorString(e_)); \
     } while (0)
+
+// Time steps of one state: runs of them through graphs of 4, 8, ... 64 steps, each made when a run first needs
+// it; the up to three steps left over, and the first run of a state, by plain launches.  A graph launch leaves
+// about 10 us between two graphs where kernels follow each other in 1 to 2, so a graph of one step is slower
+// than its four launches (C384 sbp42 FP64, 20 steps: 1797 us in graphs of one step, 1697 us by launches, 1724 us
+// in graphs of 16 and 4; C90 C grid 848, 809 and 809).  Long graphs pay where the host is what launches wait
+// for (C32 sbp21, 12 steps with three contexts at work: 192, 148 and 113 us).  Making them costs about 7 us a step,
+// which a first run that stays below FIRST steps does not earn back (C90 C grid, 10 steps: 1574 us with
+// the graphs made in the run, 850 us by launches).
+struct StepGraphs {
+    static constexpr int MIN = 4, KINDS = 5, FIRST = 128;
+    hipGraphExec_t exec[KINDS] = {};
+    bool seen = false;  // a run of the state has been made
+    void drop() {
+        for (hipGraphExec_t &g : exec) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
+        seen = false;
+    }
+    // nsteps of `step`, which enqueues one step on `stream`
+    template <class Step>
+    int run(hipStream_t stream, int nsteps, const Step &step) {
+        int rc;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(stream, &cap));
+        if (cap != hipStreamCaptureStatusNone) return fail(SWM_EHIP, "time steps cannot be captured: they run graphs of their own");
+        if (!seen) {
+            // also ahead of a long run: its first step sets up what a capture could not
+            for (int q = nsteps <= FIRST ? nsteps : 1; q > 0; --q, --nsteps)
+                if ((rc = step())) return rc;
+            seen = true;
+        }
+        for (int k = KINDS - 1; k >= 0; --k) {
+            const int per = MIN << k, times = nsteps / per;
+            nsteps -= times * per;
+            if (times && !exec[k] && (rc = make(stream, per, exec[k], step))) return rc;
+            for (int q = 0; q < times; ++q) HIP_TRY(hipGraphLaunch(exec[k], stream));
+        }
+        for (; nsteps > 0; --nsteps)
+            if ((rc = step())) return rc;
+        return SWM_OK;
+    }
+
+  private:
+    template <class Step>
+    static int make(hipStream_t stream, int steps, hipGraphExec_t &out, const Step &step) {
+        hipGraph_t g = nullptr;
+        HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        int rc = SWM_OK;
+        for (int q = 0; q < steps && !rc; ++q) rc = step();
+        hipError_t e = hipStreamEndCapture(stream, &g);
+        if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
+        if (e != hipSuccess) return fail(SWM_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
+        e = hipGraphInstantiate(&out, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        if (e == hipSuccess) return SWM_OK;
+        out = nullptr;
+        return fail(SWM_EHIP, std::string("graph instantiate: ") + hipGetErrorString(e));
+    }
+};
 
 struct AdjWork;  // adjoint work space (swm_adjoint.hip), created on first use
 void free_adj_work(AdjWork *w);
@@ -60,8 +119,7 @@ struct swm_ctx {
     void *yA = nullptr, *yB = nullptr, *acc = nullptr, *curl = nullptr;
     double *red = nullptr;
     int red_blocks = 0;
-    // captured RK4 steps: one step, and RK4_GRAPH_STEPS steps in a row (fewer graph launches)
-    hipGraphExec_t graph = nullptr, graph_multi = nullptr;
+    StepGraphs graphs;  // captured RK4 steps of (graph_state, graph_dt)
     void *graph_state = nullptr;
     double graph_dt = 0.0;
     std::vector<int> host_nbr;

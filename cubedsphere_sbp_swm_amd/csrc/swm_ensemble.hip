@@ -1,9 +1,8 @@
 // Batched ensemble form (included into swm_capi.hip): cubes of different resolutions, each
 // with its own context (geometry, work buffers) and time step, advanced together.  One RK4
 // step of the whole ensemble = 4 stage launches (ens_stage_kernel), each walking the
-// concatenated tile list of all members; the launches of one step and of RK4_GRAPH_STEPS steps
-// are captured once in hipGraphs and replayed.  The tile shape, the on-the-fly metric and the
-// grid are chosen by swm_ens_autotune, which times the stage-2 launch of the whole ensemble
+// concatenated tile list of all members; repeated runs of steps replay captured hipGraphs
+// (StepGraphs).  The tile shape, the on-the-fly metric and the grid are chosen by swm_ens_autotune, which times the stage-2 launch of the whole ensemble
 // (persistent grids of 1 or 4 blocks per resident slot, or one block per task).
 
 struct swm_ens {
@@ -20,15 +19,14 @@ struct swm_ens {
     std::vector<double> dt;
     std::vector<unsigned> hs_gen;  // the members' orography generations the tables were built with
     bool tables_ok = false;
-    hipGraphExec_t graph = nullptr, graph_multi = nullptr;  // one step; RK4_GRAPH_STEPS steps
+    StepGraphs graphs;  // captured steps
     hipEvent_t order_ev = nullptr;  // orders the members' own streams around ensemble steps
 };
 
 namespace {
 
 void ens_drop_graph(swm_ens *e) {
-    if (e->graph) { (void)hipGraphExecDestroy(e->graph); e->graph = nullptr; }
-    if (e->graph_multi) { (void)hipGraphExecDestroy(e->graph_multi); e->graph_multi = nullptr; }
+    e->graphs.drop();
 }
 
 void free_ens(swm_ens *e) {
@@ -275,30 +273,7 @@ extern "C" int swm_ens_rk4_steps(swm_ens *e, const double *dt, int nsteps) {
     int rc0;
     for (swm_ctx *c : e->m)
         if ((rc0 = ens_order(e, c->stream, e->stream))) return rc0;
-    if (!e->graph && !e->graph_multi) {
-        int rc = ens_step(e);  // eager first step: sets up the launch configuration
-        if (rc) return rc;
-        --nsteps;
-    }
-    // whole runs of RK4_GRAPH_STEPS steps replay the multi-step graph, the rest the one-step graph
-    const int nmulti = nsteps / RK4_GRAPH_STEPS, nsingle = nsteps - nmulti * RK4_GRAPH_STEPS;
-    for (int which = 0; which < 2; ++which) {
-        hipGraphExec_t &ge = which == 0 ? e->graph : e->graph_multi;
-        const int per = which == 0 ? 1 : RK4_GRAPH_STEPS;
-        if (ge || (which == 0 ? nsingle : nmulti) == 0) continue;
-        hipGraph_t g = nullptr;
-        HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-        int rc = SWM_OK;
-        for (int k = 0; k < per && !rc; ++k) rc = ens_step(e);
-        hipError_t err = hipStreamEndCapture(e->stream, &g);
-        if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-        if (err != hipSuccess) return fail(SWM_EHIP, std::string("graph capture: ") + hipGetErrorString(err));
-        err = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (err != hipSuccess) { ge = nullptr; return fail(SWM_EHIP, std::string("graph instantiate: ") + hipGetErrorString(err)); }
-    }
-    for (int s = 0; s < nmulti; ++s) HIP_TRY(hipGraphLaunch(e->graph_multi, e->stream));
-    for (int s = 0; s < nsingle; ++s) HIP_TRY(hipGraphLaunch(e->graph, e->stream));
+    if ((rc0 = e->graphs.run(e->stream, nsteps, [&] { return ens_step(e); }))) return rc0;
     // later work on a member's own stream (downloads, diagnostics) follows the ensemble steps
     for (swm_ctx *c : e->m)
         if ((rc0 = ens_order(e, e->stream, c->stream))) return rc0;
