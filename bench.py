@@ -22,10 +22,17 @@ sys.path.insert(0, ROOT)
 
 METRIC = "cell-steps/s at C384 sbp42 vs HBM roofline; adjoint/forward time ratio"
 HBM_PEAK_GBS = 8000.0
-# Algorithmic traffic per Ah point of one RK stage-2/3 launch: read y(3) + metric J, Qi11,
-# Qi12, Qi22, f (5) + v0(3) + acc(3), write y(3) + acc(3) = 20 values.
+# Algorithmic traffic per Ah point of the RK stage launch with the most of it, metric J, Qi11, Qi12, Qi22,
+# f (5) included.  By slopes (large grids) stage 3: read v0(3) + k2(3) + k1(3), write y(3) + acc(3); by
+# states stages 2 and 3: read y(3) + v0(3) + acc(3), write y(3) + acc(3): 20 values either way.
 STAGE23_VALUES = 20
-STEP_VALUES = 71  # per point per RK4 step (14 + 20 + 20 + 17)
+STEP_VALUES = 68         # per point per RK4 step by states (14 + 20 + 20 + 14)
+STEP_VALUES_SLOPES = 59  # by slopes (11 + 14 + 20 + 14)
+
+
+def by_slopes(N, order, prec):
+    """Whether the RK4 step runs by slopes: its four states take more than 36 MB (sbp63, FP32: 64 MB)."""
+    return 12 * 6 * (N + 1) ** 2 * (prec // 8) > (64e6 if order == 63 or prec == 32 else 36e6)
 
 
 def parse():
@@ -80,7 +87,7 @@ def parse():
 
 
 def profiled_traffic(N, order, prec, tiling):
-    """HBM bytes per stage-2/3 launch measured with rocprofv3 FETCH_SIZE / WRITE_SIZE (copy-kernel
+    """HBM bytes per launch of the stage kernel with the most traffic, measured with rocprofv3 FETCH_SIZE / WRITE_SIZE (copy-kernel
     calibrated) for this workload and tiling, from the committed profile summary; None if absent."""
     import re
     path = os.path.join(ROOT, "profiles", f"stage23_c{N}_sbp{order}_f{prec}.md")
@@ -145,7 +152,7 @@ def fp32_form(args, stream):
                            "rel_linf": float(np.max(np.abs(dh)) / np.max(np.abs(hp)))}
     drift = {p: (res[p]["d1"]["mass"] - res[p]["d0"]["mass"]) / res[p]["d0"]["mass"] for p in (32, 64)}
     rate = {p: cells * steps / res[p]["secs"] for p in (32, 64)}
-    step_gbs32 = STEP_VALUES * 4 * points / (res[32]["secs"] / steps) / 1e9
+    step_gbs32 = (STEP_VALUES_SLOPES if by_slopes(N, 42, 32) else STEP_VALUES) * 4 * points / (res[32]["secs"] / steps) / 1e9
     return {"workload": f"C{N} sbp42 RK4 dt={dt:g}s x {steps} steps, degree <= {args.fp32_lmax}",
             "fp32_cell_steps_per_s": rate[32], "fp64_cell_steps_per_s": rate[64],
             "speedup_vs_fp64": rate[32] / rate[64],
@@ -634,7 +641,8 @@ def main():
     eb = op.elem_bytes
     stage_bytes = STAGE23_VALUES * eb * points
     achieved = stage_bytes / (k_us * 1e-6) / 1e9
-    step_bytes = STEP_VALUES * eb * points
+    slopes = by_slopes(N, order, args.precision)
+    step_bytes = (STEP_VALUES_SLOPES if slopes else STEP_VALUES) * eb * points
     step_gbs = step_bytes / ((ms / 1e3) / args.steps) / 1e9
 
     forms = {}
@@ -676,9 +684,11 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": profiled_traffic(N, order, args.precision, tiling),
-                     "kernel": "stage_kernel<%d, %s, MODE_STAGE23, %d, %d, %s> (RK stages 2 and 3)" % (
-                         order, "double" if args.precision == 64 else "float", tiling["tile_cols"],
-                         tiling["tile_rows"], str(tiling["metric_on_the_fly"]).lower()),
+                     "kernel": "stage_kernel<%d, %s, %s, %d, %d, %s> (RK %s)" % (
+                         order, "double" if args.precision == 64 else "float",
+                         "MODE_SLOPE3" if slopes else "MODE_STAGE23", tiling["tile_cols"],
+                         tiling["tile_rows"], str(tiling["metric_on_the_fly"]).lower(),
+                         "stage 3" if slopes else "stages 2 and 3"),
                      "kernel_avg_us": k_us, "algorithmic_bytes_per_launch": stage_bytes,
                      "step_effective_GBs": step_gbs, "step_frac": step_gbs / HBM_PEAK_GBS,
                      "measured_copy": copy},

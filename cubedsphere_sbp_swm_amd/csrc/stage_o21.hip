@@ -40,8 +40,16 @@ __device__ __forceinline__ void neighbour_grad21(const DevGeo<T> &g, const EdgeD
     gy = (ed.nu_x ? tK : nK) / g.hxs;
 }
 
-template <bool OTF, typename T>
-__device__ __forceinline__ Pt21<T> point21(const DevGeo<T> &g, const T *y, const T *hs, int p, int i, int j) {
+// input of the stage at a point
+template <int MODE, typename T>
+__device__ __forceinline__ T state21(const StageArgs<T> &a, long long id) {
+    if constexpr (mode_slope(MODE)) return a.y[id] + a.ck * a.kin[id];
+    else return a.y[id];
+}
+
+template <int MODE, bool OTF, typename T>
+__device__ __forceinline__ Pt21<T> point21(const DevGeo<T> &g, const StageArgs<T> &a, int p, int i, int j) {
+    const T *hs = a.hs;
     const long long id = pidx(g, p, i, j);
     T J, q11, q12, q22;
     if constexpr (OTF) {
@@ -50,7 +58,7 @@ __device__ __forceinline__ Pt21<T> point21(const DevGeo<T> &g, const T *y, const
     } else {
         J = g.J[id]; q11 = g.Qi11[id]; q12 = g.Qi12[id]; q22 = g.Qi22[id];
     }
-    const T h = y[id], u = y[id + g.fs], v = y[id + 2 * g.fs];
+    const T h = state21<MODE>(a, id), u = state21<MODE>(a, id + g.fs), v = state21<MODE>(a, id + 2 * g.fs);
     const T ut = q11 * u + q12 * v;
     const T vt = q12 * u + q22 * v;
     Pt21<T> r;
@@ -75,7 +83,6 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
     const int rem = tile - p * ntx * nty;
     const int ty0 = (rem / ntx) * TY, tx0 = (rem % ntx) * TX;
     const int tid = threadIdx.x;
-    const T *y = a.y;
 
     // in-panel cross region (1-point halo)
     for (int c = tid; c < (TY + 2) * (TX + 2); c += NT) {
@@ -83,7 +90,7 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
         const bool row = ly >= 1 && ly <= TY, col = lx >= 1 && lx <= TX;
         const int i = tx0 - 1 + lx, j = ty0 - 1 + ly;
         if (!(row || col) || i < 0 || i >= n || j < 0 || j >= n) continue;
-        const Pt21<T> q = point21<OTF>(g, y, a.hs, p, i, j);
+        const Pt21<T> q = point21<MODE, OTF>(g, a, p, i, j);
         sm.K[ly][lx] = q.K; sm.Ud[ly][lx] = q.Ud; sm.Vd[ly][lx] = q.Vd;
         sm.Uc[ly][lx] = q.Uc; sm.Vc[ly][lx] = q.Vc; sm.J[ly][lx] = q.J;
     }
@@ -108,7 +115,7 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
             const int *ei = g.einfo + (p * 4 + e) * 8;
             const int nidx = ei[2] == 0 ? d : n - 1 - d, tidx = ei[3] + ei[4] * kk;
             const int qi = ei[1] ? nidx : tidx, qj = ei[1] ? tidx : nidx;
-            const Pt21<T> q = point21<OTF>(g, y, a.hs, ei[0], qi, qj);
+            const Pt21<T> q = point21<MODE, OTF>(g, a, ei[0], qi, qj);
             T *dst = slot < 2 ? sm.gx[slot][d][idx] : sm.gy[d][idx];
             dst[0] = q.K;
             map_vec(ei[5], q.Ud, q.Vd, dst[1], dst[2]);
@@ -258,7 +265,7 @@ __global__ void __launch_bounds__(TX * TY) stage21_kernel(DevGeo<T> g, StageArgs
     } else {
         q11 = g.Qi11[id]; q12 = g.Qi12[id]; q22 = g.Qi22[id];
     }
-    const T h = a.y[id], u = a.y[id + g.fs], v = a.y[id + 2 * g.fs];
+    const T h = state21<MODE>(a, id), u = state21<MODE>(a, id + g.fs), v = state21<MODE>(a, id + 2 * g.fs);
     const unsigned off = point_off(g, i, j);
     finish_point<T, MODE>(g, a, p, off, h, u, v, h * (q11 * u + q12 * v), h * (q12 * u + q22 * v), sm.J[ly][lx], gx, gy,
                           dv, cu, prefetch_point<T, MODE>(g, a, p, off));
@@ -274,6 +281,8 @@ hipError_t launch21(int mode, const DevGeo<T> &g, const StageArgs<T> &a, hipStre
     case MODE_STAGE1: hipLaunchKernelGGL((stage21_kernel<T, MODE_STAGE1, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_STAGE23: hipLaunchKernelGGL((stage21_kernel<T, MODE_STAGE23, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_STAGE4: hipLaunchKernelGGL((stage21_kernel<T, MODE_STAGE4, TX, TY, OTF>), grid, block, 0, s, g, a); break;
+    case MODE_SLOPE2: hipLaunchKernelGGL((stage21_kernel<T, MODE_SLOPE2, TX, TY, OTF>), grid, block, 0, s, g, a); break;
+    case MODE_SLOPE3: hipLaunchKernelGGL((stage21_kernel<T, MODE_SLOPE3, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_CURL: hipLaunchKernelGGL((stage21_kernel<T, MODE_CURL, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     default: return hipErrorInvalidValue;
     }

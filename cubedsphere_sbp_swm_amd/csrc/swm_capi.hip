@@ -31,7 +31,7 @@ int swm_host::fail(int code, const std::string &msg) {
 }
 
 int swm_host::run_stage(swm_ctx *c, int mode, const void *y, void *out, const void *v0, void *acc, double cy,
-                        double cacc, void *zeta) {
+                        double cacc, void *zeta, const void *kin, double ck, double ck1) {
     swm::StageLaunch r{};
     r.prec = c->prec;
     r.mode = mode;
@@ -42,11 +42,11 @@ int swm_host::run_stage(swm_ctx *c, int mode, const void *y, void *out, const vo
     if (c->prec == 64) {
         r.gd = make_geo<double>(c);
         r.ad = {(const double *)y, (double *)out, (const double *)v0, (double *)acc, (const double *)c->hs, cy, cacc,
-                (double *)zeta};
+                (double *)zeta, (const double *)kin, ck, ck1};
     } else {
         r.gf = make_geo<float>(c);
         r.af = {(const float *)y, (float *)out, (const float *)v0, (float *)acc, (const float *)c->hs, (float)cy,
-                (float)cacc, (float *)zeta};
+                (float)cacc, (float *)zeta, (const float *)kin, (float)ck, (float)ck1};
     }
     hipError_t e;
     switch (c->grad_order) {
@@ -62,15 +62,36 @@ int swm_host::run_stage(swm_ctx *c, int mode, const void *y, void *out, const vo
 
 namespace {
 
+// Whether a step's first stages write slopes only (StageMode).  Its state and three work states then move 39
+// instead of 48 fields a step through memory, against three more loads per point and its halo in stages 2
+// and 3.  It pays where the four states no longer stay near the chip; below, a stage is a chain of loads.
+// Us per step, states / slopes, one context alone and three at work:
+//   sbp42 FP64  C192 (21 MB) 37.6 / 39.2, 23.6 / 23.2   C256 (38) 48.2 / 47.6, 35.6 / 34.2
+//               C320 (59) 64.4 / 61.8, 51.3 / 48.8      C384 (85) 83.6 / 80.7, 91.8 / 77.8
+//   sbp63 FP64  C320 (59) 75.1 / 77.2, 58.6 / 59.5      C384 (85) 97.7 / 99.4, 105.1 / 95.4
+//   sbp42 FP32  C384 (43) 58.4 / 59.0, 45.9 / 46.0      C768 (170) 164.2 / 166.5, 233.2 / 224.6
+// The wider halo of sbp63 and the cheaper arithmetic of FP32 put their line higher.
+bool rk4_by_slopes(const swm_ctx *c) {
+    const size_t mb = (c->grad_order == 63 || c->prec == 32 ? 64 : 36);
+    return 12 * c->field_bytes() > mb * 1000000;
+}
+
 // one RK4 step = 4 fused stage launches (rk4_mod.f90:28-40); `out` = state, or another buffer
 // for a timing run that leaves the state unchanged
 int enqueue_rk4_step(swm_ctx *c, void *state, double dt, void *out = nullptr) {
     const double c1 = 0.5 * dt, c2 = dt / 6.0, c3 = dt / 3.0;
     int rc;
-    if ((rc = run_stage(c, swm::MODE_STAGE1, state, c->yA, nullptr, c->acc, c1, c2))) return rc;
-    if ((rc = run_stage(c, swm::MODE_STAGE23, c->yA, c->yB, state, c->acc, c1, c3))) return rc;
-    if ((rc = run_stage(c, swm::MODE_STAGE23, c->yB, c->yA, state, c->acc, dt, c3))) return rc;
-    if ((rc = run_stage(c, swm::MODE_STAGE4, c->yA, out ? out : state, nullptr, c->acc, c2, 0.0))) return rc;
+    if (!rk4_by_slopes(c)) {
+        if ((rc = run_stage(c, swm::MODE_STAGE1, state, c->yA, nullptr, c->yC, c1, c2))) return rc;
+        if ((rc = run_stage(c, swm::MODE_STAGE23, c->yA, c->yB, state, c->yC, c1, c3))) return rc;
+        if ((rc = run_stage(c, swm::MODE_STAGE23, c->yB, c->yA, state, c->yC, dt, c3))) return rc;
+        return run_stage(c, swm::MODE_STAGE4, c->yA, out ? out : state, nullptr, c->yC, c2, 0.0);
+    }
+    // k1 in yA (the sum of the slopes from stage 3 on), k2 in yB, the last stage's input in yC
+    if ((rc = run_stage(c, swm::MODE_RHS, state, c->yA, nullptr, nullptr, 0.0, 0.0))) return rc;
+    if ((rc = run_stage(c, swm::MODE_SLOPE2, state, c->yB, nullptr, nullptr, 0.0, 0.0, nullptr, c->yA, c1))) return rc;
+    if ((rc = run_stage(c, swm::MODE_SLOPE3, state, c->yC, nullptr, c->yA, dt, c3, nullptr, c->yB, c1, c2))) return rc;
+    if ((rc = run_stage(c, swm::MODE_STAGE4, c->yC, out ? out : state, nullptr, c->yA, c2, 0.0))) return rc;
     return SWM_OK;
 }
 
@@ -153,7 +174,7 @@ void free_ctx(swm_ctx *c) {
     if (!c) return;
     drop_graphs(c);
     void *ptrs[] = {c->J, c->Qi11, c->Qi12, c->Qi22, c->f, c->q[0], c->q[1], c->q[2], c->q[3], c->nbr, c->einfo, c->tanA, c->hs,
-                    c->J64, c->Qi64[0], c->Qi64[1], c->Qi64[2], c->f64, c->A64, c->hs64, c->yA, c->yB, c->acc,
+                    c->J64, c->Qi64[0], c->Qi64[1], c->Qi64[2], c->f64, c->A64, c->hs64, c->yA, c->yB, c->yC,
                     c->curl, c->red, c->ecs_w, c->ecs_ind, c->ecs_src, c->ecs_o_w, c->ecs_o_ind, c->ecs_o_edge,
                     c->ecs_tm};
     for (void *p : ptrs)
@@ -272,12 +293,12 @@ extern "C" int swm_ctx_create(swm_ctx **out, int N, const char *div, const char 
         hipMemcpy(c->nbr, c->host_nbr.data(), c->host_nbr.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(SWM_EHIP, "neighbour table upload failed"));
     const size_t sb = 3 * c->field_bytes();
-    if (hipMalloc(&c->yA, sb) != hipSuccess || hipMalloc(&c->yB, sb) != hipSuccess || hipMalloc(&c->acc, sb) != hipSuccess ||
+    if (hipMalloc(&c->yA, sb) != hipSuccess || hipMalloc(&c->yB, sb) != hipSuccess || hipMalloc(&c->yC, sb) != hipSuccess ||
         hipMalloc(&c->curl, c->field_bytes()) != hipSuccess)
         return bail(fail(SWM_EHIP, "work buffer allocation failed"));
     // zero the padding columns once so that every buffer holds defined values
     if (hipMemset(c->yA, 0, sb) != hipSuccess || hipMemset(c->yB, 0, sb) != hipSuccess ||
-        hipMemset(c->acc, 0, sb) != hipSuccess || hipMemset(c->curl, 0, c->field_bytes()) != hipSuccess)
+        hipMemset(c->yC, 0, sb) != hipSuccess || hipMemset(c->curl, 0, c->field_bytes()) != hipSuccess)
         return bail(fail(SWM_EHIP, "work buffer clear failed"));
     c->red_blocks = 1024;
     if (hipMalloc((void **)&c->red, sizeof(double) * 16 * (c->red_blocks + 1)) != hipSuccess)
@@ -404,7 +425,7 @@ extern "C" int swm_rk4_steps(swm_ctx *c, void *state, double dt, int nsteps) {
     if (c->graph_state != state || c->graph_dt != dt) drop_graphs(c);
     c->graph_state = state;
     c->graph_dt = dt;
-    return c->graphs.run(c->stream, nsteps, [&] { return enqueue_rk4_step(c, state, dt); });
+    return c->graphs.run(c->stream, c->fs, nsteps, [&] { return enqueue_rk4_step(c, state, dt); });
 }
 
 extern "C" int swm_ctx_set_tile_shape(swm_ctx *c, int tile_cols, int tile_rows, int metric_on_the_fly) {
@@ -492,18 +513,20 @@ extern "C" int swm_ctx_autotune(swm_ctx *c, void *state, int reps, double *best_
 }
 
 // Measurement helper: `reps` back-to-back launches of one fused stage kernel on the context
-// stream (stage 1, 2 (= 2 and 3) or 4) with the buffers the RK4 step gives it: stage 1 reads
-// `state` and writes yA, acc; stage 2 reads yA, v0 = state, acc and writes yB, acc; stage 4
-// reads yA, acc and writes yB (in place of the state).  yA starts as a copy of `state`.
+// stream (stage 1, 2 (the one with the most traffic, stage 3 of a step by slopes, else stages 2 and 3) or 4) with
+// buffers as the RK4 step's: stage 1 reads `state`; stage 2 reads `state`, yA and yC; stage 4 reads yC and yA;
+// they write work buffers only.  yA starts as a copy of `state`.
 extern "C" int swm_bench_stage(swm_ctx *c, void *state, int stage_id, int reps) {
     if (!c || !state || reps < 0) return fail(SWM_EARG, "bad argument");
     if (stage_id != 1 && stage_id != 2 && stage_id != 4) return fail(SWM_EARG, "stage_id must be 1, 2 or 4");
     if (stage_id != 1) HIP_TRY(hipMemcpyAsync(c->yA, state, 3 * c->field_bytes(), hipMemcpyDeviceToDevice, c->stream));
     for (int r = 0; r < reps; ++r) {
         int rc;
-        if (stage_id == 1) rc = run_stage(c, swm::MODE_STAGE1, state, c->yA, nullptr, c->acc, 1.0, 1.0);
-        else if (stage_id == 2) rc = run_stage(c, swm::MODE_STAGE23, c->yA, c->yB, state, c->acc, 1.0, 0.0);
-        else rc = run_stage(c, swm::MODE_STAGE4, c->yA, c->yB, nullptr, c->acc, 1.0, 0.0);
+        if (stage_id == 1 && !rk4_by_slopes(c)) rc = run_stage(c, swm::MODE_STAGE1, state, c->yA, nullptr, c->yC, 1.0, 1.0);
+        else if (stage_id == 1) rc = run_stage(c, swm::MODE_RHS, state, c->yA, nullptr, nullptr, 0.0, 0.0);
+        else if (stage_id == 2 && !rk4_by_slopes(c)) rc = run_stage(c, swm::MODE_STAGE23, c->yA, c->yB, state, c->yC, 1.0, 0.0);
+        else if (stage_id == 2) rc = run_stage(c, swm::MODE_SLOPE3, state, c->yB, nullptr, c->yC, 1.0, 0.0, nullptr, c->yA, 0.0, 0.0);
+        else rc = run_stage(c, swm::MODE_STAGE4, c->yA, c->yB, nullptr, c->yC, 1.0, 0.0);
         if (rc) return rc;
     }
     return SWM_OK;

@@ -1239,7 +1239,7 @@ extern "C" int swm_c_rk4_steps(swm_cctx *c, void *state, double dt, int nsteps) 
     if (c->graph_state != state || c->graph_dt != dt) c_drop_graphs(c);
     c->graph_state = state;
     c->graph_dt = dt;
-    return c->graphs.run(c->stream, nsteps, [&] { return c_enqueue_rk4_step(c, (double *)state, dt); });
+    return c->graphs.run(c->stream, 6LL * c->N * c->N, nsteps, [&] { return c_enqueue_rk4_step(c, (double *)state, dt); });
 }
 
 extern "C" int swm_c_diagnostics(swm_cctx *c, const void *state, double out[7]) {

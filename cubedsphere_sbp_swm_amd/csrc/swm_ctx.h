@@ -22,15 +22,18 @@ int fail(int code, const std::string &msg);
     } while (0)
 
 // Time steps of one state: runs of them through graphs of 4, 8, ... 64 steps, each made when a run first needs
-// it; the up to three steps left over, and the first run of a state, by plain launches.  A graph launch leaves
-// about 10 us between two graphs where kernels follow each other in 1 to 2, so a graph of one step is slower
-// than its four launches (C384 sbp42 FP64, 20 steps: 1797 us in graphs of one step, 1697 us by launches, 1724 us
-// in graphs of 16 and 4; C90 C grid 848, 809 and 809).  Long graphs pay where the host is what launches wait
-// for (C32 sbp21, 12 steps with three contexts at work: 192, 148 and 113 us).  Making them costs about 7 us a step,
-// which a first run that stays below FIRST steps does not earn back (C90 C grid, 10 steps: 1574 us with
-// the graphs made in the run, 850 us by launches).
+// it; the up to three steps left over, the first run of a state, and all steps of large grids by plain
+// launches.  A graph launch leaves about 10 us between two graphs where kernels follow each other in 1 to 2, so a
+// graph of one step is slower than its four launches (C384 sbp42 FP64, 20 steps: 1797 us in graphs of one
+// step, 1697 us by launches, 1724 us in graphs of 16 and 4).  Long graphs pay where launches cannot keep up: one
+// thread driving several small grids.  Us per step by graphs / by launches, three contexts: C32 sbp42
+// 9.8 / 11.7, C128 16.0 / 17.0, C256 33.8 / 34.3, C384 79.7 / 79.3; C grid C90 30.5 / 35.2, C192 60.4 / 63.1, C384
+// 232.5 / 231.3; so the line lies at POINTS, between C256 and C384.  Making graphs costs about 7 us a step, which
+// a first run of up to FIRST steps does not earn back (C90 C grid, 10 steps: 1574 us with the graphs made
+// in the run, 850 us by launches).
 struct StepGraphs {
     static constexpr int MIN = 4, KINDS = 5, FIRST = 128;
+    static constexpr long long POINTS = 600000;
     hipGraphExec_t exec[KINDS] = {};
     bool seen = false;  // a run of the state has been made
     void drop() {
@@ -40,19 +43,18 @@ struct StepGraphs {
         }
         seen = false;
     }
-    // nsteps of `step`, which enqueues one step on `stream`
+    // nsteps of `step`, which enqueues one step of a grid of `points` points on `stream`
     template <class Step>
-    int run(hipStream_t stream, int nsteps, const Step &step) {
+    int run(hipStream_t stream, long long points, int nsteps, const Step &step) {
         int rc;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         HIP_TRY(hipStreamIsCapturing(stream, &cap));
         if (cap != hipStreamCaptureStatusNone) return fail(SWM_EHIP, "time steps cannot be captured: they run graphs of their own");
-        if (!seen) {
-            // also ahead of a long run: its first step sets up what a capture could not
-            for (int q = nsteps <= FIRST ? nsteps : 1; q > 0; --q, --nsteps)
-                if ((rc = step())) return rc;
-            seen = true;
-        }
+        // a first step also goes ahead of a long run: it sets up what a capture could not
+        int plain = points > POINTS ? nsteps : seen ? 0 : nsteps <= FIRST ? nsteps : 1;
+        for (; plain > 0; --plain, --nsteps)
+            if ((rc = step())) return rc;
+        seen = true;
         for (int k = KINDS - 1; k >= 0; --k) {
             const int per = MIN << k, times = nsteps / per;
             nsteps -= times * per;
@@ -89,7 +91,7 @@ void free_hd_work(HdWork *w);
 
 // one fused stage launch on the context stream (swm_capi.hip)
 int run_stage(swm_ctx *c, int mode, const void *y, void *out, const void *v0, void *acc, double cy, double cacc,
-              void *zeta = nullptr);
+              void *zeta = nullptr, const void *kin = nullptr, double ck = 0.0, double ck1 = 0.0);
 
 }  // namespace swm_host
 
@@ -116,7 +118,7 @@ struct swm_ctx {
     double *J64 = nullptr, *Qi64[3] = {nullptr, nullptr, nullptr}, *f64 = nullptr, *A64 = nullptr;
     double *hs64 = nullptr;
     // RK4 work buffers (3 fields each) and diagnostics scratch
-    void *yA = nullptr, *yB = nullptr, *acc = nullptr, *curl = nullptr;
+    void *yA = nullptr, *yB = nullptr, *yC = nullptr, *curl = nullptr;
     double *red = nullptr;
     int red_blocks = 0;
     StepGraphs graphs;  // captured RK4 steps of (graph_state, graph_dt)

@@ -49,12 +49,12 @@ void fill_stage_table(swm_ens *e, int stage, std::vector<swm::EnsMember<T>> &tab
         a.hs = (const T *)c->hs;
         // the same buffers and coefficients as enqueue_rk4_step (rk4_mod.f90:28-40)
         switch (stage) {
-        case 0: a.y = (const T *)e->state[k]; a.out = (T *)c->yA; a.acc = (T *)c->acc; a.cy = (T)c1; a.cacc = (T)c2; break;
-        case 1: a.y = (const T *)c->yA; a.out = (T *)c->yB; a.v0 = (const T *)e->state[k]; a.acc = (T *)c->acc;
+        case 0: a.y = (const T *)e->state[k]; a.out = (T *)c->yA; a.acc = (T *)c->yC; a.cy = (T)c1; a.cacc = (T)c2; break;
+        case 1: a.y = (const T *)c->yA; a.out = (T *)c->yB; a.v0 = (const T *)e->state[k]; a.acc = (T *)c->yC;
                 a.cy = (T)c1; a.cacc = (T)c3; break;
-        case 2: a.y = (const T *)c->yB; a.out = (T *)c->yA; a.v0 = (const T *)e->state[k]; a.acc = (T *)c->acc;
+        case 2: a.y = (const T *)c->yB; a.out = (T *)c->yA; a.v0 = (const T *)e->state[k]; a.acc = (T *)c->yC;
                 a.cy = (T)dt; a.cacc = (T)c3; break;
-        default: a.y = (const T *)c->yA; a.out = (T *)e->state[k]; a.acc = (T *)c->acc; a.cy = (T)c2; a.cacc = (T)0; break;
+        default: a.y = (const T *)c->yA; a.out = (T *)e->state[k]; a.acc = (T *)c->yC; a.cy = (T)c2; a.cacc = (T)0; break;
         }
         tab[k].g = make_geo<T>(c);
         tab[k].a = a;
@@ -273,7 +273,9 @@ extern "C" int swm_ens_rk4_steps(swm_ens *e, const double *dt, int nsteps) {
     int rc0;
     for (swm_ctx *c : e->m)
         if ((rc0 = ens_order(e, c->stream, e->stream))) return rc0;
-    if ((rc0 = e->graphs.run(e->stream, nsteps, [&] { return ens_step(e); }))) return rc0;
+    long long points = 0;
+    for (const swm_ctx *c : e->m) points += c->fs;
+    if ((rc0 = e->graphs.run(e->stream, points, nsteps, [&] { return ens_step(e); }))) return rc0;
     // later work on a member's own stream (downloads, diagnostics) follows the ensemble steps
     for (swm_ctx *c : e->m)
         if ((rc0 = ens_order(e, e->stream, c->stream))) return rc0;

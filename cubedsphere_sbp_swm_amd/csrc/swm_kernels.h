@@ -78,12 +78,20 @@ struct DevGeo {
 };
 
 enum StageMode : int {
-    MODE_RHS = 0,     // out = RHS(y)
+    MODE_RHS = 0,     // out = RHS(y)                               (also the first stage of a step: out is k1)
     MODE_STAGE1 = 1,  // out = y + cy*k ; acc = y + cacc*k          (y is the step's v0)
     MODE_STAGE23 = 2, // out = v0 + cy*k ; acc = acc + cacc*k
     MODE_STAGE4 = 3,  // out = acc + cy*k                           (out is v0)
-    MODE_CURL = 4     // out(h plane) = synced relative vorticity of y
+    MODE_CURL = 4,    // out(h plane) = synced relative vorticity of y
+    MODE_SLOPE2 = 5,  // out = RHS(y + ck*kin)                      (y is v0, kin k1, out k2)
+    MODE_SLOPE3 = 6   // k = RHS(y + ck*kin): out = y + cy*k ; acc = ((y + ck1*acc) + cacc*kin) + cacc*k
+                      //                                            (y is v0, kin k2, acc holds k1 on entry)
 };
+// The stages of a step, rk4_mod.f90:28-40.  RK4 steps run RHS, SLOPE2, SLOPE3, STAGE4: stages 1 and 2 write
+// the slope only, 39 field passes a step; where the stage states themselves are wanted (the adjoint's
+// tape), STAGE1, STAGE23, STAGE23, STAGE4 write them and the sum, 48 passes.  Both form every value with
+// the same operations.
+SWM_HD constexpr bool mode_slope(int mode) { return mode == MODE_SLOPE2 || mode == MODE_SLOPE3; }
 
 template <typename T>
 struct StageArgs {
@@ -94,6 +102,8 @@ struct StageArgs {
     const T *hs;   // orography, may be null
     T cy, cacc;
     T *zeta;       // optional: the synced relative vorticity of y is also written here
+    const T *kin;  // slope of the previous stage (MODE_SLOPE2, MODE_SLOPE3)
+    T ck, ck1;
 };
 
 // Tile shapes (columns x rows of points, one thread per point) of the stage kernels: 64 x 8,
@@ -189,11 +199,14 @@ __device__ __forceinline__ T &at_byte(T *base, unsigned off) {
 template <typename T>
 struct PanelIn {
     const T *h, *u, *v, *hs, *J, *q11, *q12, *q22;
+    const T *kh, *ku, *kv;   // the stage's input is (h, u, v) + ck (kh, ku, kv) where mode_slope
+    T ck;
 };
 template <typename T>
-__device__ __forceinline__ PanelIn<T> panel_in(const DevGeo<T> &g, const T *y, const T *hs, int p) {
+__device__ __forceinline__ PanelIn<T> panel_in(const DevGeo<T> &g, const StageArgs<T> &a, int p) {
     const long long o = (long long)p * g.n * g.pitch, m = (long long)p * g.mps;
-    return {y + o, y + g.fs + o, y + 2 * g.fs + o, hs ? hs + o : nullptr, g.J + m, g.Qi11 + m, g.Qi12 + m, g.Qi22 + m};
+    return {a.y + o, a.y + g.fs + o, a.y + 2 * g.fs + o, a.hs ? a.hs + o : nullptr, g.J + m, g.Qi11 + m, g.Qi12 + m,
+            g.Qi22 + m, a.kin + o, a.kin + g.fs + o, a.kin + 2 * g.fs + o, a.ck};
 }
 template <typename T>
 __device__ __forceinline__ unsigned point_off(const DevGeo<T> &g, int i, int j) {
@@ -205,15 +218,21 @@ __device__ __forceinline__ unsigned point_off(const DevGeo<T> &g, int i, int j) 
 template <typename T>
 struct RawPoint {
     T h, u, v, J, q11, q12, q22, hs;
+    T kh, ku, kv;
 };
 
-template <bool OTF, typename T>
+template <int MODE, bool OTF, typename T>
 __device__ __forceinline__ RawPoint<T> load_point(const DevGeo<T> &g, const PanelIn<T> &in, int i, int j) {
     const unsigned o = point_off(g, i, j);
     RawPoint<T> r;
     r.h = at_byte(in.h, o);
     r.u = at_byte(in.u, o);
     r.v = at_byte(in.v, o);
+    if constexpr (mode_slope(MODE)) {
+        r.kh = at_byte(in.kh, o);
+        r.ku = at_byte(in.ku, o);
+        r.kv = at_byte(in.kv, o);
+    }
     if constexpr (OTF) {
         const Metric m = metric_otf(g.tanA, i, j);
         r.J = (T)m.J; r.q11 = (T)m.Qi11; r.q12 = (T)m.Qi12; r.q22 = (T)m.Qi22;
@@ -224,8 +243,14 @@ __device__ __forceinline__ RawPoint<T> load_point(const DevGeo<T> &g, const Pane
     return r;
 }
 
-template <typename T>
-__device__ __forceinline__ Derived<T> derived_of(const DevGeo<T> &g, const RawPoint<T> &r) {
+// r's h, u, v become the stage's input
+template <int MODE, typename T>
+__device__ __forceinline__ Derived<T> derived_of(const DevGeo<T> &g, RawPoint<T> &r, T ck) {
+    if constexpr (mode_slope(MODE)) {
+        r.h = r.h + ck * r.kh;
+        r.u = r.u + ck * r.ku;
+        r.v = r.v + ck * r.kv;
+    }
     return make_derived<T>(r.h, r.u, r.v, r.J, r.q11, r.q12, r.q22, r.hs, g.grav);
 }
 

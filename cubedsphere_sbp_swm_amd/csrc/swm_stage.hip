@@ -56,7 +56,7 @@ __device__ __forceinline__ EdgeDesc edge_desc(const int *ei) { return {ei[0], ei
 // stage vectors); loaded ahead of it so that their latency overlaps the stencil phases.
 template <typename T>
 struct OutPre {
-    T f, v0[3], acc[3];
+    T f, v0[3], acc[3], kin[3];
 };
 
 template <typename T, int MODE>
@@ -68,7 +68,11 @@ __device__ __forceinline__ OutPre<T> prefetch_point(const DevGeo<T> &g, const St
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         if constexpr (MODE == MODE_STAGE23) o.v0[k] = at_byte(a.v0 + (pb + k * g.fs), off);
-        if constexpr (MODE == MODE_STAGE23 || MODE == MODE_STAGE4) o.acc[k] = at_byte((const T *)a.acc + (pb + k * g.fs), off);
+        if constexpr (MODE == MODE_SLOPE3) {
+            o.v0[k] = at_byte(a.y + (pb + k * g.fs), off);
+            o.kin[k] = at_byte(a.kin + (pb + k * g.fs), off);
+        }
+        if constexpr (MODE == MODE_STAGE23 || MODE == MODE_STAGE4 || MODE == MODE_SLOPE3) o.acc[k] = at_byte((const T *)a.acc + (pb + k * g.fs), off);
     }
     return o;
 }
@@ -95,7 +99,7 @@ __device__ __forceinline__ void finish_point(const DevGeo<T> &g, const StageArgs
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const long long fc = c * g.fs;
-        if constexpr (MODE == MODE_RHS) {
+        if constexpr (MODE == MODE_RHS || MODE == MODE_SLOPE2) {
             at_byte(out + fc, off) = k[c];
         } else if constexpr (MODE == MODE_STAGE1) {
             at_byte(out + fc, off) = y[c] + a.cy * k[c];
@@ -103,6 +107,9 @@ __device__ __forceinline__ void finish_point(const DevGeo<T> &g, const StageArgs
         } else if constexpr (MODE == MODE_STAGE23) {
             at_byte(out + fc, off) = pre.v0[c] + a.cy * k[c];
             at_byte(acc + fc, off) = pre.acc[c] + a.cacc * k[c];
+        } else if constexpr (MODE == MODE_SLOPE3) {
+            at_byte(out + fc, off) = pre.v0[c] + a.cy * k[c];
+            at_byte(acc + fc, off) = ((pre.v0[c] + a.ck1 * pre.acc[c]) + a.cacc * pre.kin[c]) + a.cacc * k[c];
         } else if constexpr (MODE == MODE_STAGE4) {
             at_byte(out + fc, off) = pre.acc[c] + a.cy * k[c];
         }
@@ -121,9 +128,10 @@ __device__ __forceinline__ void load_rows(T *tab, int tid, int nthreads) {
 // of its halo exists and none is on a panel edge; its halo is the REACH of the interior row (2 points
 // for sbp42 and sbp43, 3 for sbp63, against 3, 5, 5 for the closure rows), its guards vanish and its
 // rows have constant weights.  The other tiles take their rows from the table.
-// At C384 sbp42 FP64 (64 x 8, metric read) an RK4 step takes 83 us in a long run, 20.7 us per stage: the
-// kernel moves about 135 MB per stage 2/3 at the 7 TB/s that a copy of cache-resident buffers of this
-// size reaches.  Wider halos, a branch and its code per closure row, 11-instruction divisions, 64-bit
+// At C384 sbp42 FP64 (64 x 8, metric read) an RK4 step takes 79 us by slopes and 83 us by states, 20.7 us per
+// stage: a stage 2/3 by states moves about 135 MB at the 7 TB/s that a copy of cache-resident buffers of
+// this size reaches.  With three contexts at work the states no longer fit the memory-side cache: 80 us by slopes, 92 by
+// states.  Wider halos, a branch and its code per closure row, 11-instruction divisions, 64-bit
 // offsets and panel-major tile order (metric read once per panel) took 24-25 us.
 template <int ORD, typename T, int MODE, int TX, int TY, bool OTF, bool PERSIST, bool INNER>
 __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T> &a, int p, int tx0, int ty0,
@@ -135,7 +143,7 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
     // and held in registers
     int tid = threadIdx.x;
     if constexpr (PERSIST) asm volatile("" : "+v"(tid));
-    const PanelIn<T> in = panel_in(g, a.y, a.hs, p);
+    const PanelIn<T> in = panel_in(g, a, p);
 
     // ---- load phase: every thread loads its own tile point (kept in registers for the output
     // phase), plus at most NH halo points, the y-halo rows first (whole waves), then the x-halo
@@ -146,7 +154,7 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
     const int i = tx0 + tx, j = ty0 + ty;
     const bool own_ok = INNER || (i < n && j < n);
     RawPoint<T> own{};
-    if (own_ok) own = load_point<OTF>(g, in, i, j);
+    if (own_ok) own = load_point<MODE, OTF>(g, in, i, j);
     RawPoint<T> rh[NH];
     int hc[NH], hr[NH];   // tile column and row of the halo point, relative to (tx0, ty0)
     bool okh[NH];
@@ -167,14 +175,14 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
             const int hi = tx0 + hc[k], hj = ty0 + hr[k];
             okh[k] = okh[k] && hi >= 0 && hj >= 0 && hi < n && hj < n;
         }
-        if (okh[k]) rh[k] = load_point<OTF>(g, in, tx0 + hc[k], ty0 + hr[k]);
+        if (okh[k]) rh[k] = load_point<MODE, OTF>(g, in, tx0 + hc[k], ty0 + hr[k]);
     }
     if constexpr (!INNER) load_rows<ORD, T>(tab, tid, NT);
     // of the own point only h, u, v, J and the mass fluxes h*ut, h*vt stay live for the output
     // phase (the same products the Coriolis term forms)
     T own_hu = T(0), own_hv = T(0);
     if (own_ok) {
-        const Derived<T> d = derived_of(g, own);
+        const Derived<T> d = derived_of<MODE>(g, own, in.ck);
         own_hu = d.hu;
         own_hv = d.hv;
         sm.K[ty + R][tx + R] = d.K;
@@ -186,7 +194,7 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
 #pragma unroll
     for (int k = 0; k < NH; ++k) {
         if (!okh[k]) continue;
-        const Derived<T> d = derived_of(g, rh[k]);
+        const Derived<T> d = derived_of<MODE>(g, rh[k], in.ck);
         sm.K[hr[k] + R][hc[k] + R] = d.K;
         if (tid + k * NT < NYH) {
             sm.Gyd[hr[k] + R][hc[k]] = d.Gyd;
@@ -298,9 +306,9 @@ __device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T
         }
         if (!ok) continue;
         const int nidx = ei.tnu == 0 ? d : n - 1 - d, tidx = ei.a_base + ei.s * kk;
-        const PanelIn<T> in = panel_in(g, a.y, a.hs, ei.q);
-        const RawPoint<T> rp = load_point<OTF>(g, in, ei.nu_x ? nidx : tidx, ei.nu_x ? tidx : nidx);
-        const Derived<T> dv = derived_of(g, rp);
+        const PanelIn<T> in = panel_in(g, a, ei.q);
+        RawPoint<T> rp = load_point<MODE, OTF>(g, in, ei.nu_x ? nidx : tidx, ei.nu_x ? tidx : nidx);
+        const Derived<T> dv = derived_of<MODE>(g, rp, in.ck);
         const T nD = ei.nu_x ? dv.Gxd : dv.Gyd, nC = ei.nu_x ? dv.Gxc : dv.Gyc;
         const T tD = ei.nu_x ? dv.Gyd : dv.Gxd, tC = ei.nu_x ? dv.Gyc : dv.Gxc;
         if (!corner) {
@@ -496,6 +504,8 @@ hipError_t launch_one(int mode, const DevGeo<T> &g, const StageArgs<T> &a, hipSt
     case MODE_STAGE1: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_STAGE1, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_STAGE23: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_STAGE23, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_STAGE4: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_STAGE4, TX, TY, OTF>), grid, block, 0, s, g, a); break;
+    case MODE_SLOPE2: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_SLOPE2, TX, TY, OTF>), grid, block, 0, s, g, a); break;
+    case MODE_SLOPE3: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_SLOPE3, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     case MODE_CURL: hipLaunchKernelGGL((stage_kernel<ORD, T, MODE_CURL, TX, TY, OTF>), grid, block, 0, s, g, a); break;
     default: return hipErrorInvalidValue;
     }
