@@ -11,7 +11,7 @@ struct swm_ens {
     int prec = 64, order = 42;
     hipStream_t stream = nullptr;
     int num_cu = 0;
-    int tx = 64, ty = 8, bps = 1;  // tile shape (swm::tile_shape_ok), blocks per resident slot (0: one per task)
+    int tx = 32, ty = 16, bps = 0;  // tile shape (swm::tile_shape_ok), blocks per resident slot (0: one per task)
     bool otf = false;
     void *tables[4] = {nullptr, nullptr, nullptr, nullptr};  // EnsMember<T>[m] per RK stage
     int2 *tasks = nullptr;  // per task of the launch: (member, task index within the member)
@@ -194,6 +194,18 @@ extern "C" int swm_ens_create(swm_ctx *const *members, void *const *states, int 
         e->state.push_back(states[k]);
     }
     e->stream = members[0]->stream;
+    // Defaults (the autotuner measures): one block per task in hardware order; FP64 metric terms from the tangents,
+    // as each member has planes of its own, which no other member's tiles share; 32 x 16 tiles, or for sbp42 in
+    // FP64, whose halo is the narrowest, 32 x 8 from 1e6 points on, where there are tasks enough for the
+    // smaller blocks.  Us per step, 64 x 8 with the metric read in a persistent grid / 32 x 16 / 32 x 8:
+    //   sbp42 FP64  16 members C48-C192 (1.7e6 points) 246 / 211 / 204, 64 members 1200 / 1003 / 968,
+    //               32 x C64 213 / 184 / 170, 4 members C32-C64 37.8 / 35.6 / 41.0, C17-C250 75.2 / 70.2 / 71.8
+    //   sbp43 FP64  8 x C128 134 / 123 / 127;  sbp63 FP64  16 members 277 / 232 / 240, 8 x C96 106 / 89 / 96
+    //   sbp42 FP32  16 members 173 / 151 / 149, 8 x C192 145 / 132 / 137
+    long long points = 0;
+    for (const swm_ctx *c : e->m) points += c->fs;
+    e->otf = e->prec == 64;
+    if (points >= 1000000 && e->order == 42 && e->prec == 64) e->ty = 8;
     int dev = 0;
     hipDeviceProp_t prop;
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) {
