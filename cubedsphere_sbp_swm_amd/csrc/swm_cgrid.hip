@@ -403,7 +403,7 @@ __device__ __forceinline__ double curl_at(const CGeo &g, const double *__restric
 // One tile configuration: TX x TY cells, NT threads
 template <int TX, int TY, int NT>
 struct CTiles {
-static constexpr int X = TX, Y = TY, THREADS = NT;
+static constexpr int X = TX, Y = TY, THREADS = NT, SLOTS = 256 * 2048 / NT;
 
 // every point (column c, row r, pass k) of a W x R box dealt to the NT threads, the first to thread FROM
 template <int W, int R, int FROM = 0, class F>
@@ -417,19 +417,21 @@ static __device__ __forceinline__ void each(int tid, const F &f) {
 }
 template <int W, int R> static constexpr int passes() { return (W * R + NT - 1) / NT; }
 
-static __device__ __forceinline__ CTile c_tile(const CGeo &g, int t) {
-    const int ntx = (g.N + TX - 1) / TX, strip = t / (6 * ntx), rem = t - strip * 6 * ntx;
+static __device__ __forceinline__ CTile c_tile(const CGeo &g, const swm::TilePos &at) {
     CTile c;
-    c.p = rem / ntx;
-    c.x0 = (rem - c.p * ntx) * TX + 1;
-    c.y0 = strip * TY + 1;
+    c.p = at.p;
+    c.x0 = at.cx * TX + 1;
+    c.y0 = at.cy * TY + 1;
     c.x1 = min(c.x0 + TX - 1, g.N);
     c.y1 = min(c.y0 + TY - 1, g.N);
     c.fx1 = c.x1 + (c.x1 == g.N);
     c.fy1 = c.y1 + (c.y1 == g.N);
     return c;
 }
-// full tiles all of whose rows are interior ones
+// inner tiles: full ones all of whose rows are interior ones (7 <= x0, x1 <= N - 5)
+static swm::TileOrder order(int N) {
+    return swm::tile_order(SLOTS, (N + TX - 1) / TX, (N + TY - 1) / TY, (6 + TX - 1) / TX, (N - 5) / TX, (6 + TY - 1) / TY, (N - 5) / TY);
+}
 static __device__ __forceinline__ bool c_inner(const CGeo &g, const CTile &c) {
     return c.x0 >= 7 && c.y0 >= 7 && c.x1 <= g.N - 5 && c.y1 <= g.N - 5 && c.x1 - c.x0 == TX - 1 && c.y1 - c.y0 == TY - 1;
 }
@@ -798,27 +800,28 @@ static __device__ __forceinline__ void tend_tile(const CGeo &g, const double *__
 
 // 16 x 8 cells and two threads per cell: the phases of a tile have 1.3 to 3 tasks per cell, a block is a
 // chain of load, three LDS phases and stores whose length is what a launch of few tiles takes, and 8 such
-// blocks fit a CU.  RK4 step (8 launches), C90 / C384 / C512: 73 / 241 / 361 us; 8 x 8 cells 75 / 342 / 537,
-// 32 x 4 69 / 273 / 406, 32 x 8 with 512 threads 85 / 306 / 460, with 256 124 / 287 / 383; the
+// blocks fit a CU.  RK4 step (8 launches), C90 / C384 / C512: 74 / 241 / 365 us in plain band order, 75 / 191 / 306
+// with the ring first (TileOrder: 29 and 35 us a launch at C384, 24 and 29 then); in band order 8 x 8 cells
+// 75 / 342 / 537, 32 x 4 69 / 273 / 406, 32 x 8 with 512 threads 85 / 306 / 460, with 256 124 / 287 / 383; the
 // eight-launch form with its intermediates in memory 140 / 391 us.
 using Tiles = CTiles<16, 8, 256>;
 
-__global__ void __launch_bounds__(Tiles::THREADS) k_flux(CGeo g, const double *__restrict__ y, double *__restrict__ G,
-                                                         double *__restrict__ KE, double *__restrict__ W, int ntiles) {
+__global__ void __launch_bounds__(Tiles::THREADS) k_flux(swm::TileOrder order, CGeo g, const double *__restrict__ y, double *__restrict__ G,
+                                                         double *__restrict__ KE, double *__restrict__ W) {
     __shared__ union { Tiles::FluxSmem<true> in; Tiles::FluxSmem<false> any; } sm;
     __shared__ double tab[ROW_SIZE];
-    const CTile t = Tiles::c_tile(g, swm::xcd_tile(blockIdx.x, ntiles));
+    const CTile t = Tiles::c_tile(g, swm::tile_pos(order, blockIdx.x));
     if (Tiles::c_inner(g, t)) Tiles::flux_tile<true>(g, y, G, KE, W, t, sm.in, tab);
     else Tiles::flux_tile<false>(g, y, G, KE, W, t, sm.any, tab);
 }
 
 template <int RKM>
-__global__ void __launch_bounds__(Tiles::THREADS) k_tend(CGeo g, const double *__restrict__ h, const double *__restrict__ G,
+__global__ void __launch_bounds__(Tiles::THREADS) k_tend(swm::TileOrder order, CGeo g, const double *__restrict__ h, const double *__restrict__ G,
                                                             const double *__restrict__ KE, const double *__restrict__ W,
-                                                            RkArgs r, int ntiles) {
+                                                            RkArgs r) {
     __shared__ union { Tiles::TendSmem<true> in; Tiles::TendSmem<false> any; } sm;
     __shared__ double tab[ROW_SIZE];
-    const CTile t = Tiles::c_tile(g, swm::xcd_tile(blockIdx.x, ntiles));
+    const CTile t = Tiles::c_tile(g, swm::tile_pos(order, blockIdx.x));
     if (Tiles::c_inner(g, t)) Tiles::tend_tile<RKM, true>(g, h, G, KE, W, r, t, sm.in, tab);
     else Tiles::tend_tile<RKM, false>(g, h, G, KE, W, r, t, sm.any, tab);
 }
@@ -963,11 +966,10 @@ template <int RKM>
 int c_enqueue_rhs(swm_cctx *c, const double *y, const swmc::RkArgs &r) {
     using K = swmc::Tiles;
     const swmc::CGeo g = make_cgeo(c);
-    const int ntiles = 6 * ((c->N + K::X - 1) / K::X) * ((c->N + K::Y - 1) / K::Y);
-    const dim3 blk(K::THREADS), grd(ntiles);
-    hipLaunchKernelGGL(swmc::k_flux, grd, blk, 0, c->stream, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W), ntiles);
-    hipLaunchKernelGGL(swmc::k_tend<RKM>, grd, blk, 0, c->stream, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W), r,
-                       ntiles);
+    const swm::TileOrder o = K::order(c->N);
+    const dim3 blk(K::THREADS), grd(o.blocks());
+    hipLaunchKernelGGL(swmc::k_flux, grd, blk, 0, c->stream, o, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W));
+    hipLaunchKernelGGL(swmc::k_tend<RKM>, grd, blk, 0, c->stream, o, g, y, c->wf(CW_G), c->wf(CW_KE), c->wf(CW_W), r);
     HIP_TRY(hipGetLastError());
     return SWM_OK;
 }

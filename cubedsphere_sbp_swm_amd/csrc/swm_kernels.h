@@ -395,4 +395,44 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
     return xcd < r ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// Order of the tiles of a cube (ntx x nty per panel) whose launch treats tiles with closure rows (the ring) apart
+// from the inner ones, columns bx0..bx1-1 of strips by0..by1-1.  A ring tile takes several times an inner
+// one; in band order the first and the last XCD would hold a strip of nothing else, and the last one start
+// it last.  So the ring goes first, dealt evenly to the XCDs, then the inner tiles, an even share of bands each.
+// Within both parts: row strips outermost, then panels, then columns; an XCD's contiguous range is a band of
+// all six panels, which read the same metric there.  Where all blocks are resident at once (`slots` of
+// them) none waits for another, and all tiles go as ring.
+struct TileOrder {
+    int ntx, nty, bx0, bx1, by0, by1, ring, inner;
+    SWM_HD int blocks() const { return ring + inner; }
+};
+inline TileOrder tile_order(int slots, int ntx, int nty, int bx0, int bx1, int by0, int by1) {
+    TileOrder o{ntx, nty, bx0, bx1, by0, by1, 0, 0};
+    if (6 * ntx * nty <= slots || bx1 <= bx0 || by1 <= by0) o.bx0 = o.bx1 = o.by0 = o.by1 = 0;
+    o.inner = 6 * (o.bx1 - o.bx0) * (o.by1 - o.by0);
+    o.ring = 6 * ntx * nty - o.inner;
+    return o;
+}
+struct TilePos {
+    int p, cx, cy;
+};
+// Selects only: with branches here the kernel's other arguments are loaded after them, a second trip to
+// memory (0.6 us a launch).
+__device__ __forceinline__ TilePos tile_pos(const TileOrder &o, int b) {
+    const bool in = b >= o.ring;
+    const unsigned nb = in ? o.inner : o.ring, lb = in ? b - o.ring : b;
+    // xcd_tile(lb, nb); the inner tiles' shares rotate over the XCDs by ring
+    const unsigned q8 = nb / 8, r8 = nb % 8, xcd = lb % 8, extra = xcd < r8 ? xcd : r8;
+    unsigned q = xcd * q8 + extra + lb / 8;
+    const unsigned wi = o.bx1 - o.bx0, full = 6u * o.ntx * (o.nty - (o.by1 - o.by0));
+    const bool sides = !in && q >= full;   // beside the inner tiles of a strip, not a strip without any
+    q = sides ? q - full : q;
+    const unsigned w = in ? wi : sides ? o.ntx - wi : o.ntx;
+    const unsigned s = q / (6 * w), rem = q - s * 6 * w, p = rem / w;
+    int cx = rem - p * w, cy = s;
+    cx = in || (sides && cx >= o.bx0) ? cx + (in ? o.bx0 : (int)wi) : cx;
+    cy = in || sides ? cy + o.by0 : cy >= o.by0 ? cy + (o.by1 - o.by0) : cy;
+    return {(int)p, cx, cy};
+}
+
 }  // namespace swm
