@@ -272,6 +272,7 @@ struct AdjTile {
     static constexpr int R = SbpT<ORD>::R, B = SbpT<ORD>::B, NR = SbpT<ORD>::B + SbpT<ORD>::W;
     static constexpr int span(int t) { return (t + R + B - 1 > NR) ? t + R + B - 1 : NR; }
     static constexpr int LW = span(TX), LH = span(TY), NT = TX * TY;
+    static constexpr int M = B > R ? B : R + 1;   // points between an inner tile and the panel edge
     static_assert(TX >= B && TY >= B, "a tile holds the closure columns of at most one boundary");
 };
 
@@ -565,17 +566,14 @@ __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, 
 }
 
 template <int ORD, int MODE, int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) adj_tile(AdjGeo g, AdjArgs A, AdjEll ell) {
+__global__ void __launch_bounds__(TX * TY) adj_tile(TileOrder order, AdjGeo g, AdjArgs A, AdjEll ell) {
     using Tl = AdjTile<ORD, TX, TY>;
     __shared__ double box[4][Tl::LH][Tl::LW];
     __shared__ double tab[ColWeights<ORD>::SIZE];
-    const int n = g.n, ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
-    // row strips outermost, then panels: an XCD's contiguous range is a band of all six panels, which share
-    // the metric
-    const int t = xcd_tile(blockIdx.x, 6 * ntx * nty);
-    const int strip = t / (6 * ntx), rem = t - strip * 6 * ntx, p = rem / ntx;
-    const int x0 = (rem - p * ntx) * TX, y0 = strip * TY;
-    constexpr int M = Tl::B > Tl::R ? Tl::B : Tl::R + 1;
+    const int n = g.n;
+    const TilePos at = tile_pos(order, blockIdx.x);
+    const int p = at.p, x0 = at.cx * TX, y0 = at.cy * TY;
+    constexpr int M = Tl::M;
     if (x0 >= M && y0 >= M && x0 + TX <= n - M && y0 + TY <= n - M)
         adj_tile_run<ORD, MODE, TX, TY, true>(g, A, ell, p, x0, y0, box, tab);
     else
@@ -759,13 +757,13 @@ hipError_t launch_adj_main(int mode, const swm::AdjGeo &g, const swm::AdjArgs &a
 template <int ORD, int TX>
 hipError_t launch_adj_tile(int mode, const swm::AdjGeo &g, const swm::AdjArgs &a, const swm::AdjEll &e, hipStream_t s) {
     constexpr int TY = 16;
-    const int nb = 6 * ((g.n + TX - 1) / TX) * ((g.n + TY - 1) / TY);
-    const dim3 blk(TX * TY), grd(nb);
+    const swm::TileOrder o = swm::point_tile_order(256 * 1024 / (TX * TY), g.n, 0, g.n, swm::AdjTile<ORD, TX, TY>::M, TX, TY);
+    const dim3 blk(TX * TY), grd(o.blocks());
     switch (mode) {
-    case swm::ADJ_VJP: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_VJP, TX, TY>), grd, blk, 0, s, g, a, e); break;
-    case swm::ADJ_S4: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S4, TX, TY>), grd, blk, 0, s, g, a, e); break;
-    case swm::ADJ_S32: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S32, TX, TY>), grd, blk, 0, s, g, a, e); break;
-    default: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S1, TX, TY>), grd, blk, 0, s, g, a, e); break;
+    case swm::ADJ_VJP: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_VJP, TX, TY>), grd, blk, 0, s, o, g, a, e); break;
+    case swm::ADJ_S4: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S4, TX, TY>), grd, blk, 0, s, o, g, a, e); break;
+    case swm::ADJ_S32: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S32, TX, TY>), grd, blk, 0, s, o, g, a, e); break;
+    default: hipLaunchKernelGGL((swm::adj_tile<ORD, swm::ADJ_S1, TX, TY>), grd, blk, 0, s, o, g, a, e); break;
     }
     return hipGetLastError();
 }

@@ -403,7 +403,7 @@ __device__ __forceinline__ double curl_at(const CGeo &g, const double *__restric
 // One tile configuration: TX x TY cells, NT threads
 template <int TX, int TY, int NT>
 struct CTiles {
-static constexpr int X = TX, Y = TY, THREADS = NT, SLOTS = 256 * 2048 / NT;
+static constexpr int X = TX, Y = TY, THREADS = NT, SLOTS = 512;
 
 // every point (column c, row r, pass k) of a W x R box dealt to the NT threads, the first to thread FROM
 template <int W, int R, int FROM = 0, class F>

@@ -232,6 +232,7 @@ struct HdTile {
     static constexpr int one(int t) { return ext(t) > NR ? ext(t) : NR; }
     static constexpr int span(int t) { return one(t) > both(t) ? one(t) : both(t); }
     static constexpr int LW = span(TX), LH = span(TY), NT = TX * TY;
+    static constexpr int M = B > R ? B : R + 1;   // points between an inner tile and the panel edge
 };
 template <int W, int H, int TX, int TY, int NF>
 struct HdSmem {
@@ -302,7 +303,8 @@ struct HdFin {
 // tile +-R, no panel-edge point, so every row of it is an interior row.
 // Bound by latency with three blocks a CU (LDS 41 KB at sbp42, 96 and 115 registers): its waves wait 57 % of
 // their cycles, its vector instructions need 14 us and its fields at the rate of a large copy 10 us of the
-// 45 (STEP 1) and 56 us (STEP 2) at C384 sbp42, alone on the chip; C191 sbp63: 27 and 33 us.  The six separate
+// 45 (STEP 1) and 56 us (STEP 2) at C384 sbp42, alone on the chip, in plain band order; with the ring first
+// (TileOrder) the step takes 86 us instead of 103.  C191 sbp63: 27 and 33 us in band order.  The six separate
 // launches of the four fields that they take the place of took 167 us and 85 us with the edge launches.
 template <int ORD, bool H, bool UV, int STEP, int TX, int TY, bool INNER, class Smem>
 __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const double *__restrict__ in, double *__restrict__ out,
@@ -543,19 +545,16 @@ __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const
 }
 
 template <int ORD, bool H, bool UV, int STEP, int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) hd_lap(HdGeo g, HdLn ln, const double *__restrict__ in, double *__restrict__ out,
+__global__ void __launch_bounds__(TX * TY) hd_lap(TileOrder order, HdGeo g, HdLn ln, const double *__restrict__ in, double *__restrict__ out,
                                                   const double *__restrict__ Ein, double *__restrict__ Eout, HdFin fin) {
     using C = HdTile<ORD, TX, TY>;
     constexpr int NF = (H ? 1 : 0) + (UV ? 3 : 0), R = C::R;
     __shared__ union { HdSmem<TX + 2 * R, TY + 2 * R, TX, TY, NF> in; HdSmem<C::LW, C::LH, TX, TY, NF> any; } sm;
     __shared__ double tab[RowWeights<ORD>::SIZE];
-    const int n = g.n, ntx = (n + TX - 1) / TX, nty = (n + TY - 1) / TY;
-    // row strips outermost, then panels: an XCD's contiguous range is a band of all six panels, which share
-    // the metric, the weights and the basis planes
-    const int t = xcd_tile(blockIdx.x, 6 * ntx * nty);
-    const int strip = t / (6 * ntx), rem = t - strip * 6 * ntx, p = rem / ntx;
-    const int x0 = (rem - p * ntx) * TX, y0 = strip * TY;
-    constexpr int M = C::B > R ? C::B : R + 1;
+    const int n = g.n;
+    const TilePos at = tile_pos(order, blockIdx.x);
+    const int p = at.p, x0 = at.cx * TX, y0 = at.cy * TY;
+    constexpr int M = C::M;
     if (x0 >= M && x0 + TX <= n - M && y0 >= M && y0 + TY <= n - M)
         hd_lap_run<ORD, H, UV, STEP, TX, TY, true>(g, ln, in, out, Ein, Eout, fin, p, x0, y0, sm.in, tab);
     else
@@ -741,8 +740,7 @@ void hd_edge_tables(const swm_ctx *c, const std::vector<double> &b1, const std::
     const size_t depths = c->host_nbr.size() / ((size_t)6 * 4 * n * 4);
     for (int p = 0; p < 6; ++p)
         for (int j = 0; j < n; ++j)
-            for (int i = 0; i < n; ++i) {
-                if (i && j && i < n - 1 && j < n - 1) continue;
+            for (int i = 0; i < n; i += j == 0 || j == n - 1 ? 1 : n - 1) {
                 const int t = p * es + slot(i, j);
                 int4 e = make_int4(-1, -1, 0, 0);
                 for (int d = 0; d < 2; ++d) {   // 0: across an x edge, 1: across a y edge
@@ -828,16 +826,16 @@ int ensure_hd(swm_ctx *c, int order) {
 }
 
 // 16 x 16 points, a thread each.  Both steps of four fields at C384 sbp42 / C191 sbp63, per pass with three
-// contexts at work: 70 us / 124 us; 32 x 8 86 / 154, 16 x 8 with 128 threads 78 / 152; more threads than points, so
+// contexts at work and in band order: 70 us / 124 us; 32 x 8 86 / 154, 16 x 8 with 128 threads 78 / 152; more threads than points, so
 // that each phase of a box is one round (320 to 448), 102 to 113 / 139 to 150; two threads a point with two
 // fields each 93 / 128.
-constexpr int HTX = 16, HTY = 16;
+constexpr int HTX = 16, HTY = 16, HSLOTS = 768;
 
 template <int ORD, bool H, bool UV, int STEP>
 int launch_lap(swm_ctx *c, const double *in, double *out, const double *Ein, double *Eout, const swm::HdFin &fin) {
-    const int tiles = 6 * ((c->n + HTX - 1) / HTX) * ((c->n + HTY - 1) / HTY);
-    hipLaunchKernelGGL((swm::hd_lap<ORD, H, UV, STEP, HTX, HTY>), dim3(tiles), dim3(HTX * HTY), 0, c->stream, hd_geo(c), hd_ln<ORD>(c),
-                       in, out, Ein, Eout, fin);
+    const swm::TileOrder o = swm::point_tile_order(HSLOTS, c->n, 0, c->n, swm::HdTile<ORD, HTX, HTY>::M, HTX, HTY);
+    hipLaunchKernelGGL((swm::hd_lap<ORD, H, UV, STEP, HTX, HTY>), dim3(o.blocks()), dim3(HTX * HTY), 0, c->stream, o, hd_geo(c),
+                       hd_ln<ORD>(c), in, out, Ein, Eout, fin);
     HIP_TRY(hipGetLastError());
     return SWM_OK;
 }

@@ -400,8 +400,12 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
 // one; in band order the first and the last XCD would hold a strip of nothing else, and the last one start
 // it last.  So the ring goes first, dealt evenly to the XCDs, then the inner tiles, an even share of bands each.
 // Within both parts: row strips outermost, then panels, then columns; an XCD's contiguous range is a band of
-// all six panels, which read the same metric there.  Where all blocks are resident at once (`slots` of
-// them) none waits for another, and all tiles go as ring.
+// all six panels, which read the same metric there.  Up to `slots` tiles, where nearly all blocks are resident
+// at once and little waits for a ring tile, all go as ring.  Us alone on the chip, band order / ring first: C-grid
+// step C192 113 / 98, C384 241 / 191; hyperdiffusion step C256 sbp42 70 / 51, C384 103 / 86, sbp63 160 / 119;
+// transposed RHS with its curl C256 sbp42 28.0 / 24.4, C384 43.5 / 37.7.  Below the lines: C-grid step C64
+// 74.9 / 77.3, transposed RHS C192 19.8 / 20.5.  The RK stage kernels stay in band order: their large tiles are a
+// third ring, and a C384 step with three contexts at work went from 80 to 81 us (C768 FP32 alone 166 to 155).
 struct TileOrder {
     int ntx, nty, bx0, bx1, by0, by1, ring, inner;
     SWM_HD int blocks() const { return ring + inner; }
@@ -412,6 +416,13 @@ inline TileOrder tile_order(int slots, int ntx, int nty, int bx0, int bx1, int b
     o.inner = 6 * (o.bx1 - o.bx0) * (o.by1 - o.by0);
     o.ring = 6 * ntx * nty - o.inner;
     return o;
+}
+// the order for tiles of tx x ty points covering the points first .. first + len - 1 of a panel line of n
+// points, inner where all their points lie in margin .. n - 1 - margin
+inline TileOrder point_tile_order(int slots, int n, int first, int len, int margin, int tx, int ty) {
+    auto lo = [&](int t) { return (margin - first + t - 1) / t; };
+    auto hi = [&](int t) { return n - margin - first > 0 ? (n - margin - first) / t : 0; };
+    return tile_order(slots, (len + tx - 1) / tx, (len + ty - 1) / ty, lo(tx), hi(tx), lo(ty), hi(ty));
 }
 struct TilePos {
     int p, cx, cy;
