@@ -128,21 +128,22 @@ extern "C" void swmh_geometry(int N, int pitch, double omega, const double axis[
 extern "C" void swmh_basis_b(int N, int pitch, double *b1, double *b2) {
     const int n = N + 1;
     const long plane = 6L * n * pitch;
-    for (int p = 0; p < 6; ++p)
-        for (int j = 1; j <= n; ++j) {
-            const double beta = grid_coord(N, j);
-            for (int i = 1; i <= n; ++i) {
-                const double alpha = grid_coord(N, i);
+    for (int j = 1; j <= n; ++j) {
+        const double beta = grid_coord(N, j);
+        for (int i = 1; i <= n; ++i) {
+            const double alpha = grid_coord(N, i);
+            double v1[3], v2[3], w[3];
+            b1_proto(alpha, beta, v1);
+            b2_proto(alpha, beta, v2);
+            for (int p = 0; p < 6; ++p) {
                 const long id = ((long)p * n + (j - 1)) * pitch + (i - 1);
-                double v[3], w[3];
-                b1_proto(alpha, beta, v);
-                to_panel(p, v, w);
+                to_panel(p, v1, w);
                 for (int k = 0; k < 3; ++k) b1[id + k * plane] = w[k];
-                b2_proto(alpha, beta, v);
-                to_panel(p, v, w);
+                to_panel(p, v2, w);
                 for (int k = 0; k < 3; ++k) b2[id + k * plane] = w[k];
             }
         }
+    }
 }
 
 // create_latlon_interp (regrid_factory_mod.f90:183-301) on the Ah (xy) mesh: stencil bounds
