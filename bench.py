@@ -297,11 +297,10 @@ def _adjoint_single_segment(args, op, tape, y0, lam, grads, timed_pair, stream):
             "gradient_ms": (t_f + t_b) * 1e3, "gradient_bitwise_equal_to_checkpointed": bool(same)}
 
 
-# algorithmic FP64 values per point of one explicit hyperdiffusion step (4 fields: h and the
-# Cartesian velocity): to Cartesian 9 read (h, u, v, b1, b2) / 4 written; per Laplacian
-# application the 4 fields and J, Qi11, Qi12, Qi22 read once / 4 written; tendencies and Euler
-# step 13 read / 3 written (edge syncs O(N))
-DIFF_VALUES = (9 + 4) + 2 * ((4 + 4) + 4) + (13 + 3)
+# FP64 values per point of one explicit hyperdiffusion step, each field of a launch read or written once,
+# the planes that all panels share (basis, metric, D2 weights) not counted: first Laplacian h, u, v
+# read / 4 written; second Laplacian and Euler step 4 + 3 read / 3 written (panel edges O(N))
+DIFF_VALUES = (3 + 4) + (4 + 3 + 3)
 
 
 def hyperdiffusion_form(args, stream, op, x):
@@ -328,19 +327,17 @@ def hyperdiffusion_form(args, stream, op, x):
     points = 6 * (args.N + 1) ** 2
     gbs = DIFF_VALUES * 8 * points / (us * 1e-6) / 1e9
     return {"workload": f"C{args.N} sbp42 FP64 explicit_Eul1 hyperdiffusion step, hordiff_vec_xyz_Ah_sbp_42_narrow "
-                        "0.03 + hordiff_scalar_Ah_sbp_42_narrow 0.01 (7 launches)",
+                        "0.03 + hordiff_scalar_Ah_sbp_42_narrow 0.01 (3 launches)",
             "us_per_step": us, "algorithmic_bytes_per_step": DIFF_VALUES * 8 * points,
             "effective_GBs": gbs, "frac": gbs / HBM_PEAK_GBS,
             "sbp63_us_per_step": us63}
 
 
-# Field passes of one C-grid RK4 step as implemented (fields read or written once per kernel,
-# shared metric planes not counted): RHS = 4 (contra_o: u, v; A, B) + 9 (flux: A, B, h, u, v;
-# G pair, KEu, KEv) + 6 (ke_div: KEu, KEv, h, G pair; KE) + 3 (curl: u, v; W) + 3 (w2uv: W; fu,
-# fv) + 7 (cor_o: fu, fv, G pair, h, f; cup, cvp) + 3 (mom: KE, cup, cvp) = 35, plus the
-# tendency outputs: stages 1-3 write k (3), read v0 (3) and write the next input (3), stage 4
-# reads v0, k0, k1, k2 (12) and writes v0 (3): step = 4 x 35 + 3 x 9 + 15.
-C_STEP_FIELD_PASSES = 182
+# Field passes of one C-grid RK4 step as implemented (fields read or written once per kernel, shared
+# metric planes not counted): RHS = 7 (flux: h, u, v; G pair, KE, W) + 6 (tend: h, G pair, KE, W, f), and
+# the stage updates in tend: stage 1 reads v0 (3) and writes the next input and the sum (6), stages 2 and 3
+# also read the sum (12), stage 4 reads the sum and writes the state (6): step = 4 x 13 + 9 + 2 x 12 + 6.
+C_STEP_FIELD_PASSES = 91
 
 
 def cgrid_ecs_timings(args, op, xs, reps=200):

@@ -24,8 +24,7 @@
 // in k_flux; the curl at x and y points and the Coriolis terms at o points in k_tend) lives in LDS on
 // the tile and the halo that the next stencil reads; only the four fields that need the neighbour
 // panels' values go through memory between the two.  Eight launches with the intermediates in
-// memory move 140 field passes per step more and leave each launch near its latency floor.  The RK4
-// step is captured into a HIP graph.
+// memory move 91 field passes per step more and leave each launch near its latency floor.
 //
 // Every expression keeps the reference's operation order with no fused multiply-adds
 // (-ffp-contract=off), so results match an FP64 CPU evaluation of the same algorithm bit for bit.

@@ -303,9 +303,8 @@ struct HdFin {
 // tile +-R, no panel-edge point, so every row of it is an interior row.
 // Bound by latency with three blocks a CU (LDS 41 KB at sbp42, 96 and 115 registers): its waves wait 57 % of
 // their cycles, its vector instructions need 14 us and its fields at the rate of a large copy 10 us of the
-// 45 (STEP 1) and 56 us (STEP 2) at C384 sbp42, alone on the chip, in plain band order; with the ring first
-// (TileOrder) the step takes 86 us instead of 103.  C191 sbp63: 27 and 33 us in band order.  The six separate
-// launches of the four fields that they take the place of took 167 us and 85 us with the edge launches.
+// 37 (STEP 1) and 40 us (STEP 2) at C384 sbp42, alone on the chip (45 and 56 in plain band order); C191 sbp63:
+// 23 and 28 us (27 and 33).  The six separate launches of the four fields that they take the place of took 167 us and 85 us with the edge launches.
 template <int ORD, bool H, bool UV, int STEP, int TX, int TY, bool INNER, class Smem>
 __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const double *__restrict__ in, double *__restrict__ out,
                                            const double *__restrict__ Ein, double *__restrict__ Eout, const HdFin &fin,

@@ -77,7 +77,8 @@ int swm_assign(swm_ctx *ctx, void *out, double s1, const void *v1, double s2, co
 int swm_update(swm_ctx *ctx, void *out, double s1, const void *v1, double s2, const void *v2);
 
 /* timescheme_t%step for rk4 (time_schemes/rk4_mod.f90:20-42), nsteps times, in place,
- * one fused kernel per RK stage (4 launches per step, captured in a HIP graph) */
+ * one fused kernel per RK stage (4 launches per step; repeated runs of steps of small grids go through
+ * HIP graphs) */
 int swm_rk4_steps(swm_ctx *ctx, void *state, double dt, int nsteps);
 
 /* operator_t%get_diagnostics (operator_swm_mod.f90:115-260):
@@ -177,8 +178,8 @@ int swm_ctx_autotune(swm_ctx *ctx, void *state, int reps, double *best_us);
 
 /* Measurement helper (no counterpart in the reference): `reps` back-to-back launches of one
  * fused RK stage kernel (stage_id 1, 2 or 4) on the context stream, with the buffers the RK4 step
- * gives it (stage 2: y = a work copy of `state`, v0 = `state`); outputs go to internal work
- * buffers, `state` is unchanged. */
+ * gives it (stage 2: the stage with the most traffic of the step's form, on `state` and work copies);
+ * outputs go to internal work buffers, `state` is unchanged. */
 int swm_bench_stage(swm_ctx *ctx, void *state, int stage_id, int reps);
 
 /* ---- Adjoint form (no counterpart in the reference, which has no adjoint) ----
@@ -211,8 +212,8 @@ int swm_adj_set_tiling(swm_ctx *ctx, int tile_x);
 /* ---- Batched ensemble form (no counterpart in the reference) ----
  * Cubes of different resolutions, one context and one state vector each (same precision and
  * SBP family 42/43/63, N >= 16), advanced together: every RK4 stage of the whole ensemble is
- * one kernel launch over all members' tiles, and one ensemble step (4 launches) and a run of
- * steps are captured once in hipGraphs.  dt holds one time step per member.  The ensemble runs
+ * one kernel launch over all members' tiles (4 launches per step; repeated runs of steps of small
+ * ensembles go through hipGraphs).  dt holds one time step per member.  The ensemble runs
  * on the first member's stream; the states stay owned by the caller.  The launch's blocks walk
  * the task list of all members: blocks_per_slot = 1..64 sizes a persistent grid of that many
  * blocks per resident block slot, 0 launches one block per task (the hardware dispatcher
@@ -313,7 +314,7 @@ int swm_c_set_orography(swm_cctx *ctx, const double *hs, int halo_width);
 /* operator_swm_t%apply (operator_swm_mod.f90:61-113) with the C-grid operators: vout = RHS(vin),
  * enqueued on the context stream */
 int swm_c_rhs(swm_cctx *ctx, const void *vin, void *vout);
-/* nsteps of rk4_t%step (time_schemes/rk4_mod.f90:20-42) in place, HIP-graph captured */
+/* nsteps of rk4_t%step (time_schemes/rk4_mod.f90:20-42) in place */
 int swm_c_rk4_steps(swm_cctx *ctx, void *state, double dt, int nsteps);
 /* operator_t%get_diagnostics (operator_swm_mod.f90:115-236) with SBP_C42_quadrature
  * (quadrature_factory_mod.f90:88-175): out = {hmin, hmax, mass, TE, KE, PE, enstrophy} with
