@@ -906,13 +906,13 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
         }
         __syncthreads();
     }
-    if (t < 2 * CD_NQ + 2) part[(long long)tile_ * 10 + t] = sh[0][t];
+    if (t < 2 * CD_NQ + 2) part[(long long)t * g.ntiles + tile_] = sh[0][t];
 }
 
 // the block partials summed by one block: {mass, KE_u, KE_v, PE, hmin, hmax}
 __global__ void __launch_bounds__(swm::FINAL_THREADS) k_cdiag_final(const double *__restrict__ part, long long nblocks,
                                                                     double *__restrict__ out) {
-    swm::sum_partials<CD_NQ, 10>(part, nblocks, out);
+    swm::sum_partials<CD_NQ>(part, nblocks, out);
 }
 
 #undef C_POINT

@@ -67,11 +67,11 @@ __global__ void __launch_bounds__(256) diag_partial(const T *y, const T *curl, c
         }
         __syncthreads();
     }
-    if (t < 2 * NQ + 2) part[blockIdx.x * 16 + t] = sh[0][t];
+    if (t < 2 * NQ + 2) part[(long long)t * gridDim.x + blockIdx.x] = sh[0][t];
 }
 
 __global__ void __launch_bounds__(FINAL_THREADS) diag_final(const double *part, int nblocks, double *out) {
-    sum_partials<NQ, 16>(part, nblocks, out);
+    sum_partials<NQ>(part, nblocks, out);
 }
 
 // the seven diagnostics in the order of swm_diagnostics from the sums of diag_final (the same

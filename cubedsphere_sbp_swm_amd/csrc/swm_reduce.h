@@ -14,73 +14,59 @@ __device__ __forceinline__ void neu_add(double &s, double &c, double x) {
     s = t;
 }
 
-// Sums of the per-block partials (STRIDE doubles per block: K pairs (sum, compensation), min, max)
-// into out = {K sums, min, max}: one block, each thread over every 1024th partial, then the waves'
-// lanes by shuffles and the 16 waves through LDS, compensated additions throughout.  One thread
-// walking the partials alone is a chain of dependent loads and additions: 371 us for the 1024 of
-// swm_diagnostics (72 us for the 216 of a C-grid C90 state).  With this block the whole call at
-// C384 takes 64 us instead of 424 us.
+// Sums of the per-block partials (value-major, nblocks each: K pairs (sum, compensation), min, max)
+// into out = {K sums, min, max}: one block, two waves to each of the K + 2 values, every lane over each
+// 128th partial with eight loads in flight, then the lanes by shuffles and the two waves through LDS,
+// compensated additions throughout.  One CU's units and the length of a wave's chain are the time: 4.7 us for
+// the 1024 partials of swm_diagnostics, 9.7 us with the values of a block side by side (each lane its own
+// line), 11.4 us with every thread on all values of a partial, 371 us with one thread walking them.
+// swm_diagnostics at C384 takes 56 us, 424 with that one thread.
 constexpr int FINAL_THREADS = 1024;
 
 template <int K>
-__device__ __forceinline__ void lanes_combine(double (&s)[K], double (&c)[K], double &lo, double &hi, int width) {
-    for (int off = width / 2; off > 0; off >>= 1) {
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            const double s2 = __shfl_down(s[q], off, 64), c2 = __shfl_down(c[q], off, 64);
-            neu_add(s[q], c[q], s2);
-            c[q] += c2;
-        }
-        lo = fmin(lo, __shfl_down(lo, off, 64));
-        hi = fmax(hi, __shfl_down(hi, off, 64));
-    }
-}
-
-template <int K, int STRIDE>
 __device__ __forceinline__ void sum_partials(const double *__restrict__ part, long long nblocks,
                                              double *__restrict__ out) {
-    constexpr int NWAVES = FINAL_THREADS / 64;
-    __shared__ double sh[NWAVES][2 * K + 2];
-    const int t = threadIdx.x, lane = t % 64, wave = t / 64;
-    double s[K], c[K], lo = 1e300, hi = -1e300;
-#pragma unroll
-    for (int q = 0; q < K; ++q) s[q] = c[q] = 0.0;
-    for (long long b = t; b < nblocks; b += FINAL_THREADS) {
-        const double *p = part + b * STRIDE;
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            neu_add(s[q], c[q], p[2 * q]);
-            c[q] += p[2 * q + 1];
+    constexpr int PER = 2, LOADS = 8;   // waves per value, loads in flight
+    static_assert((K + 2) * PER * 64 <= FINAL_THREADS, "two waves per value");
+    __shared__ double sh[K + 2][PER][2];
+    const int t = threadIdx.x, lane = t % 64, wave = __builtin_amdgcn_readfirstlane(t / 64);
+    const int q = wave / PER, w = wave % PER;   // q < K: sum q, K: min, K + 1: max
+    double s = q == K ? 1e300 : q == K + 1 ? -1e300 : 0.0, c = 0.0;
+    auto add = [&](double x, double xc) {
+        if (q < K) {
+            neu_add(s, c, x);
+            c += xc;
+        } else {
+            s = q == K ? fmin(s, x) : fmax(s, x);
         }
-        lo = fmin(lo, p[2 * K]);
-        hi = fmax(hi, p[2 * K + 1]);
-    }
-    lanes_combine<K>(s, c, lo, hi, 64);
-    if (lane == 0) {
+    };
+    if (q < K + 2) {
+        const double *p = part + (q <= K ? 2 * q : 2 * K + 1) * nblocks;
+        for (long long b = w * 64 + lane; b < nblocks; b += 64 * PER * LOADS) {
+            double x[LOADS], xc[LOADS];
 #pragma unroll
-        for (int q = 0; q < K; ++q) {
-            sh[wave][2 * q] = s[q];
-            sh[wave][2 * q + 1] = c[q];
+            for (int k = 0; k < LOADS; ++k) {
+                const long long i = b + 64 * PER * k;
+                x[k] = i < nblocks ? p[i] : 0.0;
+                xc[k] = q < K && i < nblocks ? p[nblocks + i] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < LOADS; ++k)
+                if (b + 64 * PER * k < nblocks) add(x[k], xc[k]);
         }
-        sh[wave][2 * K] = lo;
-        sh[wave][2 * K + 1] = hi;
+        for (int off = 32; off > 0; off >>= 1) {
+            const double x = __shfl_down(s, off, 64), xc = __shfl_down(c, off, 64);
+            add(x, xc);
+        }
+        if (lane == 0) {
+            sh[q][w][0] = s;
+            sh[q][w][1] = c;
+        }
     }
     __syncthreads();
-    if (wave != 0) return;
-    const int w = lane % NWAVES;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        s[q] = sh[w][2 * q];
-        c[q] = sh[w][2 * q + 1];
-    }
-    lo = sh[w][2 * K];
-    hi = sh[w][2 * K + 1];
-    lanes_combine<K>(s, c, lo, hi, NWAVES);
-    if (lane != 0) return;
-#pragma unroll
-    for (int q = 0; q < K; ++q) out[q] = s[q] + c[q];
-    out[K] = lo;
-    out[K + 1] = hi;
+    if (q >= K + 2 || w != 0 || lane != 0) return;
+    add(sh[q][1][0], sh[q][1][1]);
+    out[q] = q < K ? s + c : s;
 }
 
 }  // namespace swm
