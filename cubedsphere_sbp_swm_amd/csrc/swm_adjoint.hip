@@ -107,7 +107,7 @@ struct AdjGeo {
     const double *J, *Qi11, *Qi12, *Qi22, *f;
     int n, pitch, es;
     long long fs, mps;   // elements per field; panel stride of J, Qi (0 where all panels hold the same values)
-    double hxs, rhxs, grav;
+    double hxs, grav;
 };
 
 // One launch for the pointwise seeds and the transposed edge syncs.  Blocks below nb_edge
@@ -368,9 +368,8 @@ struct AdjPoint {
 // resident at once, so that chain is the launch's time.  It is kept short: the loads of the own and the
 // halo points are issued together, the own point stays in registers and what only the output reads is
 // in flight across the barrier; the closure columns come from the table (written out, they took a branch
-// with its code per column).  C192 sbp42, stages 3 and 2: 13.6 us, 3.2 TB/s over its 24 values per point;
-// 17.3 us with the halo, the edge gathers and the output's loads one after the other and the divisions
-// on their own.
+// with its code per column).  C192 sbp42, stages 3 and 2: 14.0 us, 3.1 TB/s over its 24 values per point;
+// 17.3 us with the halo, the edge gathers and the output's loads one after the other.
 template <int ORD, int MODE, int TX, int TY, bool INNER>
 __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, const AdjEll &ell, int p, int x0, int y0,
                                              double (&box)[4][AdjTile<ORD, TX, TY>::LH][AdjTile<ORD, TX, TY>::LW],
@@ -385,7 +384,6 @@ __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, 
         adj_rows<ORD, TX, TY>(y0, ye, n, ly, hy);
     }
     const double alpha = A.alpha;
-    const Rcp<double> rhxs{g.hxs, g.rhxs};
     const long long pb = (long long)p * n * g.pitch, mb = (long long)p * g.mps;
     const double *yu = A.y + (pb + g.fs), *yv = yu + g.fs, *Mh = A.M + pb, *Mu = Mh + g.fs, *Mv = Mu + g.fs;
     const double *J = g.J + mb, *Q11 = g.Qi11 + mb, *Q12 = g.Qi12 + mb, *Q22 = g.Qi22 + mb;
@@ -407,8 +405,8 @@ __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, 
         const double vt = q.q12 * q.u + q.q22 * q.v;
         const double mh = alpha * q.mh, mu = alpha * q.mu, mv = alpha * q.mv;
         const double z = q.J * (vt * mu - ut * mv);
-        const Rcp<double> rd = rcp_of(q.J * g.hxs);
-        put(i, j, -mh / rd, z / rd, -mu / rhxs, -mv / rhxs);
+        const double dnm = q.J * g.hxs;
+        put(i, j, -mh / dnm, z / dnm, -mu / g.hxs, -mv / g.hxs);
     };
 
     // the halo points: tile rows outside [x0, xe), then tile columns outside [y0, ye)
@@ -488,14 +486,14 @@ __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, 
                 a += sw[q] * -mh;
                 b += sw[q] * z;
             }
-            const Rcp<double> rd = rcp_of(eJ * g.hxs);
+            const double dnm = eJ * g.hxs;
             double w2 = 0.0, w3 = 0.0;
 #pragma unroll
             for (int q = 0; q < ELL_V; ++q) {
-                w2 += wx[q] * (-(alpha * A.M[g.fs + vx[q]]) / rhxs);
-                w3 += wy[q] * (-(alpha * A.M[g.fs + vy[q]]) / rhxs);
+                w2 += wx[q] * (-(alpha * A.M[g.fs + vx[q]]) / g.hxs);
+                w3 += wy[q] * (-(alpha * A.M[g.fs + vy[q]]) / g.hxs);
             }
-            put(ei, ej, a / rd, b / rd, w2, w3);
+            put(ei, ej, a / dnm, b / dnm, w2, w3);
         }
     }
     if (own && !on_edge(gx, gy)) put_seed(gx, gy, me);
@@ -544,9 +542,8 @@ __device__ __forceinline__ void adj_tile_run(const AdjGeo &g, const AdjArgs &A, 
     const double lut = h * lFx - qz * Jv * mv;
     const double lvt = h * lFy + qz * Jv * mu;
     const double gh = ut * lFx + vt * lFy + g.grav * lK;
-    const Rcp<double> rJ = rcp_of(Jv);
-    const double gu = ut * lK - lAy / rJ + q11 * lut + q12 * lvt;
-    const double gv = vt * lK + lAx / rJ + q12 * lut + q22 * lvt;
+    const double gu = ut * lK - lAy / Jv + q11 * lut + q12 * lvt;
+    const double gv = vt * lK + lAx / Jv + q12 * lut + q22 * lvt;
     const double gg[3] = {gh, gu, gv};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -736,7 +733,7 @@ swm::AdjGeo adj_geo(const swm_ctx *c) {
     swm::AdjGeo g;
     g.J = c->J64; g.Qi11 = c->Qi64[0]; g.Qi12 = c->Qi64[1]; g.Qi22 = c->Qi64[2]; g.f = c->f64;
     g.n = c->n; g.pitch = c->pitch; g.es = 4 * c->N; g.fs = c->fs;
-    g.hxs = c->hx * c->scale; g.rhxs = 1.0 / g.hxs; g.grav = c->grav;
+    g.hxs = c->hx * c->scale; g.grav = c->grav;
     g.mps = c->metric_shared ? 0 : (long long)c->n * c->pitch;
     return g;
 }

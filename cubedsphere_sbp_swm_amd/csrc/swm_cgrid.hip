@@ -551,7 +551,7 @@ static __device__ __forceinline__ void flux_tile(const CGeo &g, const double *__
         const int i = FX.lo + c, j = y0 + r;
         if (!in(i, j, FX, cy)) return;
         const double tt = trow<W42c2i, INNER>(tab, inx, i, N, [&](int q) { return sm.A[r][q - OX.lo]; });
-        const double uu = sm.u[j - OY.lo][c], ut = q11[k] * uu + tt / swm::rcp_of(jx[k]);
+        const double uu = sm.u[j - OY.lo][c], ut = q11[k] * uu + tt / jx[k];
         sm.ku[r][c] = jx[k] * (uu * ut) / 2.0;
         if (i >= x0 && i <= t.fx1) {
             const double hh = trow<W42c2i, INNER>(tab, inx, i, N, [&](int q) { return sm.h[j - CY.lo][q - CX.lo]; });
@@ -563,7 +563,7 @@ static __device__ __forceinline__ void flux_tile(const CGeo &g, const double *__
         const int i = x0 + c, j = FY.lo + r;
         if (!in(i, j, cx, FY)) return;
         const double tt = trow<W42c2i, INNER>(tab, iny, j, N, [&](int q) { return sm.B[q - OY.lo][c]; });
-        const double vv = sm.v[r][i - OX.lo], vt = q22[k] * vv + tt / swm::rcp_of(jy[k]);
+        const double vv = sm.v[r][i - OX.lo], vt = q22[k] * vv + tt / jy[k];
         sm.kv[r][c] = jy[k] * (vv * vt) / 2.0;
         if (j >= y0 && j <= t.fy1) {
             const double hh = trow<W42c2i, INNER>(tab, iny, j, N, [&](int q) { return sm.h[q - CY.lo][i - CX.lo]; });
@@ -579,7 +579,7 @@ static __device__ __forceinline__ void flux_tile(const CGeo &g, const double *__
         const unsigned o = c_off(g, i, j);
         const double kuh = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.ku[r][q - FX.lo]; });
         const double kvh = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.kv[q - FY.lo][c]; });
-        double ke = (kuh + kvh) / swm::rcp_of(swm::at_byte(g.Jo, o));
+        double ke = (kuh + kvh) / swm::at_byte(g.Jo, o);
         ke = ke + g.grav * sm.h[j - CY.lo][i - CX.lo] + g.grav * (g.hs ? swm::at_byte(g.hs + pb, o) : 0.0);
         swm::at_byte(KE + pb, o) = ke;
     });
@@ -607,7 +607,7 @@ static __device__ __forceinline__ void flux_tile(const CGeo &g, const double *__
                 duy = duy + 0.5 * d / A_IF1;
             }
         }
-        swm::at_byte(W + pb, o) = (dvx - duy) / swm::rcp_of(swm::at_byte(g.Jq, o) * g.hx * g.scale);
+        swm::at_byte(W + pb, o) = (dvx - duy) / (swm::at_byte(g.Jq, o) * g.hx * g.scale);
     });
 }
 
@@ -735,13 +735,13 @@ static __device__ __forceinline__ void tend_tile(const CGeo &g, const double *__
         const int i = CX.lo + c, j = y0 + r;
         if (!in(i, j, CX, cy)) return;
         const double gv = trow<W42i2c, INNER>(tab, iny, j, N + 1, [&](int q) { return sm.gv[q - GY.lo][c]; });
-        sm.cu[r][c] = (fa[k] + curl_p(i, j)) * gv / swm::rcp_of(ha[k]);
+        sm.cu[r][c] = (fa[k] + curl_p(i, j)) * gv / ha[k];
     });
     each<TX, TY + C>(tid, [&](int k, int c, int r) {
         const int i = x0 + c, j = CY.lo + r;
         if (!in(i, j, cx, CY)) return;
         const double gu = trow<W42i2c, INNER>(tab, inx, i, N + 1, [&](int q) { return sm.gu[r][q - GX.lo]; });
-        sm.cv[r][c] = -(fb[k] + curl_p(i, j)) * gu / swm::rcp_of(hb[k]);
+        sm.cv[r][c] = -(fb[k] + curl_p(i, j)) * gu / hb[k];
     });
     // the stage vectors of the own points, in flight across the barrier (tiles of interior rows: one
     // point of each field per thread)
@@ -772,7 +772,7 @@ static __device__ __forceinline__ void tend_tile(const CGeo &g, const double *__
             if (j >= N - 2) dy = dy + 0.5 * PEN_R[j - N + 2] * (ny - gy(N + 1));
             qh = rk_pre<RKM>(rk, pb, o);
         }
-        const double div = (dx + dy) / swm::rcp_of(swm::at_byte(g.Jo, o) * g.hx * g.scale);
+        const double div = (dx + dy) / (swm::at_byte(g.Jo, o) * g.hx * g.scale);
         rk_out<RKM>(rk, pb, o, qh, -1.0 * div);
     });
     each<INNER ? TX : TX + 1, TY, NT - TX * TY>(tid, [&](int, int c, int r) {

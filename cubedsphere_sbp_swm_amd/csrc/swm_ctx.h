@@ -162,7 +162,6 @@ swm::DevGeo<T> make_geo(const swm_ctx *c) {
     g.fs = c->fs;
     g.mps = c->metric_shared ? 0 : (long long)c->n * c->pitch;
     g.hxs = (T)(c->hx * c->scale);
-    g.rhxs = T(1) / g.hxs;
     g.hx = (T)c->hx;
     g.scale = (T)c->scale;
     g.grav = (T)c->grav;

@@ -25,7 +25,7 @@
 //
 // A tile runs all its fields together.  The D2 weights depend on the metric only and are formed once per
 // context (hd_weights) with the operations of the reference; a thread loads those of its point once and
-// applies them to every field, as it does its indices, its metric terms and the reciprocal of J.
+// applies them to every field, as it does its indices and its metric terms.
 
 #include <algorithm>
 #include <type_traits>
@@ -96,7 +96,7 @@ struct HdGeo {
     const double *eq, *eb;
     int n, pitch, es;
     long long fs, mps;
-    double hs2, rhs2;                       // (hx * scale)^2 and its reciprocal
+    double hs2;                             // (hx * scale)^2
 };
 
 // D2 weights of one family: interior planes (2R+1 per direction, point (i, j) at j*pitch + i), closure rows
@@ -302,8 +302,8 @@ struct HdFin {
 // to the state of `fin`.  Panel-edge results go to Eout.  INNER: the tile holds no closure row and its box, the
 // tile +-R, no panel-edge point, so every row of it is an interior row.
 // Bound by latency with three blocks a CU (LDS 41 KB at sbp42, 96 and 115 registers): its waves wait 57 % of
-// their cycles, its vector instructions need 14 us and its fields at the rate of a large copy 10 us of the
-// 37 (STEP 1) and 40 us (STEP 2) at C384 sbp42, alone on the chip (45 and 56 in plain band order); C191 sbp63:
+// their cycles, its vector instructions need 15 us and its fields at the rate of a large copy 10 us of the
+// 39 (STEP 1) and 42 us (STEP 2) at C384 sbp42, alone on the chip (45 and 56 in plain band order); C191 sbp63:
 // 23 and 28 us (27 and 33).  The six separate launches of the four fields that they take the place of took 167 us and 85 us with the edge launches.
 template <int ORD, bool H, bool UV, int STEP, int TX, int TY, bool INNER, class Smem>
 __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const double *__restrict__ in, double *__restrict__ out,
@@ -486,7 +486,6 @@ __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const
 
     // ---- D2 rows, cross derivatives, penalties of the cross terms (sbp42 :716-742, sbp63 :1671-1697) ----
     const int cx = i - lx, cy = j - ly;
-    const Rcp<double> rJ = rcp_of(Jo), rhs{g.hs2, g.rhs2};
     auto d2 = [&](const double *w, int b, int s, int cnt, double ih, bool closure, const auto &get) {
         double v = w[0] * get(b);
         if constexpr (INNER) {
@@ -519,7 +518,7 @@ __device__ __forceinline__ void hd_lap_run(const HdGeo &g, const HdLn &ln, const
         const double d2xy = d1(i, lx, [&](int q) { return sm.dy[l][ty][q]; });
         double v = 1.0 * d2x + 1.0 * d2y;
         v = v + 1.0 * d2xy + 1.0 * d2yx;
-        res[l] = v / rhs / rJ;
+        res[l] = v / g.hs2 / Jo;
     }
     if (edge) {
         const int sl = p * g.es + edge_slot(n, i, j);
@@ -683,7 +682,7 @@ swm::HdGeo hd_geo(const swm_ctx *c) {
     g.et = c->hd->et; g.eq = c->hd->eq; g.eb = c->hd->eb;
     g.n = c->n; g.pitch = c->pitch; g.es = 4 * c->N; g.fs = c->fs; g.mps = 0;
     const double hs = c->hx * c->scale;
-    g.hs2 = hs * hs; g.rhs2 = 1.0 / g.hs2;
+    g.hs2 = hs * hs;
     return g;
 }
 

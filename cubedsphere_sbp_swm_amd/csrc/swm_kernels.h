@@ -28,39 +28,6 @@
 namespace swm {
 
 // ----------------------------------------------------------------------------------------
-// Division a / b by a denominator that several quotients share: the reciprocal is refined once
-// (hardware approximation and Newton steps), each quotient is then a product corrected by its exact
-// residual a - b q (Markstein's method: with a reciprocal good to the last place the corrected
-// quotient is the correctly rounded one), and v_div_fixup keeps zeros, infinities and NaN as IEEE
-// division gives them.  FP64: 5 + 4 instructions for the first quotient and 4 for each further one,
-// against 11 for each division on its own.  Same bits as a / b unless the quotient or the residual
-// falls into the subnormal range.
-template <typename T>
-struct Rcp {
-    T b, r;
-};
-__device__ __forceinline__ Rcp<double> rcp_of(double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(fma(-b, r, 1.0), r, r);
-    r = fma(fma(-b, r, 1.0), r, r);
-    return {b, r};
-}
-__device__ __forceinline__ Rcp<float> rcp_of(float b) {
-    float r = __builtin_amdgcn_rcpf(b);
-    r = fmaf(fmaf(-b, r, 1.0f), r, r);
-    return {b, r};
-}
-__device__ __forceinline__ double operator/(double a, const Rcp<double> &d) {
-    const double q = a * d.r;
-    return __builtin_amdgcn_div_fixup(fma(fma(-d.b, q, a), d.r, q), d.b, a);
-}
-__device__ __forceinline__ float operator/(float a, const Rcp<float> &d) {
-    float q = a * d.r;
-    q = fmaf(fmaf(-d.b, q, a), d.r, q);
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d.b, q, a), d.r, q), d.b, a);
-}
-
-// ----------------------------------------------------------------------------------------
 // Geometry and per-launch arguments
 template <typename T>
 struct DevGeo {
@@ -73,7 +40,7 @@ struct DevGeo {
     const double *tanA;                    // tan(alpha_i), i = 0..n-1 (metric evaluated on the fly)
     int n, pitch;
     long long fs;                          // elements per field (6*n*pitch)
-    T hxs, rhxs;                           // hx*scale and its reciprocal, correctly rounded
+    T hxs;                                 // hx*scale
     T hx, scale, grav;
 };
 
@@ -135,7 +102,11 @@ struct EnsMember {
 // ----------------------------------------------------------------------------------------
 // Pointwise stencil inputs of one point (co2contra_colocated_mod.f90:55-56,
 // massflux_colocated_mod.f90:26-27, KE_colocated_mod.f90:44, operator_swm_mod.f90:85,
-// div_ah_sbp_mod.f90:80-91, curl_div_based_mod.f90:58-59)
+// div_ah_sbp_mod.f90:80-91, curl_div_based_mod.f90:58-59).
+// Here and in all kernels a quotient is a plain division, correctly rounded over the whole range.  Quotients of one
+// denominator by a shared, refined reciprocal take less than half the instructions (C384 step alone 79.7 us against 82.7,
+// with three contexts at work 79.7 against 80.5; ensemble step 199 against 206), but are not the same where
+// the denominator, the quotient or its residual is subnormal.
 template <typename T>
 struct Derived {
     T K, Gxd, Gyd, Gxc, Gyc;
@@ -151,14 +122,13 @@ __device__ __forceinline__ Derived<T> make_derived(T h, T u, T v, T J, T q11, T 
     const T hv = h * vt;
     T K = (u * ut + v * vt) / T(2);
     K = K + grav * h + grav * hsv;
-    const Rcp<T> rJ = rcp_of(J);
     d.K = K;
     d.hu = hu;
     d.hv = hv;
     d.Gxd = J * hu;
-    d.Gxc = J * (v / rJ);
+    d.Gxc = J * (v / J);
     d.Gyd = J * hv;
-    d.Gyc = J * (-u / rJ);
+    d.Gyc = J * (-u / J);
     return d;
 }
 
@@ -402,8 +372,8 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
 // Within both parts: row strips outermost, then panels, then columns; an XCD's contiguous range is a band of
 // all six panels, which read the same metric there.  Up to `slots` tiles, where nearly all blocks are resident
 // at once and little waits for a ring tile, all go as ring.  Us alone on the chip, band order / ring first: C-grid
-// step C192 113 / 98, C384 241 / 191; hyperdiffusion step C256 sbp42 70 / 51, C384 103 / 86, sbp63 160 / 119;
-// transposed RHS with its curl C256 sbp42 28.0 / 24.4, C384 43.5 / 37.7.  Below the lines: C-grid step C64
+// step C192 112 / 97, C384 243 / 189; hyperdiffusion step C256 sbp42 68 / 48, C384 100 / 77, sbp63 156 / 112;
+// transposed RHS with its curl C256 sbp42 27.8 / 23.3, C384 41.9 / 36.8.  Below the lines: C-grid step C64
 // 74.9 / 77.3, transposed RHS C192 19.8 / 20.5.  The RK stage kernels stay in band order: their large tiles are a
 // third ring, and a C384 step with three contexts at work went from 80 to 81 us (C768 FP32 alone 166 to 155).
 struct TileOrder {

@@ -91,9 +91,8 @@ __device__ __forceinline__ void finish_point(const DevGeo<T> &g, const StageArgs
     }
     if (a.zeta) at_byte(a.zeta + pb, off) = cu;
     const T fz = pre.f + cu;
-    const Rcp<T> rh = rcp_of(h);
-    const T cor_u = fz * hv / rh * Jv;
-    const T cor_v = -(fz * hu / rh * Jv);
+    const T cor_u = fz * hv / h * Jv;
+    const T cor_v = -(fz * hu / h * Jv);
     const T k[3] = {-dv, -gx + cor_u, -gy + cor_v}, y[3] = {h, u, v};
     T *acc = a.acc + pb;
 #pragma unroll
@@ -128,11 +127,11 @@ __device__ __forceinline__ void load_rows(T *tab, int tid, int nthreads) {
 // of its halo exists and none is on a panel edge; its halo is the REACH of the interior row (2 points
 // for sbp42 and sbp43, 3 for sbp63, against 3, 5, 5 for the closure rows), its guards vanish and its
 // rows have constant weights.  The other tiles take their rows from the table.
-// At C384 sbp42 FP64 (64 x 8, metric read) an RK4 step takes 79 us by slopes and 83 us by states, 20.7 us per
-// stage: a stage 2/3 by states moves about 135 MB at the 7 TB/s that a copy of cache-resident buffers of
-// this size reaches.  With three contexts at work the states no longer fit the memory-side cache: 80 us by slopes, 92 by
-// states.  Wider halos, a branch and its code per closure row, 11-instruction divisions, 64-bit
-// offsets and panel-major tile order (metric read once per panel) took 24-25 us.
+// At C384 sbp42 FP64 (64 x 8, metric read) an RK4 step takes 83 us by slopes and 85 us by states, 21.3 us per
+// stage: a stage 2/3 by states moves about 135 MB at nearly the 7 TB/s that a copy of cache-resident buffers of
+// this size reaches.  With three contexts at work the states no longer fit the memory-side cache: 80 us by slopes, 91 by
+// states.  Wider halos, a branch and its code per closure row, 64-bit offsets and panel-major tile order (metric
+// read once per panel) took 24-25 us a stage.
 template <int ORD, typename T, int MODE, int TX, int TY, bool OTF, bool PERSIST, bool INNER>
 __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T> &a, int p, int tx0, int ty0,
                                            TileFields<T, TX, TY, tile_halo<ORD, INNER>()> &sm, T *tab) {
@@ -234,9 +233,9 @@ __device__ __forceinline__ void stage_tile(const DevGeo<T> &g, const StageArgs<T
             x = sm.K[by + m][lx]; y = sm.Gyd[by + m][tx]; z = sm.Gyc[by + m][tx];
         }, dyK, dyD, dyC);
     }
-    const Rcp<T> rhxs{g.hxs, g.rhxs}, rJd = rcp_of(own.J * g.hx * g.scale);
-    finish_point<T, MODE>(g, a, p, off, own.h, own.u, own.v, own_hu, own_hv, own.J, dxK / rhxs, dyK / rhxs,
-                          (dxD + dyD) / rJd, (dxC + dyC) / rJd, pre);
+    const T Jd = own.J * g.hx * g.scale;
+    finish_point<T, MODE>(g, a, p, off, own.h, own.u, own.v, own_hu, own_hv, own.J, dxK / g.hxs, dyK / g.hxs,
+                          (dxD + dyD) / Jd, (dxC + dyC) / Jd, pre);
 }
 
 // Edge segment `seg` of the cube (edge_segs(n, REACH) per cube): positions k0..k1-1 of one panel
@@ -372,12 +371,12 @@ __device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T
             const T *q = tb + ed.s * (rt.base + m - a0);
             x = q[0]; y = q[ts]; z = q[2 * ts];
         }, tK, tD, tC);
-        const Rcp<T> rhxs{g.hxs, g.rhxs}, rJd = rcp_of(*Jb * g.hx * g.scale);
+        const T Jd = *Jb * g.hx * g.scale;
         // x before y in the sums: the operands commute, so the order does not matter
-        sm.raw[wave][0][lane] = (ed.nu_x ? nK : tK) / rhxs;
-        sm.raw[wave][1][lane] = (ed.nu_x ? tK : nK) / rhxs;
-        sm.raw[wave][2][lane] = (nD + tD) / rJd;
-        sm.raw[wave][3][lane] = (nC + tC) / rJd;
+        sm.raw[wave][0][lane] = (ed.nu_x ? nK : tK) / g.hxs;
+        sm.raw[wave][1][lane] = (ed.nu_x ? tK : nK) / g.hxs;
+        sm.raw[wave][2][lane] = (nD + tD) / Jd;
+        sm.raw[wave][3][lane] = (nC + tC) / Jd;
     }
     __syncthreads();
     if (wave != 0 || !act) return;
