@@ -196,16 +196,24 @@ extern "C" int swm_ens_create(swm_ctx *const *members, void *const *states, int 
     e->stream = members[0]->stream;
     // Defaults (the autotuner measures): one block per task in hardware order; FP64 metric terms from the tangents,
     // as each member has planes of its own, which no other member's tiles share; 32 x 16 tiles, or for sbp42 in
-    // FP64, whose halo is the narrowest, 32 x 8 from 1e6 points on, where there are tasks enough for the
-    // smaller blocks.  Us per step, 64 x 8 with the metric read in a persistent grid / 32 x 16 / 32 x 8:
-    //   sbp42 FP64  16 members C48-C192 (1.7e6 points) 246 / 211 / 204, 64 members 1200 / 1003 / 968,
-    //               32 x C64 213 / 184 / 170, 4 members C32-C64 37.8 / 35.6 / 41.0, C17-C250 75.2 / 70.2 / 71.8
-    //   sbp43 FP64  8 x C128 134 / 123 / 127;  sbp63 FP64  16 members 277 / 232 / 240, 8 x C96 106 / 89 / 96
-    //   sbp42 FP32  16 members 173 / 151 / 149, 8 x C192 145 / 132 / 137
-    long long points = 0;
-    for (const swm_ctx *c : e->m) points += c->fs;
+    // FP64, whose halo is the narrowest, 32 x 8 where 32 x 16 gives more than SMALL_TILES blocks: about two rounds
+    // of the 768 that are resident at once.  With more rounds the edge segments, which fill 4 waves no better
+    // than 8, and the last round cost less in small blocks; with fewer a larger tile's smaller halo counts.
+    // Us per step, one ensemble alone, 32 x 16 / 32 x 8 (blocks of 32 x 16):
+    //   sbp42 FP64  C32, 40, 48, 64 (252) 33.1 / 39.9, 8 x C64 (768) 53.2 / 54.7, 6 x C96 (936) 66.7 / 64.7,
+    //               8 x C96 (1248) 76.7 / 79.4, 4 x C144 (1368) 78.3 / 79.7, 16 x C64 (1536) 92.6 / 89.2,
+    //               3 x C192 (1584) 86.8 / 86.7, 12 x C96 (1872) 105.5 / 102.3, 64 x C32 (2304) 172.5 / 153.7,
+    //               8 x C144 (2736) 130.1 / 127.0, 32 x C64 (3072) 164.0 / 150.6, 2 x C384 (3792) 165.1 / 169.7,
+    //               16 members C48-C192 (4344) 218.7 / 210.8, 64 members (17376) 954.9 / 919.8
+    //   others      sbp43 FP64 12 x C96 (1872) 111.7 / 118.7, sbp63 FP64 8 x C96 (1248) 84.8 / 93.1, 32 x C64 (3072)
+    //               186.8 / 186.3, sbp42 FP32 16 members (4344) 141.4 / 140.7, 32 x C64 (3072) 133.5 / 126.0
+    // A persistent grid of 64 x 8 tiles that reads the metric: 16 members 246, 4 members 37.8, 8 x C96 sbp63 106.
+    constexpr long long SMALL_TILES = 1450;
+    long long blocks = 0;
+    for (const swm_ctx *c : e->m)
+        blocks += 6 * swm::tiles_along(c->n, 32) * swm::tiles_along(c->n, 16) + swm::edge_segs(c->n, swm::Sbp<42>::REACH);
     e->otf = e->prec == 64;
-    if (points >= 1000000 && e->order == 42 && e->prec == 64) e->ty = 8;
+    if (blocks > SMALL_TILES && e->order == 42 && e->prec == 64) e->ty = 8;
     int dev = 0;
     hipDeviceProp_t prop;
     if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) {
