@@ -30,9 +30,13 @@ STEP_VALUES = 68         # per point per RK4 step by states (14 + 20 + 20 + 14)
 STEP_VALUES_SLOPES = 59  # by slopes (11 + 14 + 20 + 14)
 
 
-def by_slopes(N, order, prec):
-    """Whether the RK4 step runs by slopes: its four states take more than 36 MB (sbp63, FP32: 64 MB)."""
-    return 12 * 6 * (N + 1) ** 2 * (prec // 8) > (64e6 if order == 63 or prec == 32 else 36e6)
+def by_slopes(op):
+    """Whether the operator's RK4 steps run by slopes, from the library."""
+    import ctypes
+    from cubedsphere_sbp_swm_amd import _capi
+    form = ctypes.c_int()
+    _capi.check(_capi.lib().swm_rk4_by_slopes(op.ctx, ctypes.byref(form)))
+    return bool(form.value)
 
 
 def parse():
@@ -152,7 +156,7 @@ def fp32_form(args, stream):
                            "rel_linf": float(np.max(np.abs(dh)) / np.max(np.abs(hp)))}
     drift = {p: (res[p]["d1"]["mass"] - res[p]["d0"]["mass"]) / res[p]["d0"]["mass"] for p in (32, 64)}
     rate = {p: cells * steps / res[p]["secs"] for p in (32, 64)}
-    step_gbs32 = (STEP_VALUES_SLOPES if by_slopes(N, 42, 32) else STEP_VALUES) * 4 * points / (res[32]["secs"] / steps) / 1e9
+    step_gbs32 = (STEP_VALUES_SLOPES if by_slopes(ops[32][0]) else STEP_VALUES) * 4 * points / (res[32]["secs"] / steps) / 1e9
     return {"workload": f"C{N} sbp42 RK4 dt={dt:g}s x {steps} steps, degree <= {args.fp32_lmax}",
             "fp32_cell_steps_per_s": rate[32], "fp64_cell_steps_per_s": rate[64],
             "speedup_vs_fp64": rate[32] / rate[64],
@@ -638,7 +642,7 @@ def main():
     eb = op.elem_bytes
     stage_bytes = STAGE23_VALUES * eb * points
     achieved = stage_bytes / (k_us * 1e-6) / 1e9
-    slopes = by_slopes(N, order, args.precision)
+    slopes = by_slopes(op)
     step_bytes = (STEP_VALUES_SLOPES if slopes else STEP_VALUES) * eb * points
     step_gbs = step_bytes / ((ms / 1e3) / args.steps) / 1e9
 

@@ -42,6 +42,7 @@ SIGNATURES = {
     "swm_ctx_get_tiling": (_i, [_vp, _ip, _ip]),
     "swm_ctx_autotune": (_i, [_vp, _vp, _i, _dp]),
     "swm_bench_stage": (_i, [_vp, _vp, _i, _i]),
+    "swm_rk4_by_slopes": (_i, [_vp, _ip]),
     "swm_debug_geometry": (_i, [_vp, _i, _dp, _i]),
     "swm_debug_halo_table": (_i, [_vp, _ip]),
     "swm_rhs_vjp": (_i, [_vp, _vp, _vp, _vp]),

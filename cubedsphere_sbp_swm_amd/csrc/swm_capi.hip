@@ -532,6 +532,12 @@ extern "C" int swm_bench_stage(swm_ctx *c, void *state, int stage_id, int reps) 
     return SWM_OK;
 }
 
+extern "C" int swm_rk4_by_slopes(const swm_ctx *c, int *by_slopes) {
+    if (!c || !by_slopes) return fail(SWM_EARG, "NULL argument");
+    *by_slopes = rk4_by_slopes(c) ? 1 : 0;
+    return SWM_OK;
+}
+
 extern "C" int swm_set_orography(swm_ctx *c, const double *hs, int hw) {
     if (!c) return fail(SWM_EARG, "ctx is NULL");
     HIP_TRY(hipStreamSynchronize(c->stream));

@@ -182,6 +182,10 @@ int swm_ctx_autotune(swm_ctx *ctx, void *state, int reps, double *best_us);
  * outputs go to internal work buffers, `state` is unchanged. */
 int swm_bench_stage(swm_ctx *ctx, void *state, int stage_id, int reps);
 
+/* Measurement helper: *by_slopes = 1 if the context's RK4 steps write slopes in their first stages (a choice by
+ * family, precision and size of the stored fields; 39 instead of 48 field passes a step), else 0. */
+int swm_rk4_by_slopes(const swm_ctx *ctx, int *by_slopes);
+
 /* ---- Adjoint form (no counterpart in the reference, which has no adjoint) ----
  * FP64 contexts with the SBP families 42/43/63, N+1 >= 15 (42, 43) or >= 23 (63).
  *
