@@ -66,13 +66,19 @@ namespace {
 // instead of 48 fields a step through memory, against three more loads per point and its halo in stages 2
 // and 3.  It pays where the four states no longer stay near the chip; below, a stage is a chain of loads.
 // Us per step, states / slopes, one context alone and three at work:
-//   sbp42 FP64  C192 (21 MB) 37.6 / 39.2, 23.6 / 23.2   C256 (38) 48.2 / 47.6, 35.6 / 34.2
-//               C320 (59) 64.4 / 61.8, 51.3 / 48.8      C384 (85) 83.6 / 80.7, 91.8 / 77.8
-//   sbp63 FP64  C320 (59) 75.1 / 77.2, 58.6 / 59.5      C384 (85) 97.7 / 99.4, 105.1 / 95.4
-//   sbp42 FP32  C384 (43) 58.4 / 59.0, 45.9 / 46.0      C768 (170) 164.2 / 166.5, 233.2 / 224.6
-// The wider halo of sbp63 and the cheaper arithmetic of FP32 put their line higher.
+//   sbp42 FP64  C192 (22 MB) 38.8 / 40.9, 24.3 / 23.8   C256 (39) 50.2 / 50.0, 36.4 / 35.3
+//               C320 (61) 65.6 / 64.3, 53.1 / 51.0      C384 (87) 85.5 / 83.2, 91.3 / 80.4
+//   sbp21 FP64  C192 (22 MB) 46.7 / 47.2, 27.8 / 26.9   C256 (39) 61.2 / 58.7, 41.7 / 40.2
+//               C320 (61) 82.3 / 82.5, 66.3 / 61.7      C384 (87) 104.9 / 104.1, 112.1 / 104.0
+//   sbp43 FP64  C288 (49 MB) 67.1 / 68.1, 50.5 / 50.9   C320 (61) 72.7 / 73.7, 58.1 / 57.9
+//               C352 (73) 85.3 / 86.7, 72.3 / 71.3      C384 (87) 95.0 / 95.2, 98.9 / 89.5
+//   sbp63 FP64  C320 (61 MB) 76.8 / 78.5, 61.7 / 62.1   C384 (87) 101.0 / 101.5, 101.6 / 92.3
+//   sbp42 FP32  C384 (43 MB) 59.3 / 59.7, 47.8 / 47.8   C768 (172) 168.1 / 169.1, 232.2 / 224.3
+//   sbp21 FP32  C384 (43 MB) 68.8 / 70.9, 52.3 / 53.5   C512 (77) 99.7 / 102.4, 111.7 / 102.9
+// The wider halos of sbp43 and sbp63 and the cheaper arithmetic of FP32 put their line higher.
 bool rk4_by_slopes(const swm_ctx *c) {
-    const size_t mb = (c->grad_order == 63 || c->prec == 32 ? 64 : 36);
+    const bool narrow = c->grad_order == 21 || c->grad_order == 42;
+    const size_t mb = narrow && c->prec == 64 ? 36 : 64;
     return 12 * c->field_bytes() > mb * 1000000;
 }
 
