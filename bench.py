@@ -137,7 +137,7 @@ def fp32_form(args, stream):
         x.upload(h0, u0, v0)
         d0 = op.get_diagnostics(x)
         ts = swm.create_timescheme(op, "rk4")
-        ts.steps(x, dt, 5)  # warm-up / graph capture
+        ts.steps(x, dt, 5)  # warm-up
         x.upload(h0, u0, v0)
         secs = _timed_steps(ts, x, dt, steps, stream)
         d1 = op.get_diagnostics(x)
@@ -198,7 +198,7 @@ def adjoint_form(args, stream):
         return torch.cuda.Event(enable_timing=True)
 
     def timed(fn, reps=3):
-        fn()  # warm-up (graph capture, lazy work buffers)
+        fn()  # warm-up (the graphs of steps, lazy work buffers)
         best = 1e30
         for _ in range(reps):
             e0, e1 = ev(), ev()
@@ -452,7 +452,7 @@ def cgrid_form(args, stream):
 
 
 def batched_form(args, stream):
-    """One launch per RK stage over all members (hipGraph per step) vs the plain
+    """One launch per RK stage over all members vs the plain
     single-cube path run member after member; same states bit for bit."""
     import numpy as np
     import torch
@@ -480,7 +480,7 @@ def batched_form(args, stream):
     def ev():
         return torch.cuda.Event(enable_timing=True)
 
-    ens.steps(dts, 2)  # tables, graph capture
+    ens.steps(dts, 2)  # tables
     for x, ic in zip(xs, ics):
         x.upload(*ic)
     torch.cuda.synchronize()
@@ -505,14 +505,16 @@ def batched_form(args, stream):
     points = sum(6 * (N + 1) ** 2 for N in Ns)
     cells = sum(6 * N * N for N in Ns)
     stage_bytes = STAGE23_VALUES * 8 * points
-    # plain path: the same members one after another (each its own autotuned tiling, graph)
+    # plain path: the same members one after another (each its own autotuned tiling and graphs)
     for op, x, ic in zip(ops, xs, ics):
         op.set_stream(stream.cuda_stream)
         x.upload(*ic)
         op.autotune(x, reps=5)
         x.upload(*ic)
     for op, x, ic, dt in zip(ops, xs, ics, dts):
-        swm.create_timescheme(op, "rk4").steps(x, dt, 1)  # graph capture for this state and dt
+        # a state's first run is launched step by step, the second captures the graphs of a run of this length
+        for n in (1, steps):
+            swm.create_timescheme(op, "rk4").steps(x, dt, n)
         x.upload(*ic)
     torch.cuda.synchronize()
     p0, p1 = ev(), ev()

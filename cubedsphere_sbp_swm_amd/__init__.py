@@ -377,7 +377,7 @@ class RK4:
 class Ensemble:
     """Cubes of different resolutions (one operator and one state each) advanced together:
     one launch per RK stage over all members (a persistent grid or one block per task, as the
-    autotuner picks), one captured hipGraph per step."""
+    autotuner picks); runs of steps of small ensembles go through hipGraphs of 4 to 64 steps."""
 
     def __init__(self, ops, states):
         if len(ops) != len(states) or not ops:
@@ -604,7 +604,7 @@ class StvecSWMC:
 
 
 class RK4C:
-    """Classical RK4 (time_schemes/rk4_mod.f90) on the C-grid operator, HIP-graph captured."""
+    """Classical RK4 (time_schemes/rk4_mod.f90) on the C-grid operator; repeated runs of steps go through hipGraphs."""
 
     def __init__(self, op):
         self.op = op
