@@ -831,15 +831,6 @@ __global__ void __launch_bounds__(Tiles::THREADS) k_tend(swm::TileOrder order, C
 // compensated (Neumaier) additions per block: mass, KE_u, KE_v, PE, then hmin, hmax.
 constexpr int CD_NQ = 4;
 
-__device__ __forceinline__ void cd_add(double &s, double &c, double x) {
-    const double t = s + x;
-    if (fabs(s) >= fabs(x))
-        c += (s - t) + x;
-    else
-        c += (x - t) + s;
-    s = t;
-}
-
 __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__restrict__ y,
                                                        const double *__restrict__ Acen,
                                                        const double *__restrict__ Aint, double *__restrict__ part) {
@@ -854,10 +845,10 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
         const double hh = h[id];
         hmin = hh;
         hmax = hh;
-        cd_add(s[0], cc[0], hh * g.Jo[mid] * hx * hx * Acen[i] * Acen[j]);
+        swm::neu_add(s[0], cc[0], hh * g.Jo[mid] * hx * hx * Acen[i] * Acen[j]);
         const double pe = 1.0 * hh + 1.0 * (g.hs ? g.hs[id] : 0.0);
         const double PE = 0.5 * g.grav * pe * pe;
-        cd_add(s[3], cc[3], PE * g.Jo[mid] * hx * hx * Acen[i] * Acen[j]);
+        swm::neu_add(s[3], cc[3], PE * g.Jo[mid] * hx * hx * Acen[i] * Acen[j]);
     }
     if (i <= N + 1 && j <= N) {  // KE_diag_u = 0.5 * hu * u at x points, hu = massflux(h, ut)
         const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
@@ -869,7 +860,7 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
         const double ut = g.Qi11x[mid] * u[id] + t / g.Jx[mid];
         const double hu = ut * sop<W42c2i>(i, N, h + cid(g, p, 0, j), 1);
         const double ke = 0.5 * hu * u[id];
-        cd_add(s[1], cc[1], ke * g.Jx[mid] * hx * hx * Aint[i] * Acen[j]);
+        swm::neu_add(s[1], cc[1], ke * g.Jx[mid] * hx * hx * Aint[i] * Acen[j]);
     }
     if (i <= N && j <= N + 1) {
         const long long id = cid(g, p, i, j), mid = id - (long long)p * g.plane;
@@ -881,7 +872,7 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
         const double vt = g.Qi22y[mid] * v[id] + t / g.Jy[mid];
         const double hv = vt * sop<W42c2i>(j, N, h + cid(g, p, i, 0), g.pitch);
         const double ke = 0.5 * hv * v[id];
-        cd_add(s[2], cc[2], ke * g.Jy[mid] * hx * hx * Acen[i] * Aint[j]);
+        swm::neu_add(s[2], cc[2], ke * g.Jy[mid] * hx * hx * Acen[i] * Aint[j]);
     }
     __shared__ double sh[256][2 * CD_NQ + 2];
     const int t = threadIdx.y * BX + threadIdx.x;
@@ -896,7 +887,7 @@ __global__ void __launch_bounds__(256) k_cdiag_partial(CGeo g, const double *__r
         if (t < w) {
             for (int q = 0; q < CD_NQ; ++q) {
                 double a = sh[t][2 * q], ac = sh[t][2 * q + 1];
-                cd_add(a, ac, sh[t + w][2 * q]);
+                swm::neu_add(a, ac, sh[t + w][2 * q]);
                 ac += sh[t + w][2 * q + 1];
                 sh[t][2 * q] = a;
                 sh[t][2 * q + 1] = ac;
