@@ -179,7 +179,7 @@ void drop_graphs(swm_ctx *c) {
 void free_ctx(swm_ctx *c) {
     if (!c) return;
     drop_graphs(c);
-    void *ptrs[] = {c->J, c->Qi11, c->Qi12, c->Qi22, c->f, c->q[0], c->q[1], c->q[2], c->q[3], c->nbr, c->einfo, c->tanA, c->hs,
+    void *ptrs[] = {c->J, c->Qi11, c->Qi12, c->Qi22, c->f, c->q[0], c->q[1], c->q[2], c->q[3], c->einfo, c->tanA, c->hs,
                     c->J64, c->Qi64[0], c->Qi64[1], c->Qi64[2], c->f64, c->A64, c->hs64, c->yA, c->yB, c->yC,
                     c->curl, c->red, c->ecs_w, c->ecs_ind, c->ecs_src, c->ecs_o_w, c->ecs_o_ind, c->ecs_o_edge,
                     c->ecs_tm};
@@ -295,9 +295,6 @@ extern "C" int swm_ctx_create(swm_ctx **out, int N, const char *div, const char 
         for (int i = 0; i < c->n; ++i) ta[i] = std::tan(-0.25 * std::acos(-1.0) + ((double)i + 0.0) * c->hx);
         if ((rc = upload_f64(&c->tanA, ta))) return bail(rc);
     }
-    if (hipMalloc((void **)&c->nbr, c->host_nbr.size() * sizeof(int)) != hipSuccess ||
-        hipMemcpy(c->nbr, c->host_nbr.data(), c->host_nbr.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
-        return bail(fail(SWM_EHIP, "neighbour table upload failed"));
     const size_t sb = 3 * c->field_bytes();
     if (hipMalloc(&c->yA, sb) != hipSuccess || hipMalloc(&c->yB, sb) != hipSuccess || hipMalloc(&c->yC, sb) != hipSuccess ||
         hipMalloc(&c->curl, c->field_bytes()) != hipSuccess)

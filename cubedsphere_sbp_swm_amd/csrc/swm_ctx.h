@@ -107,7 +107,6 @@ struct swm_ctx {
     // device geometry in the context precision
     void *J = nullptr, *Qi11 = nullptr, *Qi12 = nullptr, *Qi22 = nullptr, *f = nullptr;
     void *q[4] = {nullptr, nullptr, nullptr, nullptr};
-    int4 *nbr = nullptr;
     int *einfo = nullptr;
     double *tanA = nullptr;
     bool otf = false;   // FP64: metric terms evaluated on the fly from tan(alpha)

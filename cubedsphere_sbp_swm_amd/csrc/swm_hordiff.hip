@@ -87,7 +87,6 @@ template <> struct Ln<21> {
 // prototype component k on panel p; perm[8 p + 4 + k]: its sign.
 struct HdGeo {
     const double *J, *Qi11, *Qi12, *Qi22;   // panel 0 serves all panels if mps = 0
-    const double *qb, *qt, *ql, *qr;
     const double *B0, *B1, *B2a, *B2b;      // b1 of component 0, b2 of component 1, b1 and b2 of component 2
     const int *perm;
     // per panel-edge slot: (slot of the neighbour's copy across the x edge or -1, across the y edge or -1,
@@ -675,8 +674,6 @@ swm::HdGeo hd_geo(const swm_ctx *c) {
     swm::HdGeo g;
     const size_t P = (size_t)c->n * c->pitch;
     g.J = c->J64; g.Qi11 = c->Qi64[0]; g.Qi12 = c->Qi64[1]; g.Qi22 = c->Qi64[2];
-    g.qb = (const double *)c->q[0]; g.qt = (const double *)c->q[1];
-    g.ql = (const double *)c->q[2]; g.qr = (const double *)c->q[3];
     g.B0 = c->hd->basis; g.B1 = g.B0 + P; g.B2a = g.B0 + 2 * P; g.B2b = g.B0 + 3 * P;
     g.perm = c->hd->perm;
     g.et = c->hd->et; g.eq = c->hd->eq; g.eb = c->hd->eb;

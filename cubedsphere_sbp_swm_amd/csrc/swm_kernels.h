@@ -136,11 +136,6 @@ template <typename T>
 __device__ __forceinline__ long long pidx(const DevGeo<T> &g, int p, int i, int j) {
     return ((long long)p * g.n + j) * g.pitch + i;
 }
-// index of the metric terms J, Qi of point (i, j) of panel p
-template <typename T>
-__device__ __forceinline__ long long midx(const DevGeo<T> &g, int p, int i, int j) {
-    return (long long)p * g.mps + (long long)j * g.pitch + i;
-}
 
 // Metric terms of Ah point (i,j) from tan(alpha_i), tan(beta_j), with the operation order of
 // the host set-up (ecs_metric_mod.f90:413-463); FP64 only.

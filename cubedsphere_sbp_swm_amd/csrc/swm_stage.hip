@@ -253,7 +253,7 @@ template <int ORD, typename T, int MODE, bool OTF, bool PERSIST = false>
 __device__ __forceinline__ void stage_edge(const DevGeo<T> &g, const StageArgs<T> &a, int seg, EdgeFields<ORD, T> &sm,
                                            T *tab, int nthreads) {
     constexpr int R = Sbp<ORD>::REACH, D = Sbp<ORD>::last[0], S = edge_seg_len(R);
-    constexpr int NE = Sbp<ORD>::NE, NW = RowWeights<ORD>::NW;
+    constexpr int NE = Sbp<ORD>::NE;
     const int n = g.n;
     int tid = threadIdx.x;
     if constexpr (PERSIST) asm volatile("" : "+v"(tid));
