@@ -196,9 +196,10 @@ extern "C" int swm_ens_create(swm_ctx *const *members, void *const *states, int 
     e->stream = members[0]->stream;
     // Defaults (the autotuner measures): one block per task in hardware order; FP64 metric terms from the tangents,
     // as each member has planes of its own, which no other member's tiles share; 32 x 16 tiles, or for sbp42 in
-    // FP64, whose halo is the narrowest, 32 x 8 where 32 x 16 gives more than SMALL_TILES blocks: about two rounds
-    // of the 768 that are resident at once.  With more rounds the edge segments, which fill 4 waves no better
-    // than 8, and the last round cost less in small blocks; with fewer a larger tile's smaller halo counts.
+    // FP64, whose halo is the narrowest, 32 x 8 where 32 x 16 gives more than SMALL_TILES blocks, nearly three rounds
+    // of the 512 that are resident at once.  With 91 registers a CU holds 20 waves: two blocks of 8 waves, or five
+    // of 4.  With many rounds the waves in flight count and what an edge segment leaves idle of its block, with fewer
+    // the larger tile's smaller halo.
     // Us per step, one ensemble alone, 32 x 16 / 32 x 8 (blocks of 32 x 16):
     //   sbp42 FP64  C32, 40, 48, 64 (252) 33.1 / 39.9, 8 x C64 (768) 53.2 / 54.7, 6 x C96 (936) 66.7 / 64.7,
     //               8 x C96 (1248) 76.7 / 79.4, 4 x C144 (1368) 78.3 / 79.7, 16 x C64 (1536) 92.6 / 89.2,
@@ -207,7 +208,7 @@ extern "C" int swm_ens_create(swm_ctx *const *members, void *const *states, int 
     //               16 members C48-C192 (4344) 218.7 / 210.8, 64 members (17376) 954.9 / 919.8
     //   others      sbp43 FP64 12 x C96 (1872) 111.7 / 118.7, sbp63 FP64 8 x C96 (1248) 84.8 / 93.1, 32 x C64 (3072)
     //               186.8 / 186.3, sbp42 FP32 16 members (4344) 141.4 / 140.7, 32 x C64 (3072) 133.5 / 126.0
-    // A persistent grid of 64 x 8 tiles that reads the metric: 16 members 246, 4 members 37.8, 8 x C96 sbp63 106.
+    // A persistent grid of 64 x 8 tiles that reads the metric: 16 members 231, 4 members 35.6, 8 x C96 sbp63 103.
     constexpr long long SMALL_TILES = 1450;
     long long blocks = 0;
     for (const swm_ctx *c : e->m)
