@@ -54,10 +54,10 @@ enum StageMode : int {
     MODE_SLOPE3 = 6   // k = RHS(y + ck*kin): out = y + cy*k ; acc = ((y + ck1*acc) + cacc*kin) + cacc*k
                       //                                            (y is v0, kin k2, acc holds k1 on entry)
 };
-// The stages of a step, rk4_mod.f90:28-40.  RK4 steps run RHS, SLOPE2, SLOPE3, STAGE4: stages 1 and 2 write
-// the slope only, 39 field passes a step; where the stage states themselves are wanted (the adjoint's
-// tape), STAGE1, STAGE23, STAGE23, STAGE4 write them and the sum, 48 passes.  Both form every value with
-// the same operations.
+// The stages of a step, rk4_mod.f90:28-40.  Steps of large grids run RHS, SLOPE2, SLOPE3, STAGE4: stages 1 and 2
+// write the slope only, 39 field passes a step.  Small grids, ensembles and the adjoint's tape, which wants the
+// stage states themselves, run STAGE1, STAGE23, STAGE23, STAGE4, which write them and the sum, 48 passes.  Both form
+// every value with the same operations.
 SWM_HD constexpr bool mode_slope(int mode) { return mode == MODE_SLOPE2 || mode == MODE_SLOPE3; }
 
 template <typename T>
